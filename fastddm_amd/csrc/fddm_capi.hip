@@ -35,6 +35,7 @@ struct fddm_plan {
   uint64_t L = 0, H = 0, W = 0, nx = 0, ny = 0, nt = 0, nxh = 0, nq = 0, nl = 0;
   int Tb = 2, Gx = 1, Gy = 1;
   int logn_t = 0;  // time transform length 2^logn_t (fft mode)
+  int wave_t = 0;       // > 0: register time kernel on 2^wave_t samples (fddm_time_wave.hip)
   bool long_t = false;  // four-step time transform with device scratch (fddm_time_long.hip)
   int long_slots = 0;
   uint64_t long_slot = 0, bytes_long = 0;
@@ -346,7 +347,9 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     int logn = kP2MinLog;
     while ((1ull << logn) < 2 * L - 1) ++logn;
     const int maxlog = f64 ? kP2MaxLog - 1 : kP2MaxLog;
-    if (logn > maxlog || p2_lds_bytes(logn, precision) > kLdsLimit) {
+    if (logn - 1 <= time_wave_max_log(precision)) {
+      p->wave_t = logn - 1;
+    } else if (logn > maxlog || p2_lds_bytes(logn, precision) > kLdsLimit) {
       // longer series: four-step transform through device scratch
       const int lmax = long_max_log(precision);
       if (logn > lmax)
@@ -389,6 +392,9 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
       rc = upload(&p->d_twt, wf.data(), wf.size() * sizeof(float), err, errlen);
     }
     if (rc) return fail(rc);
+  } else if (mode == MODE_FFT && p->wave_t) {
+    const std::vector<unsigned char> w = time_wave_tables(p->wave_t, precision, L);
+    if ((rc = upload(&p->d_twt, w.data(), w.size(), err, errlen))) return fail(rc);
   } else if (mode == MODE_FFT) {
     if (f64) {
       auto w = p2_twiddles<double>(p->logn_t);
@@ -555,7 +561,8 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
                               base + p->bytes_R + p->bytes_S + p->bytes_S0 + p->bytes_flags, p->long_slot,
                               p->long_slots, s));
   } else if (p->mode == MODE_FFT) {
-    FDDM_HIP(launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s));
+    FDDM_HIP(p->wave_t ? launch_time_wave(ta, p->wave_t, p->precision, p->out_dtype, s)
+                       : launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s));
   } else {
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }
@@ -808,7 +815,8 @@ int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* e
   if (p->mode == MODE_FFT && p->long_t) {
     FDDM_HIP(launch_time_long(ta, p->logn_t, p->precision, p->out_dtype, lng, p->long_slot, p->long_slots, s));
   } else if (p->mode == MODE_FFT) {
-    FDDM_HIP(launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s));
+    FDDM_HIP(p->wave_t ? launch_time_wave(ta, p->wave_t, p->precision, p->out_dtype, s)
+                       : launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s));
   } else {
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }
