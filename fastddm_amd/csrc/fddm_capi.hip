@@ -35,7 +35,7 @@ struct fddm_plan {
   uint64_t L = 0, H = 0, W = 0, nx = 0, ny = 0, nt = 0, nxh = 0, nq = 0, nl = 0;
   int Tb = 2, Gx = 1, Gy = 1;
   int logn_t = 0;  // time transform length 2^logn_t (fft mode)
-  int wave_t = 0;       // > 0: register time kernel on 2^wave_t samples (fddm_time_wave.hip)
+  int wave_t = 0;  // > 0: register time kernels on 2^wave_t samples (fddm_time_wave.hip, fddm_time_pair.hip)
   bool long_t = false;  // four-step time transform with device scratch (fddm_time_long.hip)
   int long_slots = 0;
   uint64_t long_slot = 0, bytes_long = 0;
@@ -175,8 +175,7 @@ std::vector<T> twiddles(const FftDesc& d) {
 // (cos, sin)(2 pi k / N) for k < N/2.
 template <typename T>
 std::vector<T> p2_twiddles(int logn) {
-  const bool f64 = sizeof(T) == 8;
-  const P2Plan P = p2_plan(logn, f64), Q = p2_half_plan(logn, f64);
+  const P2Plan P = p2_plan(logn), Q = p2_half_plan(logn);
   std::vector<T> w;
   const long double two_pi = 6.283185307179586476925286766559005768L;
   auto pass = [&](long long R, long long NS) {
@@ -344,12 +343,11 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     // zero-padded length >= 2L - 1.  The time kernel runs at the power of two
     // 2^logn_t >= max(2L - 1, 256).
     if (nt < 2 * L - 1) return fail(set_err(err, errlen, FDDM_ERR_ARG, "nt must be >= 2*length-1"));
-    int logn = kP2MinLog;
+    int logn = kTimeMinLog;
     while ((1ull << logn) < 2 * L - 1) ++logn;
-    const int maxlog = f64 ? kP2MaxLog - 1 : kP2MaxLog;
-    if (logn - 1 <= time_wave_max_log(precision)) {
+    if (logn - 1 <= time_pair_log(precision)) {
       p->wave_t = logn - 1;
-    } else if (logn > maxlog || p2_lds_bytes(logn, precision) > kLdsLimit) {
+    } else if (logn > time_p2_log(precision)) {
       // longer series: four-step transform through device scratch
       const int lmax = long_max_log(precision);
       if (logn > lmax)
@@ -393,7 +391,9 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     }
     if (rc) return fail(rc);
   } else if (mode == MODE_FFT && p->wave_t) {
-    const std::vector<unsigned char> w = time_wave_tables(p->wave_t, precision, L);
+    const std::vector<unsigned char> w = p->wave_t <= time_wave_max_log(precision)
+                                             ? time_wave_tables(p->wave_t, precision, L)
+                                             : time_pair_tables(precision, L);
     if ((rc = upload(&p->d_twt, w.data(), w.size(), err, errlen))) return fail(rc);
   } else if (mode == MODE_FFT) {
     if (f64) {
@@ -461,6 +461,14 @@ int record(fddm_plan* p, int slot, hipStream_t s, char* err, size_t errlen) {
   if (p->timing_cap == 0 || p->timing_steps >= p->timing_cap) return FDDM_OK;
   FDDM_HIP(hipEventRecord(p->events[p->timing_steps * kEventsPerStep + slot], s));
   return FDDM_OK;
+}
+
+// Time kernel of series that need no device scratch.
+hipError_t launch_time(const fddm_plan* p, const TimeArgs& ta, hipStream_t s) {
+  if (!p->wave_t) return launch_time_p2(ta, p->precision, p->out_dtype, s);
+  if (p->wave_t <= time_wave_max_log(p->precision))
+    return launch_time_wave(ta, p->wave_t, p->precision, p->out_dtype, s);
+  return launch_time_pair(ta, p->precision, p->out_dtype, s);
 }
 
 int run_spatial(fddm_plan* p, const void* d_img, void* ws, hipStream_t s, char* err, size_t errlen) {
@@ -561,8 +569,7 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
                               base + p->bytes_R + p->bytes_S + p->bytes_S0 + p->bytes_flags, p->long_slot,
                               p->long_slots, s));
   } else if (p->mode == MODE_FFT) {
-    FDDM_HIP(p->wave_t ? launch_time_wave(ta, p->wave_t, p->precision, p->out_dtype, s)
-                       : launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s));
+    FDDM_HIP(launch_time(p, ta, s));
   } else {
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }
@@ -815,8 +822,7 @@ int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* e
   if (p->mode == MODE_FFT && p->long_t) {
     FDDM_HIP(launch_time_long(ta, p->logn_t, p->precision, p->out_dtype, lng, p->long_slot, p->long_slots, s));
   } else if (p->mode == MODE_FFT) {
-    FDDM_HIP(p->wave_t ? launch_time_wave(ta, p->wave_t, p->precision, p->out_dtype, s)
-                       : launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s));
+    FDDM_HIP(launch_time(p, ta, s));
   } else {
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }

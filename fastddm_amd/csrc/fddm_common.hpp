@@ -43,24 +43,16 @@ struct FftDesc {
 // every 32 (see lds_pad in fddm_fft.hpp).
 __host__ __device__ constexpr int lds_padded_size(int n) { return n + (n >> 5) + 1; }
 
-// Time-axis plans for N = 2^logn: threads per transform, number of passes
-// (3 or 4) and the radices of the first transform in order; the first and
-// last passes have a whole number of butterflies per thread.  For
-// FP32 at N >= 4096 the transform is spread over 512 or 1024 threads (radix
-// 8 or 16 passes) so that a CU holds 32 (N = 4096) or 16 waves despite the
-// LDS buffer; FP64 keeps three passes on 256 threads, which measured faster
-// than the four-pass plans at its register and LDS footprint.
+// Time-axis plans of the workgroup kernel (fddm_time_p2.hip), N = 2^14 in FP32
+// and 2^13 in FP64: threads per transform, number of passes (3 or 4) and the
+// radices of the first transform in order; the first and last passes have a
+// whole number of butterflies per thread.  FP64 takes three passes on 256
+// threads, which measured faster than four at its register and LDS footprint.
 struct P2Plan {
   int threads, np, r0, r1, r2, r3;
 };
-__host__ __device__ constexpr P2Plan p2_plan(int logn, bool f64) {
-  return logn == 8    ? P2Plan{64, 4, 4, 4, 4, 4}
-         : logn == 9  ? P2Plan{64, 3, 8, 8, 8, 1}
-         : logn == 10 ? P2Plan{64, 3, 16, 16, 4, 1}
-         : logn == 11 ? P2Plan{128, 3, 16, 16, 8, 1}
-         : logn == 12 ? (f64 ? P2Plan{256, 3, 16, 16, 16, 1} : P2Plan{512, 4, 8, 8, 8, 8})
-         : logn == 13 ? (f64 ? P2Plan{256, 3, 16, 16, 32, 1} : P2Plan{512, 4, 16, 8, 8, 8})
-                      : P2Plan{1024, 4, 16, 8, 8, 16};
+__host__ __device__ constexpr P2Plan p2_plan(int logn) {
+  return logn == 13 ? P2Plan{256, 3, 16, 16, 32, 1} : P2Plan{1024, 4, 16, 8, 8, 16};
 }
 __host__ __device__ constexpr int p2_radix(const P2Plan& P, int i) {
   return i == 0 ? P.r0 : i == 1 ? P.r1 : i == 2 ? P.r2 : P.r3;
@@ -69,14 +61,8 @@ __host__ __device__ constexpr int p2_radix(const P2Plan& P, int i) {
 // runs as one length-N/2 complex transform of z(n) = P(2n) + i P(2n+1) on the
 // same threads (passes with fewer butterflies than threads leave whole waves
 // idle), followed by a per-lag untangling step.
-__host__ __device__ constexpr P2Plan p2_half_plan(int logn, bool f64) {
-  return logn == 8    ? P2Plan{64, 4, 4, 4, 4, 2}
-         : logn == 9  ? P2Plan{64, 3, 8, 8, 4, 1}
-         : logn == 10 ? P2Plan{64, 3, 8, 8, 8, 1}
-         : logn == 11 ? P2Plan{128, 3, 16, 16, 4, 1}
-         : logn == 12 ? (f64 ? P2Plan{256, 3, 16, 16, 8, 1} : P2Plan{512, 4, 8, 8, 8, 4})
-         : logn == 13 ? (f64 ? P2Plan{256, 3, 16, 16, 16, 1} : P2Plan{512, 4, 8, 8, 8, 8})
-                      : P2Plan{1024, 4, 16, 8, 8, 8};
+__host__ __device__ constexpr P2Plan p2_half_plan(int logn) {
+  return logn == 13 ? P2Plan{256, 3, 16, 16, 16, 1} : P2Plan{1024, 4, 16, 8, 8, 8};
 }
 // Points already combined before pass i (product of the earlier radices).
 __host__ __device__ constexpr int p2_ns(const P2Plan& P, int i) { return i == 0 ? 1 : p2_ns(P, i - 1) * p2_radix(P, i - 1); }
@@ -88,15 +74,12 @@ __host__ __device__ constexpr int p2_ns(const P2Plan& P, int i) { return i == 0 
 __host__ __device__ constexpr int p2_tw_pass(const P2Plan& P, int i, int base) {
   return i <= 1 ? base : p2_tw_pass(P, i - 1, base) + p2_ns(P, i - 1) * p2_radix(P, i - 1);
 }
-__host__ __device__ constexpr int p2_tw_a(int logn, bool f64, int i) { return p2_tw_pass(p2_plan(logn, f64), i, 0); }
-__host__ __device__ constexpr int p2_tw_h(int logn, bool f64, int i) {
-  return p2_tw_pass(p2_half_plan(logn, f64), i, p2_tw_a(logn, f64, p2_plan(logn, f64).np));
+__host__ __device__ constexpr int p2_tw_a(int logn, int i) { return p2_tw_pass(p2_plan(logn), i, 0); }
+__host__ __device__ constexpr int p2_tw_h(int logn, int i) {
+  return p2_tw_pass(p2_half_plan(logn), i, p2_tw_a(logn, p2_plan(logn).np));
 }
-__host__ __device__ constexpr int p2_tw_post(int logn, bool f64) {
-  return p2_tw_h(logn, f64, p2_half_plan(logn, f64).np);
-}
-__host__ __device__ constexpr int p2_tw_total(int logn, bool f64) { return p2_tw_post(logn, f64) + (1 << (logn - 1)); }
-constexpr int kP2MinLog = 8, kP2MaxLog = 14;
+__host__ __device__ constexpr int p2_tw_post(int logn) { return p2_tw_h(logn, p2_half_plan(logn).np); }
+constexpr int kTimeMinLog = 8;  // shortest time transform
 
 template <typename T> struct Cplx;
 template <> struct Cplx<float> { using type = float2; };

@@ -90,15 +90,20 @@ __device__ __forceinline__ size_t col_out(const TimeArgs& a, int c) {
 hipError_t launch_rows(const RowArgs& a, int precision, hipStream_t s);
 hipError_t launch_cols(const ColArgs& a, int precision, hipStream_t s);
 hipError_t launch_diff(const TimeArgs& a, int precision, int out_dtype, hipStream_t s);
-// Time kernel at N = 2^logn (p2_plan): LDS bytes per workgroup and launcher.
-size_t p2_lds_bytes(int logn, int precision);
-hipError_t launch_time_p2(const TimeArgs& a, int logn, int precision, int out_dtype, hipStream_t s);
+// Time kernel with one column per workgroup (fddm_time_p2.hip), N = 2^time_p2_log.
+int time_p2_log(int precision);
+hipError_t launch_time_p2(const TimeArgs& a, int precision, int out_dtype, hipStream_t s);
 // Time kernel with every transform in the registers of one wave
 // (fddm_time_wave.hip): M = 2^logm samples (zero-padded, M >= L), logm in
 // [7, time_wave_max_log].  time_wave_tables: the tables it reads from a.twt.
 int time_wave_max_log(int precision);
 std::vector<unsigned char> time_wave_tables(int logm, int precision, uint64_t L);
 hipError_t launch_time_wave(const TimeArgs& a, int logm, int precision, int out_dtype, hipStream_t s);
+// The same with a column's even and odd bins on two waves
+// (fddm_time_pair.hip), M = 2^time_pair_log samples.
+int time_pair_log(int precision);
+std::vector<unsigned char> time_pair_tables(int precision, uint64_t L);
+hipError_t launch_time_pair(const TimeArgs& a, int precision, int out_dtype, hipStream_t s);
 // Power-of-two spatial kernels (256 <= n <= 4096): plan radices and launchers.
 bool p2_spatial_ok(int logn);
 int p2_spatial_plan(int logn, bool cols, int* r0, int* r1, int* r2);

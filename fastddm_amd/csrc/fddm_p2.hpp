@@ -1,6 +1,6 @@
 // Compile-time power-of-two FFT machinery shared by the time kernel and the
 // power-of-two spatial kernels: constant-folded twiddle factors, radix
-// 2..32 butterflies (16 and 32 as Cooley-Tukey composites), and a Stockham
+// 2..64 butterflies (16, 32 and 64 as Cooley-Tukey composites), and a Stockham
 // pass whose size, radix, stride and data layout are template parameters, so
 // every LDS address is one per-butterfly base plus immediate offsets.
 #pragma once
@@ -131,9 +131,11 @@ __device__ __forceinline__ void dft(cplx_t<T> (&v)[R]) {
     butterfly<T, R>(v);
   } else if constexpr (R == 16) {
     dft_composite<T, 4, 4>(v);
-  } else {
-    static_assert(R == 32, "radix");
+  } else if constexpr (R == 32) {
     dft_composite<T, 8, 4>(v);
+  } else {
+    static_assert(R == 64, "radix");
+    dft_composite<T, 8, 8>(v);
   }
 }
 

@@ -8,281 +8,29 @@
 // and Re C(d) = Re IFFT_N(|G|^2) needs one more, Z = FFT_M(z) of
 // z(k) = |G(2k)|^2 + i |G(2k + 1)|^2.
 //
-// An M-point transform is worked on by P lanes of one wave holding R points
-// each (M = P R, sample t = p + P r in register r of lane p; 64 / P columns
-// per wave): a radix-R DFT in registers, the twiddles W_M^(p k1), one exchange
-// through the wave's own LDS, and a second DFT in registers (P points, or R
-// points after one radix-2 step between the wave's halves when P = 2R).  The
-// result is again in natural order, bin k = p + P r in register r of lane p.
-// All LDS addresses are one base per lane plus immediate offsets, so next to
-// no integer arithmetic is left, and nothing waits at a workgroup barrier
-// until the results of the workgroup's columns are written out.
+// A wave holds 64 / P columns (fddm_time_wave.hpp) and nothing waits at a
+// workgroup barrier until the results of the workgroup's columns are written.
 //
 // What bounds it: VALU issue (74 % busy at M = 2048; 5400 instructions per
 // column against 9600 of the workgroup form, k_time_p2, which spent 62 % of
 // them on addresses, moves and conversions and met at two barriers per pass).
-// Kernel time, before and after: 3.06 -> 1.89 ms for 131584 columns of 2000
+// Kernel time, before and after: 3.06 -> 1.85 ms for 131584 columns of 2000
 // samples in compensated FP32, 1.58 -> 1.15 ms for 154080 of 997, 0.142 ->
 // 0.088 ms for 15456 of 271 in FP64.
+// Waves per workgroup: four, so that two or more workgroups per CU overlap;
+// eight at M = 1024 in FP32, whose lag rows then leave in 32-byte pieces
+// (1.35 -> 1.05 ms with all of 1002 lags); at M = 2048 and 512 and in FP64
+// eight measured slower.
 // Every batch of global loads is issued well before its use (issued()): with
 // two to four waves per SIMD the latency is not hidden otherwise (the same
 // kernel with the loads left to the scheduler: 3.7 ms at M = 2048).
 #include <vector>
 
-#include "fddm_kernels.hpp"
-#include "fddm_p2.hpp"
-#include "fddm_wave.hpp"
+#include "fddm_time_wave.hpp"
 
 namespace fddm {
 namespace {
-using namespace p2;
-
-constexpr int kWaves = 4;  // waves per workgroup
-constexpr int kEdge = 32;  // lags of at most this many pairs: direct sums (compensated paths)
-
-// Shape and LDS layout of M = P R.  Elements are 8 bytes: a float complex
-// value, or one component of a double one (exchanged one after the other).
-template <int R_, int P_>
-struct WaveLay {
-  static constexpr int R = R_, P = P_, M = R * P, GROUPS = 64 / P, Q = kWaves * GROUPS;
-  // second stage, P points per k1: one pass (P <= R), a radix-2 step between
-  // the halves of the wave and one pass (P = 2R = 64), or two passes R R3
-  static constexpr bool LANE2 = P == 64 && R == 32;
-  static constexpr int R3 = P > R && !LANE2 ? P / R : 1;
-  static_assert(LANE2 || (P <= R ? R % P == 0 : R % R3 == 0), "plan");
-  // exchange: rows of NC elements, read back 16 bytes at a time; blocks of
-  // NC + 2 put eight such reads in distinct banks (three passes: R3 blocks
-  // of R a row, then R3 rows of R^2)
-  static constexpr int NC = LANE2 || R3 > 1 ? R : P, RS = R3 > 1 ? R3 * (R + 2) + 2 : NC + 2;
-  static constexpr int ROWS = R3 > 1 ? R : M / NC, RS3 = R * R + 16;
-  static constexpr int GS0 = ROWS * RS > R3 * RS3 || R3 == 1 ? ROWS * RS : R3 * RS3;
-  static constexpr int GS = GS0 + (GROUPS > 2 ? P : 0);  // groups start in distinct banks
-  // chunks of R consecutive samples, stride R + 2
-  static constexpr int CS = R + 2, CG = P * CS;
-  static constexpr int NB = P >= R ? 1 : R / P;  // register rows per chunk, where a chunk is longer than a row
-  static constexpr int chunk_row(int r) { return P >= R ? r * (P / R) * CS : (r / NB) * CS + (r % NB) * P; }
-  // the exchange buffer or the chunks, then the last kEdge samples of each group
-  static constexpr int BUF = GROUPS * (GS > CG ? GS : CG), WAVE = BUF + GROUPS * kEdge;
-  // results of one column, by lag; the columns' strides spread over the banks
-  static constexpr int SS = M + 32 / Q;
-  static_assert(Q <= 32 && Q * SS <= kWaves * WAVE, "results fit the exchange buffers");
-  static constexpr size_t bytes = sizeof(double) * kWaves * WAVE;
-  // tables, complex of the compute type: W_M^(p k1) at [k1][p],
-  // W_M^(p (k1 + 1/2)) at [k1][p], then W_P^j (j < R; LANE2) or W_P^(p0 k2) at
-  // [k2][p0] (R3 > 1), (cos, sin)(2 pi d / N) for d < M / 2; in double
-  // 1 / (L - d) for d < M
-  static constexpr int TW_E = 0, TW_O = M, TW_2 = 2 * M, TW_CS = TW_2 + (LANE2 ? R : R3 > 1 ? P : 0);
-  static constexpr int TW_END = TW_CS + M / 2;
-};
-
-// Position of sample t in the chunk layout.
-template <int R>
-__device__ __forceinline__ int chunk_pos(int t) {
-  constexpr int LR = R == 32 ? 5 : R == 16 ? 4 : 3;
-  static_assert(R == 1 << LR, "R");
-  return t + ((t >> LR) << 1);
-}
-
-// Orders this wave's LDS writes before its later reads (the hardware keeps a
-// wave's LDS accesses in order; this keeps the compiler from moving them).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-
-// a: [a of lanes 0..31 | b of lanes 0..31], b: [a of 32..63 | b of 32..63]
-__device__ __forceinline__ void swap32(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]);
-  b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void swap32(double& a, double& b) {
-  const uint64_t ua = static_cast<uint64_t>(__double_as_longlong(a)), ub = static_cast<uint64_t>(__double_as_longlong(b));
-  const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
-  const auto hi =
-      __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32), false, false);
-  a = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi[0]) << 32) | lo[0]));
-  b = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi[1]) << 32) | lo[1]));
-}
-
-__device__ __forceinline__ float from_lane(float v, int addr) {
-  return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(v)));
-}
-__device__ __forceinline__ double from_lane(double v, int addr) {
-  const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
-  const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(addr, static_cast<int>(u & 0xffffffffull)));
-  const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(addr, static_cast<int>(u >> 32)));
-  return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
-}
-
-// Inclusive scan over the P lanes of a group, and the group's total in every lane.
-template <int P>
-__device__ __forceinline__ double group_scan(double v, int p) {
-  if constexpr (P == 64) return wave::incl_scan(v);
-#pragma unroll
-  for (int s = 1; s < P; s *= 2) {
-    const double u = __shfl_up(v, s, P);
-    v += p >= s ? u : 0.0;
-  }
-  return v;
-}
-template <int P>
-__device__ __forceinline__ double group_last(double v) {
-  if constexpr (P == 64) return wave::lane63(v);
-  return __shfl(v, P - 1, P);
-}
-
-// Keeps what is written before it (a batch of loads) ahead of what follows:
-// left alone, the scheduler sinks each load to its use to save registers and
-// waits for them one by one.
-__device__ __forceinline__ void issued() { __builtin_amdgcn_sched_barrier(0); }
-
-// Element i + p of a table (i the same for all lanes).
-template <typename E>
-__device__ __forceinline__ E entry(const E* __restrict__ table, int i, unsigned p) {
-  return *reinterpret_cast<const E*>(reinterpret_cast<const char*>(table + i) + p * static_cast<unsigned>(sizeof(E)));
-}
-
-// Exchange between two passes: register i written to position wpos(i), then
-// runs of NC registers read from consecutive positions from rpos(run) on
-// (16 bytes at a time where NC > 1).
-template <int R, int NC, typename E, typename FR>
-__device__ __forceinline__ void read_rows(const E* b, E (&x)[R], FR&& rpos) {
-  if constexpr (NC == 1) {
-#pragma unroll
-    for (int i = 0; i < R; ++i) x[i] = b[rpos(i)];
-  } else {
-    struct alignas(16) Two {
-      E a, b;
-    };
-#pragma unroll
-    for (int i = 0; i < R; i += 2) {
-      const Two t = *reinterpret_cast<const Two*>(b + rpos(i / NC) + i % NC);
-      x[i] = t.a;
-      x[i + 1] = t.b;
-    }
-  }
-}
-template <typename T, int R, int NC, typename FW, typename FR>
-__device__ __forceinline__ void exchange(cplx_t<T> (&v)[R], double* lds, FW&& wpos, FR&& rpos) {
-  if constexpr (sizeof(T) == 4) {
-    float2* const b = reinterpret_cast<float2*>(lds);
-#pragma unroll
-    for (int i = 0; i < R; ++i) b[wpos(i)] = v[i];
-    wave_sync();
-    read_rows<R, NC>(b, v, rpos);
-    wave_sync();
-  } else {
-    double x[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) lds[wpos(i)] = v[i].x;
-    wave_sync();
-    read_rows<R, NC>(lds, x, rpos);
-    wave_sync();
-#pragma unroll
-    for (int i = 0; i < R; ++i) lds[wpos(i)] = v[i].y;
-    wave_sync();
-#pragma unroll
-    for (int i = 0; i < R; ++i) v[i].x = x[i];
-    read_rows<R, NC>(lds, x, rpos);
-#pragma unroll
-    for (int i = 0; i < R; ++i) v[i].y = x[i];
-    wave_sync();
-  }
-}
-
-// Forward M-point transform, natural order in and out.  ODD: of x(t) W_N^t,
-// the odd bins of the N-point one (in the first DFT W_R^(r / 2), the rest in
-// its twiddle table).  mid() runs after the exchange (the place to issue
-// loads for what follows the transform).
-template <typename T, typename Lay, bool ODD, typename F>
-__device__ __forceinline__ void wave_fft(cplx_t<T> (&v)[Lay::R], double* lds, const cplx_t<T>* __restrict__ tw, int p,
-                                         F&& mid) {
-  using C = cplx_t<T>;
-  constexpr int R = Lay::R, P = Lay::P, RS = Lay::RS, R3 = Lay::R3;
-  C w[R];
-#pragma unroll
-  for (int k = ODD ? 0 : 1; k < R; ++k) w[k] = entry(tw, (ODD ? Lay::TW_O : Lay::TW_E) + k * P, p);
-  C wl{};
-  if constexpr (Lay::LANE2) wl = entry(tw, Lay::TW_2, p & (R - 1));
-  issued();
-  if constexpr (ODD) sfor<1, R>([&](auto rc) {
-      constexpr int r = decltype(rc)::value;
-      v[r] = mul_w<T, r, 2 * R>(v[r]);
-    });
-  dft<T, R>(v);
-#pragma unroll
-  for (int k = ODD ? 0 : 1; k < R; ++k) v[k] = cmul(v[k], w[k]);
-  if constexpr (Lay::LANE2) {
-    // bins k1 + R k2, k2 = 2 kappa + g: sums (g = 0) and differences (g = 1)
-    // of samples j and j + R of the P-point transforms; lanes below 32 take
-    // the even k1, the others the odd ones
-    const int j = p & (R - 1), hi = p >> 5;
-    static_assert(R == 32, "the halves of the wave");
-#pragma unroll
-    for (int i = 0; i < R; i += 2) {
-      swap32(v[i].x, v[i + 1].x);
-      swap32(v[i].y, v[i + 1].y);
-      const C a = v[i], b = v[i + 1];
-      v[i] = cadd(a, b);
-      v[i + 1] = cmul(csub(a, b), wl);
-    }
-    const int wb = hi * RS + j, rb = p * RS;
-    // register i + g holds (k1 = i + hi, g): row k1 + R g
-    exchange<T, R, R>(v, lds, [&](int i) { return wb + ((i & ~1) + R * (i & 1)) * RS; }, [&](int) { return rb; });
-    mid();
-    dft<T, R>(v);
-  } else if constexpr (R3 > 1) {
-    // sample p = p0 + R3 p1 of the P-point transforms: radix R over p1 (lane
-    // p0 R + k1), twiddles, then radix R3 over p0 of the bins j = k1 + R k2
-    // = p + P i, which leaves bin j + R^2 k3 in register i + (R / R3) k3
-    const int k1 = p & (R - 1), p0 = p / R;
-    const int wb = (p & (R3 - 1)) * (R + 2) + p / R3, rb = k1 * RS + p0 * (R + 2);
-    exchange<T, R, R>(v, lds, [&](int i) { return wb + i * RS; }, [&](int) { return rb; });
-#pragma unroll
-    for (int k = 1; k < R; ++k) w[k] = entry(tw, Lay::TW_2 + k * R3, p0);
-    issued();
-    dft<T, R>(v);
-#pragma unroll
-    for (int k = 1; k < R; ++k) v[k] = cmul(v[k], w[k]);
-    const int wb3 = p0 * Lay::RS3 + k1;
-    constexpr int NI = R / R3;
-    exchange<T, R, 1>(v, lds, [&](int i) { return wb3 + i * R; },
-                      [&](int i) { return p + (i % NI) * P + (i / NI) * Lay::RS3; });
-    mid();
-    // register i + NI p0 holds sample p0 of butterfly i
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      C u[R3];
-#pragma unroll
-      for (int k = 0; k < R3; ++k) u[k] = v[i + NI * k];
-      dft<T, R3>(u);
-#pragma unroll
-      for (int k = 0; k < R3; ++k) v[i + NI * k] = u[k];
-    }
-  } else {
-    constexpr int CN = R / P;
-    const int rb = p * RS;
-    exchange<T, R, P>(v, lds, [&](int i) { return p + i * RS; }, [&](int i) { return rb + i * P * RS; });
-    mid();
-    C o[R];
-#pragma unroll
-    for (int i = 0; i < CN; ++i) {
-      C u[P];
-#pragma unroll
-      for (int k = 0; k < P; ++k) u[k] = v[i * P + k];
-      dft<T, P>(u);
-#pragma unroll
-      for (int k = 0; k < P; ++k) o[i + CN * k] = u[k];
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = o[r];
-  }
-}
+using namespace tw;
 
 // Waves per SIMD: what the LDS of M = 2^10 and 2^11 allows in FP32, 3 where
 // the registers of the others fit, 2 in double.
@@ -291,11 +39,11 @@ constexpr int wave_occ() {
   return sizeof(T) == 8 ? (R == 8 ? 3 : 2) : R == 32 ? 2 : P == 64 || R == 8 ? 4 : 3;
 }
 
-template <typename T, typename OutT, int R, int P>
-__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(wave_occ<T, R, P>(), wave_occ<T, R, P>())))
+template <typename T, typename OutT, int R, int P, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(wave_occ<T, R, P>(), wave_occ<T, R, P>())))
     k_time_wave(TimeArgs a, int wg_per_xcd, int wgs, int subtract_mean) {
   using C = cplx_t<T>;
-  using Lay = WaveLay<R, P>;
+  using Lay = WaveLay<R, P, W>;
   constexpr int M = Lay::M, Q = Lay::Q;
   constexpr bool F64 = sizeof(T) == 8;
 
@@ -314,8 +62,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   if constexpr (P == 64) q = __builtin_amdgcn_readfirstlane(q);
   const int L = a.L;
   const C* __restrict__ src = static_cast<const C*>(a.S) + static_cast<size_t>(q - a.s_q0) * a.Lp;
-  const C* __restrict__ tw = static_cast<const C*>(a.twt);
-  const double* __restrict__ inv = reinterpret_cast<const double*>(tw + Lay::TW_END);
+  const C* __restrict__ tab = static_cast<const C*>(a.twt);
+  const double* __restrict__ inv = reinterpret_cast<const double*>(tab + Lay::TW_END);
   double* const wlds = reinterpret_cast<double*>(smem) + wave * Lay::WAVE;
   double* const xlds = wlds + g * Lay::GS;  // exchange
   double* const clds = wlds + g * Lay::CG;  // chunks
@@ -340,6 +88,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   C v[R], x[R];
   load(v);
   const double rl = inv[0];
+  C first{0, 0};  // F(0) of the raw first frame
+  if (a.S0) first = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
   T m_r = 0, m_i = 0;
   center(v, T(0), T(0));
   double sr = 0, si = 0;
@@ -364,17 +114,17 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   C cs[R / 2];
   {
     T pe[R];
-    wave_fft<T, Lay, false>(v, xlds, tw, p, [&] { load(x); });
+    wave_fft<T, Lay>(v, xlds, tab + Lay::TW_E, tab + Lay::TW_2, p, std::false_type{}, [&] { load(x); });
 #pragma unroll
     for (int r = 0; r < R; ++r) pe[r] = v[r].x * v[r].x + v[r].y * v[r].y;
     center(x, m_r, m_i);
-    wave_fft<T, Lay, true>(x, xlds, tw, p, [] {});
+    wave_fft<T, Lay>(x, xlds, tab + Lay::TW_O, tab + Lay::TW_2, p, std::true_type{}, [] {});
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = C{pe[r], x[r].x * x[r].x + x[r].y * x[r].y};
   }
-  wave_fft<T, Lay, false>(v, xlds, tw, p, [&] {
+  wave_fft<T, Lay>(v, xlds, tab + Lay::TW_E, tab + Lay::TW_2, p, std::false_type{}, [&] {
 #pragma unroll
-    for (int r = 0; r < R / 2; ++r) cs[r] = entry(tw, Lay::TW_CS + P * r, p);
+    for (int r = 0; r < R / 2; ++r) cs[r] = entry(tab, Lay::TW_CS + P * r, p);
     issued();
   });
   load(x);
@@ -387,23 +137,33 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   double ca[R / 2], cb[R / 2];
   {
     const int other = ((lane - p) + ((P - p) & (P - 1))) * 4;
+    constexpr int B = 4;  // values fetched from other lanes at once
 #pragma unroll
-    for (int r = 0; r < R / 2; ++r) {
-      const int r0 = r == 0 ? R / 2 : R - r;
-      C b;
-      b.x = from_lane(p == 0 ? v[r0].x : v[R - 1 - r].x, other);
-      b.y = from_lane(p == 0 ? v[r0].y : v[R - 1 - r].y, other);
-      double ax = v[r].x, ay = v[r].y;
-      const double bx = b.x;
-      double by = b.y;
-      if (r == 0) {
-        ax = p == 0 ? bx : ax;
-        ay = p == 0 ? 0.0 : ay;
-        by = p == 0 ? 0.0 : by;
+    for (int rb = 0; rb < R / 2; rb += B) {
+      C o[B];
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const int r = rb + i, r0 = r == 0 ? R / 2 : R - r;
+        o[i].x = from_lane(p == 0 ? v[r0].x : v[R - 1 - r].x, other);
+        o[i].y = from_lane(p == 0 ? v[r0].y : v[R - 1 - r].y, other);
       }
-      const double s = ax + bx, w = static_cast<double>(cs[r].x) * (ay + by) - static_cast<double>(cs[r].y) * (ax - bx);
-      ca[r] = s + w;
-      cb[r] = s - w;
+      issued();
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const int r = rb + i;
+        double ax = v[r].x, ay = v[r].y;
+        const double bx = o[i].x;
+        double by = o[i].y;
+        if (r == 0) {
+          ax = p == 0 ? bx : ax;
+          ay = p == 0 ? 0.0 : ay;
+          by = p == 0 ? 0.0 : by;
+        }
+        const double s = ax + bx;
+        const double w = static_cast<double>(cs[r].x) * (ay + by) - static_cast<double>(cs[r].y) * (ax - bx);
+        ca[r] = s + w;
+        cb[r] = s - w;
+      }
     }
   }
 
@@ -533,23 +293,35 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
       ql[i] = chunk_pos<R>(L - M + p + P * i);
     }
     auto row = [&](int r) { return P >= R ? r * (P / R) * Lay::CS : (r / NB) * Lay::CS; };
-    auto value = [&](double cc, int d, int tail, int head, double rn, bool first) {
-      const double num = clds[head] + (ptot - clds[tail]) + k * cc;
+    auto value = [&](double cc, int d, double tail, double head, double rn, bool first) {
+      const double num = head + (ptot - tail) + k * cc;
       if constexpr (!F64) flag |= num < thr && (!first || d >= 1) && d < L - kEdge;
       return num * rn;
     };
+    constexpr int B = 4;  // lag pairs whose sums are read at once
 #pragma unroll
-    for (int r = 0; r < R / 2; ++r)
-      ca[r] = value(ca[r], p + P * r, pd[r % NB] + row(r), min(max(pl[r % NB] - row(r), 0), Lay::CG - 1), ia[r], r == 0);
+    for (int rb = 0; rb < R / 2; rb += B) {
+      double ta[B], ha[B], tb[B], hb[B];
 #pragma unroll
-    for (int r = 0; r < R / 2; ++r) {
-      int d = M - p - P * r, tail = qd[(R - 1 - r) % NB] + row(R - 1 - r), head = max(ql[r % NB] + row(r), 0);
-      if (r == 0) {
-        d = p == 0 ? M / 2 : d;
-        tail = p == 0 ? chunk_pos<R>(M / 2) : tail;
-        head = p == 0 ? chunk_pos<R>(max(L - M / 2, 0)) : head;
+      for (int i = 0; i < B; ++i) {
+        const int r = rb + i;
+        int tail = qd[(R - 1 - r) % NB] + row(R - 1 - r), head = max(ql[r % NB] + row(r), 0);
+        if (r == 0) {
+          tail = p == 0 ? chunk_pos<R>(M / 2) : tail;
+          head = p == 0 ? chunk_pos<R>(max(L - M / 2, 0)) : head;
+        }
+        ta[i] = clds[pd[r % NB] + row(r)];
+        ha[i] = clds[min(max(pl[r % NB] - row(r), 0), Lay::CG - 1)];
+        tb[i] = clds[tail];
+        hb[i] = clds[head];
       }
-      cb[r] = value(cb[r], d, tail, head, ib[r], false);
+      issued();
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const int r = rb + i, d = p + P * r;
+        ca[r] = value(ca[r], d, ta[i], ha[i], ia[r], r == 0);
+        cb[r] = value(cb[r], r == 0 && p == 0 ? M / 2 : M - d, tb[i], hb[i], ib[r], false);
+      }
     }
   }
   if constexpr (!F64) {
@@ -563,23 +335,22 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     const size_t oq = col_out(a, c);
     const double mr2 = fsr * rl, mi2 = fsi * rl;
     const double var = ptot * rl - (mr2 * mr2 + mi2 * mi2);
-    double fr = static_cast<double>(m_r) + mr2, fi = static_cast<double>(m_i) + mi2;
-    if (a.S0) {
-      const C z = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
-      fr += static_cast<double>(z.x);
-      fi += static_cast<double>(z.y);
-    }
+    const double fr = static_cast<double>(m_r) + mr2 + static_cast<double>(first.x);
+    const double fi = static_cast<double>(m_i) + mi2 + static_cast<double>(first.y);
     const double ps = var + fr * fr + fi * fi;
     out[static_cast<size_t>(a.nl) * ldo + oq] = static_cast<OutT>(ps);
     out[static_cast<size_t>(a.nl + 1) * ldo + oq] = static_cast<OutT>(var);
   }
+
+  using Rows = LagRows<OutT, 64 * W, Q, M>;
+  static_assert(Q * Rows::SS * sizeof(OutT) <= Lay::bytes, "results fit the exchange buffers");
 
   // 6. results to LDS by column and lag (over the exchange buffers), then
   // every requested lag's row of Q neighbouring columns to the output
   __syncthreads();
   OutT* const stage = reinterpret_cast<OutT*>(smem);
   {
-    OutT* const st = stage + qi * Lay::SS;
+    OutT* const st = stage + qi * Rows::SS;
 #pragma unroll
     for (int r = 0; r < R / 2; ++r) st[p + P * r] = static_cast<OutT>(ca[r]);
 #pragma unroll
@@ -596,48 +367,21 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     }
   }
   __syncthreads();
-  {
-    const int qq = tid % Q, i0 = tid / Q;
-    constexpr int STEP = 64 * kWaves / Q, B = 8;  // lags per round of the workgroup, rounds in flight
-    if (c0 + qq < a.cols) {
-      const OutT* const st = stage + qq * Lay::SS;
-      OutT* dst = out + static_cast<size_t>(i0) * ldo + col_out(a, c0 + qq);
-      const size_t step = STEP * ldo;
-      for (int ib = 0; ib < a.nl; ib += B * STEP) {
-        const int left = a.nl - ib - i0;  // lags of this lane from here on: b STEP < left
-        uint32_t d[B];
-#pragma unroll
-        for (int b = 0; b < B; ++b) d[b] = a.lags[min(ib + i0 + b * STEP, a.nl - 1)];
-        issued();
-        OutT r[B];
-#pragma unroll
-        for (int b = 0; b < B; ++b) r[b] = st[d[b]];
-        if (ib + B * STEP <= a.nl) {
-#pragma unroll
-          for (int b = 0; b < B; ++b) dst[b * step] = r[b];
-        } else {
-#pragma unroll
-          for (int b = 0; b < B; ++b)
-            if (b * STEP < left) dst[b * step] = r[b];
-        }
-        dst += B * step;
-      }
-    }
-  }
+  Rows::write(a, stage, c0, tid);
 }
 
-template <typename T, typename OutT, int R, int P>
+template <typename T, typename OutT, int R, int P, int W = 4>
 hipError_t launch_one(const TimeArgs& a, bool subtract_mean, hipStream_t s) {
-  using Lay = WaveLay<R, P>;
+  using Lay = WaveLay<R, P, W>;
   const int wgs = (a.cols + Lay::Q - 1) / Lay::Q;
   const int wpx = (wgs + 7) / 8;
-  auto kernel = k_time_wave<T, OutT, R, P>;
+  auto kernel = k_time_wave<T, OutT, R, P, W>;
   if (Lay::bytes > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(Lay::bytes));
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kernel, dim3(8u * wpx), dim3(64 * kWaves), Lay::bytes, s, a, wpx, wgs, subtract_mean ? 1 : 0);
+  hipLaunchKernelGGL(kernel, dim3(8u * wpx), dim3(64 * W), Lay::bytes, s, a, wpx, wgs, subtract_mean ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -648,7 +392,7 @@ hipError_t launch_logm(const TimeArgs& a, int logm, bool sub, hipStream_t s) {
     case 7: return launch_one<T, OutT, 8, 16>(a, sub, s);
     case 8: return launch_one<T, OutT, 16, 16>(a, sub, s);
     case 9: return launch_one<T, OutT, 16, 32>(a, sub, s);
-    case 10: return launch_one<T, OutT, 16, 64>(a, sub, s);
+    case 10: return launch_one<T, OutT, 16, 64, sizeof(T) == 4 ? 8 : 4>(a, sub, s);
     case 11:
       if constexpr (sizeof(T) == 4) return launch_one<T, OutT, 32, 64>(a, sub, s);
       return hipErrorInvalidValue;
@@ -663,37 +407,11 @@ int time_wave_max_log(int precision) { return precision == PREC_FP64 ? 10 : 11; 
 std::vector<unsigned char> time_wave_tables(int logm, int precision, uint64_t L) {
   const long long M = 1ll << logm;
   const int R = logm == 7 ? 8 : logm <= 10 ? 16 : 32;
-  const long long P = M / R;
-  const long double two_pi = 6.283185307179586476925286766559005768L;
   const bool f64 = precision == PREC_FP64;
   std::vector<unsigned char> out;
-  auto put = [&](long double v, bool dbl) {
-    const double d = static_cast<double>(v);
-    const float f = static_cast<float>(v);
-    const unsigned char* b = dbl ? reinterpret_cast<const unsigned char*>(&d) : reinterpret_cast<const unsigned char*>(&f);
-    out.insert(out.end(), b, b + (dbl ? 8 : 4));
-  };
-  auto w = [&](long double num, long double den) {
-    const long double ang = -two_pi * num / den;
-    put(cosl(ang), f64);
-    put(sinl(ang), f64);
-  };
-  for (long long k = 0; k < R; ++k)
-    for (long long p = 0; p < P; ++p) w(static_cast<long double>(p * k), static_cast<long double>(M));
-  for (long long k = 0; k < R; ++k)
-    for (long long p = 0; p < P; ++p) w(static_cast<long double>(p * (2 * k + 1)), static_cast<long double>(2 * M));
-  if (R == 32) {
-    for (long long j = 0; j < R; ++j) w(static_cast<long double>(j), static_cast<long double>(P));
-  } else if (P > R) {
-    for (long long k = 0; k < R; ++k)
-      for (long long p0 = 0; p0 < P / R; ++p0) w(static_cast<long double>(p0 * k), static_cast<long double>(P));
-  }
-  for (long long d = 0; d < M / 2; ++d) {
-    const long double ang = two_pi * static_cast<long double>(d) / static_cast<long double>(2 * M);
-    put(cosl(ang), f64);
-    put(sinl(ang), f64);
-  }
-  for (uint64_t d = 0; d < static_cast<uint64_t>(M); ++d) put(d < L ? 1.0L / static_cast<long double>(L - d) : 0.0L, true);
+  put_transform(out, M, M / R, f64, true);
+  for (long long d = 0; d < M / 2; ++d) put_root(out, -d, 2 * M, f64);
+  put_reciprocals(out, M, L);
   return out;
 }
 

@@ -10,9 +10,9 @@ from oracle import oracle_np as onp
 
 pytestmark = pytest.mark.gpu
 
-# series of every transform length M = 128 ... 2048: its shortest, one with a
+# series of every transform length M = 128 ... 4096: its shortest, one with a
 # remainder, its longest
-LENGTHS = [2, 3, 33, 64, 65, 127, 128, 129, 200, 256, 257, 300, 512, 513, 700, 1024, 1025, 1500, 2048]
+LENGTHS = [2, 3, 33, 64, 65, 127, 128, 129, 200, 256, 257, 300, 512, 513, 700, 1024, 1025, 1500, 2048, 2049, 3000, 4096]
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
