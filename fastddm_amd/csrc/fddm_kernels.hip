@@ -6,9 +6,9 @@
 //   k_cols  stage (a) column pass + stage (b) transpose: length-ny FFT of Tb
 //           frames of one kx column at once, store q-major S[q][t] in runs of
 //           Tb consecutive frames.
-//   k_diff  stage (d) + (e): direct lag differences, one wave per q, PS and VAR.
 //
-// The fft-mode time stage lives in fddm_time_p2.hip (power-of-two lengths).
+// The time stages live in fddm_time_wave.hip, fddm_time_pair.hip,
+// fddm_time_p2.hip and fddm_time_long.hip (fft mode) and fddm_diff.hip.
 //
 // Semantics follow the reference cores: spectra and normalisation
 // src/cpp/ddm.cc:288-323, correlation and two-ended sums ddm.cc:344-426,
@@ -17,12 +17,10 @@
 
 #include "fddm_fft.hpp"
 #include "fddm_kernels.hpp"
-#include "fddm_wave.hpp"
 
 namespace fddm {
 
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
 
 int fft_bucket(long long work) {
   const long long e = (work + kThreads - 1) / kThreads;
@@ -153,131 +151,6 @@ __global__ void __launch_bounds__(kThreads) k_cols(ColArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Stage (d)+(e): direct differences.  A wave works on QPW q at once, one per
-// segment of SEG = 64 / QPW lanes (QPW = 4: one q per 16-lane DPP row, 2: one
-// per half wave); the
-// segment's series sits in its own LDS slice when the workgroup's slices fit
-// 64 KiB (else it is read from L2).  Lane l of a segment takes t = l, l + SEG,
-// ...; lags go in batches of kLagBatch, so each F(t) load serves kLagBatch
-// differences, and each lag's SEG partial sums are added by a DPP scan inside
-// the segment, whose last lane writes D: one 4-step scan serves four q, one
-// 5-step scan two.  Differences are formed after widening to Acc, so they are exact on
-// the compensated paths.
-// ---------------------------------------------------------------------------
-constexpr int kLagBatch = 4;
-
-// Inclusive scan inside segments of SEG lanes (16: DPP rows; 32: wave
-// halves, rows 1 and 3 adding the last lane of rows 0 and 2; 64: the wave).
-template <int SEG, typename A>
-__device__ __forceinline__ A seg_total_scan(A v) {
-  if constexpr (SEG == 64) {
-    return wave::incl_scan(v);
-  } else {
-    static_assert(SEG == 16 || SEG == 32, "segment");
-    v += wave::dpp_zero<wave::kRowShr1, 0xf>(v);
-    v += wave::dpp_zero<wave::kRowShr2, 0xf>(v);
-    v += wave::dpp_zero<wave::kRowShr4, 0xf>(v);
-    v += wave::dpp_zero<wave::kRowShr8, 0xf>(v);
-    if constexpr (SEG == 32) v += wave::dpp_zero<wave::kRowBcast15, 0xa>(v);
-    return v;
-  }
-}
-
-template <typename T, typename OutT, int PREC, bool USE_LDS, int QPW>
-__global__ void __launch_bounds__(kThreads) k_diff(TimeArgs a, int wg_per_xcd, int nq) {
-  using C = cplx_t<T>;
-  using Acc = std::conditional_t<PREC == PREC_FP32, float, double>;
-  constexpr int SEG = 64 / QPW;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int sl = lane & (SEG - 1), seg = lane / SEG;
-  // columns of the launch (nq of them): cw is this wave's first
-  const int cw = ((blockIdx.x & 7) * wg_per_xcd + (blockIdx.x >> 3)) * kWaves * QPW + wid * QPW;
-  if (cw >= nq) return;  // whole waves: nothing below synchronises the workgroup
-  const int c = cw + seg;
-  const bool valid = c < nq;
-  const int q = col_q(a, valid ? c : cw);
-  const int L = a.L, Lv = valid ? L : 0;  // segments past the last column run empty loops
-  const C* __restrict__ src = static_cast<const C*>(a.S) + static_cast<size_t>(q - a.s_q0) * a.Lp;
-  const C* ser = src;
-  if constexpr (USE_LDS) {
-    C* slice = reinterpret_cast<C*>(smem) + static_cast<size_t>(wid * QPW + seg) * L;
-    for (int t0 = sl; t0 < Lv; t0 += 4 * SEG) {  // four loads in flight per lane
-      C v[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = t0 + SEG * k < Lv ? src[t0 + SEG * k] : C{0, 0};
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (t0 + SEG * k < Lv) slice[t0 + SEG * k] = v[k];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    ser = slice;
-  }
-  Acc sr = 0, si = 0, s2 = 0;
-  for (int t = sl; t < Lv; t += SEG) {
-    const C f = ser[t];
-    const Acc fx = static_cast<Acc>(f.x), fy = static_cast<Acc>(f.y);
-    sr += fx;
-    si += fy;
-    s2 += fx * fx + fy * fy;
-  }
-  sr = seg_total_scan<SEG>(sr);  // the segment's last lane holds the sums
-  si = seg_total_scan<SEG>(si);
-  s2 = seg_total_scan<SEG>(s2);
-  const bool writer = valid && sl == SEG - 1;
-
-  OutT* __restrict__ out = static_cast<OutT*>(a.out);
-  const size_t nqs = a.ldo;
-  const size_t oq = col_out(a, valid ? c : cw);
-  for (int i0 = 0; i0 < a.nl; i0 += kLagBatch) {
-    int d[kLagBatch];
-#pragma unroll
-    for (int k = 0; k < kLagBatch; ++k) d[k] = i0 + k < a.nl ? static_cast<int>(a.lags[i0 + k]) : L;
-    int dmin = d[0];
-#pragma unroll
-    for (int k = 1; k < kLagBatch; ++k) dmin = d[k] < dmin ? d[k] : dmin;
-    Acc acc[kLagBatch] = {};
-    for (int t = sl; t + dmin < Lv; t += SEG) {
-      const C v = ser[t];
-      const Acc vx = static_cast<Acc>(v.x), vy = static_cast<Acc>(v.y);
-#pragma unroll
-      for (int k = 0; k < kLagBatch; ++k) {
-        if (t + d[k] < L) {
-          const C u = ser[t + d[k]];
-          const Acc dr = static_cast<Acc>(u.x) - vx;
-          const Acc di = static_cast<Acc>(u.y) - vy;
-          acc[k] += dr * dr + di * di;
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kLagBatch; ++k) {
-      const Acc tot = seg_total_scan<SEG>(acc[k]);
-      if (writer && i0 + k < a.nl)
-        out[static_cast<size_t>(i0 + k) * nqs + oq] = static_cast<OutT>(tot / static_cast<Acc>(L - d[k]));
-    }
-  }
-  if (writer) {
-    const Acc mr = sr / L, mi = si / L;
-    Acc ps, var;
-    if (a.S0) {
-      // spectra hold F(t) - F(0): VAR is shift invariant, PS adds |F(0) + mean|^2
-      var = s2 / L - (mr * mr + mi * mi);
-      const C z = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
-      const Acc fr = mr + static_cast<Acc>(z.x), fi = mi + static_cast<Acc>(z.y);
-      ps = var + fr * fr + fi * fi;
-    } else {
-      ps = s2 / L;
-      var = ps - mr * mr - mi * mi;
-    }
-    out[static_cast<size_t>(a.nl) * nqs + oq] = static_cast<OutT>(ps);
-    out[static_cast<size_t>(a.nl + 1) * nqs + oq] = static_cast<OutT>(var);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // FFT engine test kernel: one forward transform per workgroup, in place.
 // ---------------------------------------------------------------------------
 template <typename T, int E>
@@ -366,37 +239,6 @@ hipError_t launch_cols(const ColArgs& a, int precision, hipStream_t s) {
     if (e == 32) return launch(k_cols<float, 32>, grid, lds, s, a);
   }
   return hipErrorInvalidValue;
-}
-
-namespace {
-// The most q per wave (4, 2, 1) whose staged series leave room for 8
-// workgroups (32 waves) per CU; else one q per wave, LDS-staged while the
-// workgroup's four series fit 64 KiB, else read from L2.
-template <typename T, typename OutT, int PREC>
-hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
-  const int nq = a.cols;
-  const size_t series = sizeof(cplx_t<T>) * a.L;
-  constexpr size_t kFull = 160 * 1024 / 8;  // LDS per workgroup at 8 workgroups per CU
-  auto go = [&](auto kernel, int qpw, size_t lds) {
-    const int wgs = (nq + kWaves * qpw - 1) / (kWaves * qpw);
-    const int wpx = (wgs + 7) / 8;
-    return launch(kernel, static_cast<unsigned>(wpx) * 8u, lds, s, a, wpx, nq);
-  };
-  if (series * kWaves * 4 <= kFull) return go(k_diff<T, OutT, PREC, true, 4>, 4, series * kWaves * 4);
-  if (series * kWaves * 2 <= kFull) return go(k_diff<T, OutT, PREC, true, 2>, 2, series * kWaves * 2);
-  if (series * kWaves <= 64 * 1024) return go(k_diff<T, OutT, PREC, true, 1>, 1, series * kWaves);
-  return go(k_diff<T, OutT, PREC, false, 1>, 1, 0);
-}
-}  // namespace
-
-hipError_t launch_diff(const TimeArgs& a, int precision, int out_dtype, hipStream_t s) {
-  const bool f32 = out_dtype == OUT_F32;
-  switch (precision) {
-    case PREC_FP64: return f32 ? diff_l<double, float, PREC_FP64>(a, s) : diff_l<double, double, PREC_FP64>(a, s);
-    case PREC_FP32: return f32 ? diff_l<float, float, PREC_FP32>(a, s) : diff_l<float, double, PREC_FP32>(a, s);
-    case PREC_FP32C: return f32 ? diff_l<float, float, PREC_FP32C>(a, s) : diff_l<float, double, PREC_FP32C>(a, s);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 hipError_t launch_fft_test(void* data, int n, int batch, const FftDesc& d, const void* tw, int precision,
