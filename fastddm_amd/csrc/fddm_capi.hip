@@ -54,10 +54,12 @@ struct fddm_plan {
   void* d_twt = nullptr;
   uint64_t bytes_R = 0, bytes_S = 0, bytes_S0 = 0, bytes_flags = 0, ws_bytes = 0;
   // Compensated FP32: child FP64 plan over the first and last kEdgeFrames
-  // frames (gathered into its own input unless the stack is that short); the
-  // lags from index edge_i0 on have at most kEdgeFrames pairs.
+  // frames; the lags from index edge_i0 on have at most kEdgeFrames pairs.
+  // The child also transforms the raw first frame (its frame raw_at), whose
+  // spectrum PS needs; without a child the plan does that itself (S0).
   fddm_plan* edge = nullptr;
-  uint64_t edge_frames = 0, bytes_edge_in = 0, bytes_edge_ws = 0;
+  uint64_t edge_frames = 0, bytes_edge_ws = 0;
+  uint64_t raw_at = 0;  // child plan: index of the raw first frame (0: none)
   int edge_i0 = 0;
   // timing
   std::vector<hipEvent_t> events;
@@ -424,7 +426,8 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
   }
   p->bytes_R = align256(p->nblocks * p->nxh * H * p->Tb * csz);
   p->bytes_S = align256(p->nq * p->Lp * csz);
-  p->bytes_S0 = p->subtract0 ? align256(p->nq * p->Tb * csz) : 0;
+  const bool has_edge = precision == PREC_FP32C && nl > 0 && L - lags[nl - 1] <= static_cast<uint64_t>(kEdgeFrames);
+  p->bytes_S0 = p->subtract0 && !has_edge ? align256(p->nq * p->Tb * csz) : 0;
   // fft mode, compensated: one byte per q marks lags for the direct recomputation
   p->bytes_flags = (mode == MODE_FFT && precision == PREC_FP32C) ? align256(p->nq) : 0;
   if (p->long_t) {
@@ -434,16 +437,23 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     p->bytes_long = align256(p->long_slot * static_cast<uint64_t>(p->long_slots));
   }
   p->ws_bytes = p->bytes_R + p->bytes_S + p->bytes_S0 + p->bytes_flags + p->bytes_long;
-  if (precision == PREC_FP32C && nl > 0 && L - lags[nl - 1] <= static_cast<uint64_t>(kEdgeFrames)) {
+  if (has_edge) {
     // FP64 spectra of the edge frames for the lags with few pairs
     const uint64_t E = kEdgeFrames;
     p->edge_frames = std::min<uint64_t>(L, 2 * E);
     if ((rc = plan_create_ex(&p->edge, MODE_DIFF, dtype, p->edge_frames, H, W, nullptr, 0, nx, ny, 0, window,
                              window_f32, PREC_FP64, OUT_F64, 0, err, errlen)))
       return fail(rc);
-    p->bytes_edge_in = L > 2 * E ? align256(2 * E * H * W * in_bytes(dtype)) : 0;
-    p->bytes_edge_ws = p->edge->ws_bytes;
-    p->ws_bytes += p->bytes_edge_in + p->bytes_edge_ws;
+    fddm_plan* c = p->edge;
+    c->raw_at = (p->edge_frames + 1) / 2 * 2;  // (even: a pair of its own)
+    c->nblocks = (c->raw_at + 1 + c->Tb - 1) / c->Tb;
+    c->Lp = c->nblocks * c->Tb;
+    c->bytes_R = align256(c->nblocks * c->nxh * H * c->Tb * 16);
+    c->bytes_S = align256(c->nq * c->Lp * 16);
+    c->bytes_S0 = 0;
+    c->ws_bytes = c->bytes_R + c->bytes_S;
+    p->bytes_edge_ws = c->ws_bytes;
+    p->ws_bytes += p->bytes_edge_ws;
     p->edge_i0 = static_cast<int>(nl);
     while (p->edge_i0 > 0 && L - lags[p->edge_i0 - 1] <= E) --p->edge_i0;
   }
@@ -471,17 +481,9 @@ hipError_t launch_time(const fddm_plan* p, const TimeArgs& ta, hipStream_t s) {
   return launch_time_pair(ta, p->precision, p->out_dtype, s);
 }
 
-int run_spatial(fddm_plan* p, const void* d_img, void* ws, hipStream_t s, char* err, size_t errlen) {
-  auto* base = static_cast<unsigned char*>(ws);
-  void* R = base;
-  void* S = base + p->bytes_R;
-  void* S0 = base + p->bytes_R + p->bytes_S;
-  const double norm = 1.0 / std::sqrt(static_cast<double>(p->nx) * static_cast<double>(p->ny));
+RowArgs row_args(const fddm_plan* p) {
   RowArgs ra{};
-  ra.img = d_img;
-  ra.img0 = d_img;
   ra.in_dtype = p->in_dtype;
-  ra.L = p->L;
   ra.H = static_cast<int>(p->H);
   ra.W = static_cast<int>(p->W);
   ra.nx = static_cast<int>(p->nx);
@@ -489,13 +491,15 @@ int run_spatial(fddm_plan* p, const void* d_img, void* ws, hipStream_t s, char* 
   ra.G = p->Gx;
   ra.window = p->d_window;
   ra.logn = p->logn_x;
-  ra.norm = norm;
+  ra.norm = 1.0 / std::sqrt(static_cast<double>(p->nx) * static_cast<double>(p->ny));
   ra.dx = p->dx;
   ra.twx = p->d_twx;
-  ra.R = R;
   ra.generic = p->rows_generic;
+  return ra;
+}
+
+ColArgs col_args(const fddm_plan* p) {
   ColArgs ca{};
-  ca.R = R;
   ca.H = static_cast<int>(p->H);
   ca.ny = static_cast<int>(p->ny);
   ca.nxh = static_cast<int>(p->nxh);
@@ -505,29 +509,95 @@ int run_spatial(fddm_plan* p, const void* d_img, void* ws, hipStream_t s, char* 
   ca.dy = p->dy;
   ca.twy = p->d_twy;
   ca.generic = p->cols_generic;
-  int rc;
-  if ((rc = record(p, 0, s, err, errlen))) return rc;
-  if (p->subtract0) {
-    // F(0) of the raw first frame, for the power spectrum.
-    ra.frames = 1;
-    ra.subtract0 = 0;
-    FDDM_HIP(ra.logn ? launch_rows_p2(ra, p->precision, s) : launch_rows(ra, p->precision, s));
-    ca.nblocks = 1;
-    ca.Lp = static_cast<uint64_t>(p->Tb);
-    ca.S = S0;
-    FDDM_HIP(ca.logn ? launch_cols_p2(ca, p->precision, s) : launch_cols(ca, p->precision, s));
+  return ca;
+}
+
+// Rows and columns of `frames` frames at img (frame I0 at img0 subtracted when
+// sub), blocks of Tb frames into S_dst[q][t] with row pitch `pitch`.
+int spatial_frames(const fddm_plan* p, const void* img, const void* img0, uint64_t frames, int sub, void* R,
+                   void* S_dst, uint64_t pitch, hipStream_t s, char* err, size_t errlen) {
+  RowArgs ra = row_args(p);
+  ra.img = img;
+  ra.img0 = img0;
+  ra.L = frames;
+  ra.frames = frames;
+  ra.subtract0 = sub;
+  ra.R = R;
+  FDDM_HIP(ra.logn ? launch_rows_p2(ra, p->precision, s) : launch_rows(ra, p->precision, s));
+  ColArgs ca = col_args(p);
+  ca.R = R;
+  ca.nblocks = (frames + p->Tb - 1) / p->Tb;
+  ca.Lp = pitch;
+  ca.S = S_dst;
+  FDDM_HIP(ca.logn ? launch_cols_p2(ca, p->precision, s) : launch_cols(ca, p->precision, s));
+  return FDDM_OK;
+}
+
+// F(0) of the raw first frame, for PS: in the edge child's spectra, with the
+// edge frames, or by the plan itself into S0.  edge_src: the first and last
+// kEdgeFrames frames, or with in_stack the whole stack (from which the child's
+// rows read them).
+int frame0_stage(fddm_plan* p, const void* frame0, const void* edge_src, bool in_stack, void* R, void* S0, void* edge_ws,
+                 hipStream_t s, char* err, size_t errlen) {
+  if (!p->subtract0) return FDDM_OK;
+  if (!p->edge) return spatial_frames(p, frame0, frame0, 1, 0, R, S0, p->Tb, s, err, errlen);
+  const fddm_plan* c = p->edge;
+  RowArgs ra = row_args(c);
+  ra.img = edge_src;
+  ra.img0 = edge_src;
+  ra.L = c->L;
+  ra.frames = c->raw_at + 1;
+  ra.raw = c->raw_at;
+  if (in_stack && p->L > c->L) {
+    ra.split = kEdgeFrames;
+    ra.gap = p->L - c->L;
   }
-  if ((rc = record(p, 1, s, err, errlen))) return rc;
+  ra.subtract0 = 1;
+  ra.R = edge_ws;
+  FDDM_HIP(ra.logn ? launch_rows_p2(ra, c->precision, s) : launch_rows(ra, c->precision, s));
+  ColArgs ca = col_args(c);
+  ca.R = edge_ws;
+  ca.nblocks = c->nblocks;
+  ca.Lp = c->Lp;
+  ca.S = static_cast<unsigned char*>(edge_ws) + c->bytes_R;
+  FDDM_HIP(ca.logn ? launch_cols_p2(ca, c->precision, s) : launch_cols(ca, c->precision, s));
+  return FDDM_OK;
+}
+
+// Where the time stage finds F(0).
+void set_frame0(const fddm_plan* p, TimeArgs& ta, const void* S0, const void* edge_ws) {
+  if (!p->subtract0) return;
+  if (p->edge) {
+    ta.S0 = static_cast<const unsigned char*>(edge_ws) + p->edge->bytes_R + p->edge->raw_at * 16;
+    ta.s0_stride = p->edge->Lp;
+    ta.s0_f64 = 1;
+  } else {
+    ta.S0 = S0;
+    ta.s0_stride = static_cast<uint64_t>(p->Tb);
+  }
+}
+
+// Spatial stage of the whole stack into the workspace (R, S); the timing
+// events around the passes.
+int run_spatial(fddm_plan* p, const void* d_img, void* ws, hipStream_t s, char* err, size_t errlen) {
+  auto* base = static_cast<unsigned char*>(ws);
+  RowArgs ra = row_args(p);
+  ra.img = d_img;
+  ra.img0 = d_img;
+  ra.L = p->L;
   ra.frames = p->L;
   ra.subtract0 = p->subtract0 ? 1 : 0;
+  ra.R = base;
   FDDM_HIP(ra.logn ? launch_rows_p2(ra, p->precision, s) : launch_rows(ra, p->precision, s));
+  int rc;
   if ((rc = record(p, 2, s, err, errlen))) return rc;
+  ColArgs ca = col_args(p);
+  ca.R = base;
   ca.nblocks = p->nblocks;
   ca.Lp = p->Lp;
-  ca.S = S;
+  ca.S = base + p->bytes_R;
   FDDM_HIP(ca.logn ? launch_cols_p2(ca, p->precision, s) : launch_cols(ca, p->precision, s));
-  if ((rc = record(p, 3, s, err, errlen))) return rc;
-  return FDDM_OK;
+  return record(p, 3, s, err, errlen);
 }
 
 // The kernels read pixels in 8-byte vectors and write spectra in 16-byte
@@ -546,17 +616,21 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
                  size_t errlen) {
   if (!p || !d_img || !d_out || !ws) return set_err(err, errlen, FDDM_ERR_ARG, "NULL argument to execute");
   if (const int rc = check_alignment(p, d_img, d_out, ws, err, errlen)) return rc;
-  int rc = run_spatial(p, d_img, ws, s, err, errlen);
-  if (rc) return rc;
   auto* base = static_cast<unsigned char*>(ws);
+  unsigned char* const S0 = base + p->bytes_R + p->bytes_S;
+  unsigned char* const ews = base + p->ws_bytes - p->bytes_edge_ws;
+  int rc;
+  if ((rc = record(p, 0, s, err, errlen))) return rc;
+  if ((rc = frame0_stage(p, d_img, d_img, true, base, S0, ews, s, err, errlen))) return rc;
+  if ((rc = record(p, 1, s, err, errlen))) return rc;
+  if ((rc = run_spatial(p, d_img, ws, s, err, errlen))) return rc;
   TimeArgs ta{};
   ta.S = base + p->bytes_R;
   ta.Lp = p->Lp;
   ta.L = static_cast<int>(p->L);
   ta.ny = static_cast<int>(p->ny);
   ta.nxh = static_cast<int>(p->nxh);
-  ta.S0 = p->subtract0 ? base + p->bytes_R + p->bytes_S : nullptr;
-  ta.s0_stride = static_cast<uint64_t>(p->Tb);
+  set_frame0(p, ta, S0, ews);
   ta.lags = static_cast<const uint32_t*>(p->d_lags);
   ta.nl = static_cast<int>(p->nl);
   ta.dt = p->dt;
@@ -577,22 +651,8 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
   // compensated FP32 corrections: flagged Wiener-Khinchin lags, then the lags
   // with at most kEdgeFrames pairs from FP64 spectra
   if (ta.flags) FDDM_HIP(launch_wk_fix(ta, p->out_dtype, s));
-  if (p->edge) {
-    // FP64 spectra of the edge frames, then the few-pair lags from them
-    unsigned char* ein = base + p->ws_bytes - p->bytes_edge_ws - p->bytes_edge_in;
-    unsigned char* ews = base + p->ws_bytes - p->bytes_edge_ws;
-    const void* src = d_img;
-    if (p->bytes_edge_in) {
-      FDDM_HIP(launch_gather_edges(d_img, ein, p->H * p->W * in_bytes(p->in_dtype), p->L, kEdgeFrames, s));
-      src = ein;
-    }
-    const int cap = p->edge->timing_cap;
-    p->edge->timing_cap = 0;
-    rc = run_spatial(p->edge, src, ews, s, err, errlen);
-    p->edge->timing_cap = cap;
-    if (rc) return rc;
+  if (p->edge)
     FDDM_HIP(launch_edge_fix(ta, ews + p->edge->bytes_R, p->edge->Lp, kEdgeFrames, p->edge_i0, p->out_dtype, s));
-  }
   if ((rc = record(p, 5, s, err, errlen))) return rc;
   if (p->timing_cap > 0 && p->timing_steps < p->timing_cap) ++p->timing_steps;
   return FDDM_OK;
@@ -764,58 +824,6 @@ bool plan_chunks(const fddm_plan* p, uint64_t budget, ChunkPlan* cp) {
   return false;
 }
 
-RowArgs row_args(const fddm_plan* p) {
-  RowArgs ra{};
-  ra.in_dtype = p->in_dtype;
-  ra.H = static_cast<int>(p->H);
-  ra.W = static_cast<int>(p->W);
-  ra.nx = static_cast<int>(p->nx);
-  ra.Tb = p->Tb;
-  ra.G = p->Gx;
-  ra.window = p->d_window;
-  ra.logn = p->logn_x;
-  ra.norm = 1.0 / std::sqrt(static_cast<double>(p->nx) * static_cast<double>(p->ny));
-  ra.dx = p->dx;
-  ra.twx = p->d_twx;
-  ra.generic = p->rows_generic;
-  return ra;
-}
-
-ColArgs col_args(const fddm_plan* p) {
-  ColArgs ca{};
-  ca.H = static_cast<int>(p->H);
-  ca.ny = static_cast<int>(p->ny);
-  ca.nxh = static_cast<int>(p->nxh);
-  ca.Tb = p->Tb;
-  ca.G = p->Gy;
-  ca.logn = p->logn_y;
-  ca.dy = p->dy;
-  ca.twy = p->d_twy;
-  ca.generic = p->cols_generic;
-  return ca;
-}
-
-// Rows and columns of `frames` frames at img (frame I0 at img0 subtracted when
-// sub), blocks of Tb frames into S_dst[q][t] with row pitch `pitch`.
-int spatial_frames(const fddm_plan* p, const void* img, const void* img0, uint64_t frames, int sub, void* R,
-                   void* S_dst, uint64_t pitch, hipStream_t s, char* err, size_t errlen) {
-  RowArgs ra = row_args(p);
-  ra.img = img;
-  ra.img0 = img0;
-  ra.L = frames;
-  ra.frames = frames;
-  ra.subtract0 = sub;
-  ra.R = R;
-  FDDM_HIP(ra.logn ? launch_rows_p2(ra, p->precision, s) : launch_rows(ra, p->precision, s));
-  ColArgs ca = col_args(p);
-  ca.R = R;
-  ca.nblocks = (frames + p->Tb - 1) / p->Tb;
-  ca.Lp = pitch;
-  ca.S = S_dst;
-  FDDM_HIP(ca.logn ? launch_cols_p2(ca, p->precision, s) : launch_cols(ca, p->precision, s));
-  return FDDM_OK;
-}
-
 // Time stage and corrections of one launch range (ta.c0, ta.cols, ...).
 int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* edge_S64, hipStream_t s, char* err,
                 size_t errlen) {
@@ -891,7 +899,7 @@ PlanInfo fddm::plan_info(const fddm_plan* p) {
 }
 
 // The stages after the spatial pass over every frame: F(0) from frame0, the
-// FP64 edge spectra from edge_in (the child's frames, or gathered from img
+// FP64 edge spectra from edge_in (the child's frames, or from the stack at img
 // when edge_in is null), then the time stage and its corrections over the
 // whole plane in launches of cols_per columns.
 int finish_from_spectra(fddm_plan* p, const void* frame0, const void* img, const void* edge_in, void* ws,
@@ -903,33 +911,17 @@ int finish_from_spectra(fddm_plan* p, const void* frame0, const void* img, const
   unsigned char* flags = S0 + p->bytes_S0;
   unsigned char* lng = flags + p->bytes_flags;
   const int nq = static_cast<int>(p->nq);
-  const int sub = p->subtract0 ? 1 : 0;
+  unsigned char* const ews = base + p->ws_bytes - p->bytes_edge_ws;
   int rc;
-  if (sub && (rc = spatial_frames(p, frame0, frame0, 1, 0, R, S0, p->Tb, s, err, errlen))) return rc;
-  const void* S64 = nullptr;
-  if (p->edge) {
-    unsigned char* ein = base + p->ws_bytes - p->bytes_edge_ws - p->bytes_edge_in;
-    unsigned char* ews = base + p->ws_bytes - p->bytes_edge_ws;
-    const void* src = edge_in ? edge_in : img;
-    if (!edge_in && p->bytes_edge_in) {
-      FDDM_HIP(launch_gather_edges(img, ein, p->H * p->W * in_bytes(p->in_dtype), p->L, kEdgeFrames, s));
-      src = ein;
-    }
-    const int cap = p->edge->timing_cap;
-    p->edge->timing_cap = 0;
-    rc = run_spatial(p->edge, src, ews, s, err, errlen);
-    p->edge->timing_cap = cap;
-    if (rc) return rc;
-    S64 = ews + p->edge->bytes_R;
-  }
+  if ((rc = frame0_stage(p, frame0, edge_in ? edge_in : img, !edge_in, R, S0, ews, s, err, errlen))) return rc;
+  const void* S64 = p->edge ? ews + p->edge->bytes_R : nullptr;
   TimeArgs ta{};
   ta.S = S;
   ta.Lp = p->Lp;
   ta.L = static_cast<int>(p->L);
   ta.ny = static_cast<int>(p->ny);
   ta.nxh = static_cast<int>(p->nxh);
-  ta.S0 = sub ? S0 : nullptr;
-  ta.s0_stride = static_cast<uint64_t>(p->Tb);
+  set_frame0(p, ta, S0, ews);
   ta.lags = static_cast<const uint32_t*>(p->d_lags);
   ta.nl = static_cast<int>(p->nl);
   ta.dt = p->dt;
@@ -1008,9 +1000,8 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
   const int sub = p->subtract0 ? 1 : 0;
   int rc;
 
-  // frame 0 (the subtracted frame) and its raw spectrum F(0) for PS
+  // frame 0 (the subtracted frame)
   FDDM_HIP(hipMemcpyAsync(frame0, img, frame_b, hipMemcpyHostToDevice, s));
-  if (sub && (rc = spatial_frames(p, frame0, frame0, 1, 0, work, S0, p->Tb, s, err, errlen))) return rc;
   // spatial stage in chunks of whole frame blocks
   uint64_t nchunks = 0;
   for (uint64_t t0 = 0; t0 < p->L; t0 += cp.frames_per, ++nchunks) {
@@ -1032,7 +1023,7 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
     }
     if (rc) return rc;
   }
-  // FP64 spectra of the edge frames (compensated path)
+  // raw spectrum F(0) for PS and FP64 spectra of the edge frames (compensated path)
   if (p->edge) {
     // the first and last kEdgeFrames frames (every frame of a short stack)
     const uint64_t E = kEdgeFrames;
@@ -1043,12 +1034,8 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
     } else {
       FDDM_HIP(hipMemcpyAsync(ein, img, p->L * frame_b, hipMemcpyHostToDevice, s));
     }
-    const int cap = p->edge->timing_cap;
-    p->edge->timing_cap = 0;
-    rc = run_spatial(p->edge, ein, ews, s, err, errlen);
-    p->edge->timing_cap = cap;
-    if (rc) return rc;
   }
+  if ((rc = frame0_stage(p, frame0, ein, false, work, S0, ews, s, err, errlen))) return rc;
   FDDM_HIP(hipStreamSynchronize(s));  // the work region is reused by the time chunks
 
   // time stage in chunks of whole ky rows, local (unshifted) pieces
@@ -1057,8 +1044,7 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
   ta.L = static_cast<int>(p->L);
   ta.ny = static_cast<int>(p->ny);
   ta.nxh = static_cast<int>(p->nxh);
-  ta.S0 = sub ? S0 : nullptr;
-  ta.s0_stride = static_cast<uint64_t>(p->Tb);
+  set_frame0(p, ta, S0, ews);
   ta.lags = static_cast<const uint32_t*>(p->d_lags);
   ta.nl = static_cast<int>(p->nl);
   ta.dt = p->dt;

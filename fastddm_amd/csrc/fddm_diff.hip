@@ -87,7 +87,7 @@ __device__ __forceinline__ void store_moments(const TimeArgs& a, int q, size_t o
   if (a.S0) {
     // spectra hold F(t) - F(0): VAR is shift invariant, PS adds |F(0) + mean|^2
     var = s2 / L - (mr * mr + mi * mi);
-    const C z = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
+    const C z = frame0_spectrum<C>(a, q);
     const Acc fr = mr + static_cast<Acc>(z.x), fi = mi + static_cast<Acc>(z.y);
     ps = var + fr * fr + fi * fi;
   } else {

@@ -8,7 +8,8 @@
 // For n >= 2 all n differences would have to be small at once, which does
 // not happen at these sizes.  So the first and last kEdgeFrames frames are
 // transformed once more in FP64 (a child plan over those frames, frame-0
-// subtracted like the main pass), and the lags with n <= kEdgeFrames are
+// subtracted like the main pass, whose rows read them where they lie; the raw
+// first frame is transformed beside them, for PS), and the lags with n <= kEdgeFrames are
 // recomputed from them by direct sums in FP64, after the time / diff kernel
 // has written its own values.
 //
@@ -28,24 +29,6 @@ namespace fddm {
 namespace {
 
 constexpr int kThreads = 256;
-
-// Copies frames [0, e) and [L - e, L) of an (L, frame_bytes) stack into dst,
-// 8 bytes per lane when the frame size allows it.
-__global__ void __launch_bounds__(kThreads)
-    k_gather_edges(const unsigned char* __restrict__ src, unsigned char* __restrict__ dst, uint64_t head_bytes,
-                   uint64_t tail_src_off, uint64_t total_bytes, int wide) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kThreads;
-  const uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (wide) {
-    const uint64_t n = total_bytes / 8, head = head_bytes / 8, toff = tail_src_off / 8;
-    const auto* s = reinterpret_cast<const uint64_t*>(src);
-    auto* d = reinterpret_cast<uint64_t*>(dst);
-    for (uint64_t i = i0; i < n; i += stride) d[i] = s[i < head ? i : i - head + toff];
-  } else {
-    for (uint64_t i = i0; i < total_bytes; i += stride)
-      dst[i] = src[i < head_bytes ? i : i - head_bytes + tail_src_off];
-  }
-}
 
 // One thread per output column o (y-shifted q): for every lag index i >= i0
 // (those with n = L - lags[i] <= E), D = sum_{t < n} |F(t + dt) - F(t)|^2 / n
@@ -176,21 +159,6 @@ hipError_t launch_wk_fix(const TimeArgs& a, int out_dtype, hipStream_t s) {
   } else {
     hipLaunchKernelGGL(k_wk_fix<double>, grid, dim3(kThreads), 0, s, a);
   }
-  return hipGetLastError();
-}
-
-hipError_t launch_gather_edges(const void* img, void* dst, uint64_t frame_bytes, uint64_t L, uint64_t E,
-                               hipStream_t s) {
-  const uint64_t head = E * frame_bytes, total = 2 * E * frame_bytes, toff = (L - E) * frame_bytes;
-  const int wide = (frame_bytes % 8 == 0 && reinterpret_cast<uintptr_t>(img) % 8 == 0 &&
-                    reinterpret_cast<uintptr_t>(dst) % 8 == 0)
-                       ? 1
-                       : 0;
-  const uint64_t items = wide ? total / 8 : total;
-  const unsigned blocks = static_cast<unsigned>(std::min<uint64_t>((items + kThreads - 1) / kThreads, 4096));
-  hipLaunchKernelGGL(k_gather_edges, dim3(blocks ? blocks : 1), dim3(kThreads), 0, s,
-                     static_cast<const unsigned char*>(img), static_cast<unsigned char*>(dst), head, toff, total,
-                     wide);
   return hipGetLastError();
 }
 

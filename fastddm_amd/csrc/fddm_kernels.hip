@@ -17,6 +17,7 @@
 
 #include "fddm_fft.hpp"
 #include "fddm_kernels.hpp"
+#include "fddm_spatial.hpp"
 
 namespace fddm {
 
@@ -81,7 +82,6 @@ __global__ void __launch_bounds__(kThreads) k_rows(RowArgs a) {
   const int bstride = nx + 1;
   const size_t plane = static_cast<size_t>(H) * W;
   C* __restrict__ R = static_cast<C*>(a.R);
-  const bool sub = a.subtract0 != 0;
   const C* __restrict__ tw = static_cast<const C*>(a.twx);
 
   for (int g0 = 0; g0 < Tb / 2; g0 += G) {
@@ -91,8 +91,10 @@ __global__ void __launch_bounds__(kThreads) k_rows(RowArgs a) {
       if (x < W) {
         const uint64_t ta = t0 + 2 * (g0 + p), tb2 = ta + 1;
         const size_t i0 = static_cast<size_t>(y) * W + x;
-        if (ta < a.frames) va = load_pixel<Tin, T>(img, ref, ta * plane + i0, i0, sub);
-        if (tb2 < a.frames) vb = load_pixel<Tin, T>(img, ref, tb2 * plane + i0, i0, sub);
+        if (sp::frame_here(a, ta))
+          va = load_pixel<Tin, T>(img, ref, sp::frame_src(a, ta) * plane + i0, i0, sp::frame_sub(a, ta));
+        if (sp::frame_here(a, tb2))
+          vb = load_pixel<Tin, T>(img, ref, sp::frame_src(a, tb2) * plane + i0, i0, sp::frame_sub(a, tb2));
         if (win) {
           const T wv = win[i0];
           va *= wv;

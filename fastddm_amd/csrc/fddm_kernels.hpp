@@ -12,14 +12,17 @@ namespace fddm {
 // the blocked layout R[tb][kx][y][ti] (t = tb * Tb + ti, kx < nx/2+1, y < H).
 // `window` (H*W of T) may be null.  subtract0: use I(t) - I0 in place of I(t),
 // where I0 is the frame at img0 (the stack's frame 0; img itself when the
-// launch starts at frame 0).  `frames` limits how many leading frames of img
-// are transformed (>= 1).
+// launch starts at frame 0).  `frames` limits how many leading frames are
+// transformed (>= 1).  Frames t >= split come from frame t + gap of img, and
+// frame t == raw (> 0; none: 0) is frame 0 of img without the subtraction
+// (frame_src, frame_here, frame_sub in fddm_spatial.hpp).
 struct RowArgs {
   const void* img;
   const void* img0;
   int in_dtype;
-  uint64_t L;       // frames present in img
-  uint64_t frames;  // frames to transform (<= L)
+  uint64_t L;       // frames present (t < L; besides raw)
+  uint64_t frames;  // frames to transform
+  uint64_t split, gap, raw;
   int H, W, nx, Tb, G;
   int logn;  // > 0: power-of-two kernel for nx = 2^logn (twx holds its tables)
   const void* window;
@@ -51,8 +54,9 @@ struct TimeArgs {
   const void* S;
   uint64_t Lp;
   int L, ny, nxh;
-  const void* S0;  // frame-0 spectra (stride s0_stride) or null
+  const void* S0;  // frame-0 spectra (stride s0_stride, in double when s0_f64) or null
   uint64_t s0_stride;
+  int s0_f64;
   const uint32_t* lags;
   int nl;
   FftDesc dt;
@@ -85,6 +89,17 @@ __device__ __forceinline__ int col_q(const TimeArgs& a, int c) {
 }
 __device__ __forceinline__ size_t col_out(const TimeArgs& a, int c) {
   return static_cast<size_t>(a.local ? c : a.c0 + c);
+}
+
+// F(0) of the raw first frame at q, in the compute type (zero without S0).
+template <typename C>
+__device__ __forceinline__ C frame0_spectrum(const TimeArgs& a, int q) {
+  if (!a.S0) return C{0, 0};
+  const size_t i = static_cast<size_t>(q) * a.s0_stride;
+  if (!a.s0_f64) return static_cast<const C*>(a.S0)[i];
+  const double2 z = static_cast<const double2*>(a.S0)[i];
+  using T = decltype(C{}.x);
+  return C{static_cast<T>(z.x), static_cast<T>(z.y)};
 }
 
 hipError_t launch_rows(const RowArgs& a, int precision, hipStream_t s);
@@ -124,13 +139,10 @@ hipError_t launch_fft_test(void* data, int n, int batch, const FftDesc& d, const
 // (hipHostGetDevicePointer), by a kernel; n and both addresses multiples of 16.
 hipError_t launch_copy_out(void* dst, const void* src, uint64_t n, hipStream_t s);
 
-// FP64 edge correction of the compensated path (fddm_edge.hip): frames
-// [0, E) and [L - E, L) of an (L, frame_bytes) stack copied to dst, and the
-// lags lags[i0 .. nl) (n = L - dt <= E pairs) recomputed by direct sums from
-// the FP64 spectra S64[q][c] (pitch lp) of those frames into the y-shifted
-// output.
-hipError_t launch_gather_edges(const void* img, void* dst, uint64_t frame_bytes, uint64_t L, uint64_t E,
-                               hipStream_t s);
+// FP64 edge correction of the compensated path (fddm_edge.hip): the lags
+// lags[i0 .. nl) (n = L - dt <= E pairs) recomputed by direct sums from the
+// FP64 spectra S64[q][c] (pitch lp) of the first and last E frames into the
+// y-shifted output.
 hipError_t launch_edge_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype,
                            hipStream_t s);
 constexpr int kEdgeFrames = 8;

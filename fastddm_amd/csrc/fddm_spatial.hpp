@@ -3,10 +3,21 @@
 
 #include <type_traits>
 
-#include "fddm_common.hpp"
+#include "fddm_kernels.hpp"
 
 namespace fddm {
 namespace sp {
+
+// Frame t of a row launch: whether there is one, where it lies in img, and
+// whether frame 0 is subtracted from it (RowArgs: split, gap, raw).
+__device__ __forceinline__ bool frame_raw(const RowArgs& a, uint64_t t) { return t == a.raw && a.raw != 0; }
+__device__ __forceinline__ bool frame_here(const RowArgs& a, uint64_t t) {
+  return t < a.frames && (t < a.L || frame_raw(a, t));
+}
+__device__ __forceinline__ uint64_t frame_src(const RowArgs& a, uint64_t t) {
+  return frame_raw(a, t) ? 0 : t + (t >= a.split ? a.gap : 0);
+}
+__device__ __forceinline__ bool frame_sub(const RowArgs& a, uint64_t t) { return a.subtract0 != 0 && !frame_raw(a, t); }
 
 // Pixel (p, x) of a pair row: converted, frame 0 subtracted in integer
 // arithmetic where the type allows, times the window value.

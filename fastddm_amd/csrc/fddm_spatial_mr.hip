@@ -169,17 +169,20 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
     asm volatile("" : "+v"(lane), "+v"(tidi));
     const int y = static_cast<int>(static_cast<uint32_t>(item) % static_cast<uint32_t>(H));
     const uint64_t tb = static_cast<uint32_t>(item) / static_cast<uint32_t>(H), ta = tb * TB + 2 * p;
-    const bool has_a = ta < a.frames, has_b = ta + 1 < a.frames;  // uniform over the wave
+    // (uniform over the wave)
+    const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
+    const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
     const size_t yo = static_cast<size_t>(y) * W;
-    const Tin* __restrict__ ra = img + ta * plane + yo;
+    const Tin* __restrict__ ra = img + sp::frame_src(a, ta) * plane + yo;
+    const Tin* __restrict__ rb = img + sp::frame_src(a, ta + 1) * plane + yo;
     const Tin* __restrict__ r0 = img0 + yo;
     auto scalar_rows = [&]() {
 #pragma unroll 4
       for (int x0 = lane; x0 < wl; x0 += 64) {
         const T w = win ? win[yo + x0] : T(1);
         const Tin p0 = sub ? r0[x0] : Tin(0);
-        const T fa = has_a ? sp::pixel_value<Tin, T>(ra[x0], p0, sub, w) : T(0);
-        const T fb = has_b ? sp::pixel_value<Tin, T>(ra[plane + x0], p0, sub, w) : T(0);
+        const T fa = has_a ? sp::pixel_value<Tin, T>(ra[x0], p0, sub_a, w) : T(0);
+        const T fb = has_b ? sp::pixel_value<Tin, T>(rb[x0], p0, sub_b, w) : T(0);
         row[mr_pad<T>(x0)] = C{fa, fb};
       }
     };
@@ -196,7 +199,7 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
             for (int h = 0; h < 2; ++h) {
               const int x0 = min((lane + 64 * (k0 + h)) * VX, wl - VX);
               va[h] = has_a ? *reinterpret_cast<const Vec*>(ra + x0) : Vec{};
-              vb[h] = has_b ? *reinterpret_cast<const Vec*>(ra + plane + x0) : Vec{};
+              vb[h] = has_b ? *reinterpret_cast<const Vec*>(rb + x0) : Vec{};
               v0[h] = sub ? *reinterpret_cast<const Vec*>(r0 + x0) : Vec{};
               if (win) wv[h] = *reinterpret_cast<const WVec*>(win + yo + x0);
             }
@@ -207,8 +210,8 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
 #pragma unroll
                 for (int v = 0; v < VX; ++v) {
                   const T w = win ? wv[h].v[v] : T(1);
-                  const T fa = has_a ? sp::pixel_value<Tin, T>(va[h].v[v], v0[h].v[v], sub, w) : T(0);
-                  const T fb = has_b ? sp::pixel_value<Tin, T>(vb[h].v[v], v0[h].v[v], sub, w) : T(0);
+                  const T fa = has_a ? sp::pixel_value<Tin, T>(va[h].v[v], v0[h].v[v], sub_a, w) : T(0);
+                  const T fb = has_b ? sp::pixel_value<Tin, T>(vb[h].v[v], v0[h].v[v], sub_b, w) : T(0);
                   row[mr_pad<T>(x0 + v)] = C{fa, fb};
                 }
               }

@@ -65,7 +65,6 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
   const Tin* __restrict__ img = static_cast<const Tin*>(a.img);
   const T* __restrict__ win = static_cast<const T*>(a.window);
   const size_t plane = static_cast<size_t>(H) * W;
-  const bool sub = a.subtract0 != 0;
   const C* __restrict__ tw = static_cast<const C*>(a.twx);
   const Tin* __restrict__ row0 = img + static_cast<size_t>(y) * W;  // first frame of the launch, row y
   const Tin* __restrict__ ref0 = static_cast<const Tin*>(a.img0) + static_cast<size_t>(y) * W;  // subtracted frame
@@ -83,11 +82,13 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
     for (int e = tid; e < NP * G; e += kThreads) {
       const int p = e / G, g = e - p * G, x0 = g * VX;
       const uint64_t ta = t0 + 2 * p;
+      const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
+      const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
       Vec va{}, vb{}, v0{};
       WVec wv;
-      if (ta < a.frames) va = *reinterpret_cast<const Vec*>(row0 + ta * plane + x0);
-      if (ta + 1 < a.frames) vb = *reinterpret_cast<const Vec*>(row0 + (ta + 1) * plane + x0);
-      if (sub) v0 = *reinterpret_cast<const Vec*>(ref0 + x0);
+      if (has_a) va = *reinterpret_cast<const Vec*>(row0 + sp::frame_src(a, ta) * plane + x0);
+      if (has_b) vb = *reinterpret_cast<const Vec*>(row0 + sp::frame_src(a, ta + 1) * plane + x0);
+      if (sub_a || sub_b) v0 = *reinterpret_cast<const Vec*>(ref0 + x0);
       // the VX window values in one or two vector loads issued with the
       // pixels (one load per value: row pass 9.3 ms at 1024^2 x 4000, this
       // way 7.9 ms)
@@ -96,8 +97,8 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
 #pragma unroll
       for (int v = 0; v < VX; ++v) {
         const T w = win ? wv.v[v] : T(1);
-        const T fa = ta < a.frames ? pixel_value<Tin, T>(va.v[v], v0.v[v], sub, w) : T(0);
-        const T fb = ta + 1 < a.frames ? pixel_value<Tin, T>(vb.v[v], v0.v[v], sub, w) : T(0);
+        const T fa = has_a ? pixel_value<Tin, T>(va.v[v], v0.v[v], sub_a, w) : T(0);
+        const T fb = has_b ? pixel_value<Tin, T>(vb.v[v], v0.v[v], sub_b, w) : T(0);
         d[v] = C{fa, fb};
       }
     }
@@ -108,9 +109,11 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
       T fa = 0, fb = 0;
       if (x < W) {
         const T w = win ? win[static_cast<size_t>(y) * W + x] : T(1);
-        const Tin x0v = sub ? ref0[x] : Tin(0);
-        if (ta < a.frames) fa = pixel_value<Tin, T>(row0[ta * plane + x], x0v, sub, w);
-        if (ta + 1 < a.frames) fb = pixel_value<Tin, T>(row0[(ta + 1) * plane + x], x0v, sub, w);
+        const Tin x0v = a.subtract0 ? ref0[x] : Tin(0);
+        if (sp::frame_here(a, ta))
+          fa = pixel_value<Tin, T>(row0[sp::frame_src(a, ta) * plane + x], x0v, sp::frame_sub(a, ta), w);
+        if (sp::frame_here(a, ta + 1))
+          fb = pixel_value<Tin, T>(row0[sp::frame_src(a, ta + 1) * plane + x], x0v, sp::frame_sub(a, ta + 1), w);
       }
       buf[padi(e)] = C{fa, fb};
     }
@@ -169,7 +172,6 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
   const Tin* __restrict__ img = static_cast<const Tin*>(a.img);
   const T* __restrict__ win = static_cast<const T*>(a.window);
   const size_t plane = static_cast<size_t>(H) * NX;
-  const bool sub = a.subtract0 != 0;
   const T half_norm = static_cast<T>(0.5 * a.norm);
   const uint32_t kstride = static_cast<uint32_t>(H) * TB;
   {
@@ -184,12 +186,15 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
     const uint64_t ta = static_cast<uint64_t>(item / H) * TB + 2 * p;
     const Tin* __restrict__ row0 = img + static_cast<size_t>(y) * NX;
     const Tin* __restrict__ ref0 = static_cast<const Tin*>(a.img0) + static_cast<size_t>(y) * NX;
+    const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
+    const Tin* __restrict__ rowa = row0 + sp::frame_src(a, ta) * plane;
+    const Tin* __restrict__ rowb = row0 + sp::frame_src(a, ta + 1) * plane;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int x0 = (lane + 64 * k) * VX;
-      va[k] = ta < a.frames ? *reinterpret_cast<const Vec*>(row0 + ta * plane + x0) : Vec{};
-      vb[k] = ta + 1 < a.frames ? *reinterpret_cast<const Vec*>(row0 + (ta + 1) * plane + x0) : Vec{};
-      v0[k] = sub ? *reinterpret_cast<const Vec*>(ref0 + x0) : Vec{};
+      va[k] = has_a ? *reinterpret_cast<const Vec*>(rowa + x0) : Vec{};
+      vb[k] = has_b ? *reinterpret_cast<const Vec*>(rowb + x0) : Vec{};
+      v0[k] = a.subtract0 ? *reinterpret_cast<const Vec*>(ref0 + x0) : Vec{};
       if (win) wv[k] = *reinterpret_cast<const WVec*>(win + static_cast<size_t>(y) * NX + x0);
     }
   };
@@ -200,7 +205,9 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
     load(item);
     const int y = static_cast<int>(item % H);
     const uint64_t tb = item / H, ta = tb * TB + 2 * p;
-    const bool has_a = ta < a.frames, has_b = ta + 1 < a.frames;  // uniform over the wave
+    // (uniform over the wave)
+    const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
+    const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
     // registers -> this wave's row: frames (2p, 2p+1) as one complex row
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
@@ -209,8 +216,8 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
 #pragma unroll
       for (int v = 0; v < VX; ++v) {
         const T w = win ? wv[k].v[v] : T(1);
-        const T fa = has_a ? pixel_value<Tin, T>(va[k].v[v], v0[k].v[v], sub, w) : T(0);
-        const T fb = has_b ? pixel_value<Tin, T>(vb[k].v[v], v0[k].v[v], sub, w) : T(0);
+        const T fa = has_a ? pixel_value<Tin, T>(va[k].v[v], v0[k].v[v], sub_a, w) : T(0);
+        const T fb = has_b ? pixel_value<Tin, T>(vb[k].v[v], v0[k].v[v], sub_b, w) : T(0);
         d[v] = C{fa, fb};
       }
     }

@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(kLongThreads) k_time_long(TimeArgs a, int nq, 
         var = ptot_l / L - (mr2 * mr2 + mi2 * mi2);
         Acc fr = static_cast<Acc>(m_r) + mr2, fi = static_cast<Acc>(m_i) + mi2;
         if (a.S0) {
-          const C z = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
+          const C z = frame0_spectrum<C>(a, q);
           fr += static_cast<Acc>(z.x);
           fi += static_cast<Acc>(z.y);
         }

@@ -101,8 +101,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 
   C v[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) v[r] = r < R2 ? entry(src, 64 * r, p) : entry(src, 0, min(p + 64 * r, L - 1));
-  C first{0, 0};  // F(0) of the raw first frame
-  if (a.S0) first = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
+  const C first = frame0_spectrum<C>(a, q);  // F(0) of the raw first frame
   issued();
 #pragma unroll
   for (int r = R2; r < R; ++r) v[r] = p + 64 * r < L ? v[r] : C{0, 0};

@@ -88,8 +88,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(wav
   C v[R], x[R];
   load(v);
   const double rl = inv[0];
-  C first{0, 0};  // F(0) of the raw first frame
-  if (a.S0) first = static_cast<const C*>(a.S0)[static_cast<size_t>(q) * a.s0_stride];
+  const C first = frame0_spectrum<C>(a, q);  // F(0) of the raw first frame
   T m_r = 0, m_i = 0;
   center(v, T(0), T(0));
   double sr = 0, si = 0;
