@@ -577,6 +577,10 @@ void set_frame0(const fddm_plan* p, TimeArgs& ta, const void* S0, const void* ed
   }
 }
 
+hipError_t fix_lags(const fddm_plan* p, const TimeArgs& ta, const void* edge_S64, hipStream_t s) {
+  return launch_fix(ta, edge_S64, p->edge ? p->edge->Lp : 0, kEdgeFrames, p->edge_i0, p->out_dtype, s);
+}
+
 // Spatial stage of the whole stack into the workspace (R, S); the timing
 // events around the passes.
 int run_spatial(fddm_plan* p, const void* d_img, void* ws, hipStream_t s, char* err, size_t errlen) {
@@ -648,11 +652,9 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }
   if ((rc = record(p, 4, s, err, errlen))) return rc;
-  // compensated FP32 corrections: flagged Wiener-Khinchin lags, then the lags
+  // compensated FP32 corrections: marked Wiener-Khinchin lags, and the lags
   // with at most kEdgeFrames pairs from FP64 spectra
-  if (ta.flags) FDDM_HIP(launch_wk_fix(ta, p->out_dtype, s));
-  if (p->edge)
-    FDDM_HIP(launch_edge_fix(ta, ews + p->edge->bytes_R, p->edge->Lp, kEdgeFrames, p->edge_i0, p->out_dtype, s));
+  FDDM_HIP(fix_lags(p, ta, p->edge ? ews + p->edge->bytes_R : nullptr, s));
   if ((rc = record(p, 5, s, err, errlen))) return rc;
   if (p->timing_cap > 0 && p->timing_steps < p->timing_cap) ++p->timing_steps;
   return FDDM_OK;
@@ -834,8 +836,7 @@ int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* e
   } else {
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }
-  if (ta.flags) FDDM_HIP(launch_wk_fix(ta, p->out_dtype, s));
-  if (p->edge) FDDM_HIP(launch_edge_fix(ta, edge_S64, p->edge->Lp, kEdgeFrames, p->edge_i0, p->out_dtype, s));
+  FDDM_HIP(fix_lags(p, ta, edge_S64, s));
   return FDDM_OK;
 }
 

@@ -16,7 +16,7 @@
 // The time kernel's Wiener-Khinchin values carry an absolute error of a few
 // 1e-7 of sum_t |G|^2 in (L - dt) D.  Where (L - dt) D is small against that
 // sum -- slow low-q modes and chance near-recurrences -- the kernel marks the
-// q, and k_wk_fix recomputes the affected lags of the marked q by direct
+// q, and k_fix recomputes the affected lags of the marked q by direct
 // differences of the stored float series in double: each workgroup lists its
 // marked columns (flags read in parallel), each marked one's lags are shared
 // by the workgroup's waves, lanes run over t and a wave sum closes each lag.
@@ -40,10 +40,8 @@ constexpr int kThreads = 256;
 // and are then stored to the lag rows they belong to (same order of
 // additions as the general loop, so the same values).
 template <typename OutT>
-__global__ void __launch_bounds__(kThreads)
-    k_edge_fix(TimeArgs a, const double2* __restrict__ S64, uint64_t lp, int E, int i0) {
-  const int c = blockIdx.x * kThreads + threadIdx.x;  // column of the launch
-  if (c >= a.cols) return;
+__device__ __forceinline__ void edge_fix(const TimeArgs& a, const double2* __restrict__ S64, uint64_t lp, int E, int i0,
+                                         int c) {
   const int q = col_q(a, c), L = a.L, nl = a.nl;
   const uint32_t* __restrict__ lags = a.lags;
   OutT* __restrict__ out = static_cast<OutT*>(a.out);
@@ -91,8 +89,15 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// Both corrections in one launch: they write different lags (at most E pairs;
+// more than 32).  S64 null: no edge lags; a.flags null: no marked columns.
 template <typename OutT>
-__global__ void __launch_bounds__(kThreads) k_wk_fix(TimeArgs a) {
+__global__ void __launch_bounds__(kThreads)
+    k_fix(TimeArgs a, const double2* __restrict__ S64, uint64_t lp, int E, int i0) {
+  if (S64)
+    for (int c = blockIdx.x * kThreads + threadIdx.x; c < a.cols; c += gridDim.x * kThreads)
+      edge_fix<OutT>(a, S64, lp, E, i0, c);
+  if (!a.flags) return;
   // workgroup g owns the columns g + m G (G workgroups); their flags are read
   // at once, one per thread, the marked columns listed in LDS, and the
   // waves of the workgroup share the lags of each listed column
@@ -151,25 +156,16 @@ __global__ void __launch_bounds__(kThreads) k_wk_fix(TimeArgs a) {
 
 }  // namespace
 
-hipError_t launch_wk_fix(const TimeArgs& a, int out_dtype, hipStream_t s) {
-  if (a.nl <= 0 || a.cols <= 0 || !a.flags) return hipSuccess;
-  const dim3 grid(static_cast<unsigned>(std::min(a.cols, 2048)));
+hipError_t launch_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype, hipStream_t s) {
+  if (i0 >= a.nl) S64 = nullptr;
+  if (a.nl <= 0 || a.cols <= 0 || (!S64 && !a.flags)) return hipSuccess;
+  // a column per thread for the edge lags; up to 2048 workgroups share the marked columns
+  const unsigned edge = (a.cols + kThreads - 1) / kThreads;
+  const dim3 grid(a.flags ? std::max(edge, static_cast<unsigned>(std::min(a.cols, 2048))) : edge);
   if (out_dtype == OUT_F32) {
-    hipLaunchKernelGGL(k_wk_fix<float>, grid, dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL(k_fix<float>, grid, dim3(kThreads), 0, s, a, static_cast<const double2*>(S64), lp, E, i0);
   } else {
-    hipLaunchKernelGGL(k_wk_fix<double>, grid, dim3(kThreads), 0, s, a);
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_edge_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype,
-                           hipStream_t s) {
-  if (i0 >= a.nl || a.cols <= 0) return hipSuccess;
-  const dim3 grid((a.cols + kThreads - 1) / kThreads);
-  if (out_dtype == OUT_F32) {
-    hipLaunchKernelGGL(k_edge_fix<float>, grid, dim3(kThreads), 0, s, a, static_cast<const double2*>(S64), lp, E, i0);
-  } else {
-    hipLaunchKernelGGL(k_edge_fix<double>, grid, dim3(kThreads), 0, s, a, static_cast<const double2*>(S64), lp, E, i0);
+    hipLaunchKernelGGL(k_fix<double>, grid, dim3(kThreads), 0, s, a, static_cast<const double2*>(S64), lp, E, i0);
   }
   return hipGetLastError();
 }

@@ -62,7 +62,7 @@ struct TimeArgs {
   FftDesc dt;
   const void* twt;
   void* out;
-  unsigned char* flags;  // fft mode, compensated FP32: per q, 1 = some lag needs launch_wk_fix
+  unsigned char* flags;  // fft mode, compensated FP32: per q, 1 = some lag needs launch_fix
   // Columns of this launch, c in [0, cols).  local = 0: column c is output
   // column c0 + c of the y-shifted plane (row pitch ldo) and reads the q at
   // that position; local = 1: column c reads q = c0 + c and is stored
@@ -139,18 +139,15 @@ hipError_t launch_fft_test(void* data, int n, int batch, const FftDesc& d, const
 // (hipHostGetDevicePointer), by a kernel; n and both addresses multiples of 16.
 hipError_t launch_copy_out(void* dst, const void* src, uint64_t n, hipStream_t s);
 
-// FP64 edge correction of the compensated path (fddm_edge.hip): the lags
-// lags[i0 .. nl) (n = L - dt <= E pairs) recomputed by direct sums from the
-// FP64 spectra S64[q][c] (pitch lp) of the first and last E frames into the
-// y-shifted output.
-hipError_t launch_edge_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype,
-                           hipStream_t s);
+// Corrections of the compensated path (fddm_edge.hip), in the y-shifted
+// output: the lags lags[i0 .. nl) (n = L - dt <= E pairs) by direct sums from
+// the FP64 spectra S64[q][c] (pitch lp; null: none) of the first and last E
+// frames; of the q marked in a.flags (null: none) the lags with (L - dt) D <
+// kWkFlag L VAR and L - dt > 32 by direct differences of the float series
+// S[q][t] (pitch Lp) in double.
 constexpr int kEdgeFrames = 8;
-// Lags of the q marked in flags whose (L - dt) D < kWkFlag L VAR and
-// L - dt > 32 recomputed by direct differences of the float series S[q][t]
-// (pitch Lp) in double, written to the y-shifted output.
 constexpr double kWkFlag = 2e-3;
-hipError_t launch_wk_fix(const TimeArgs& a, int out_dtype, hipStream_t s);
+hipError_t launch_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype, hipStream_t s);
 
 // Time stage for series longer than the LDS-resident plans allow
 // (fddm_time_long.hip): N = 2^logn in (2^12, 2^long_max_log] as a four-step

@@ -51,7 +51,7 @@ constexpr int kEdge = 32;
 // cells at N = 8192).  A q with a lag whose (L - dt) D falls below
 // kWkFlag x sum |G|^2 (2e-3: a relative error bound above ~1.5e-4) -- slow
 // low-q modes at short lags, chance near-recurrences at large lags -- is
-// marked in a.flags; launch_wk_fix then recomputes those lags by direct
+// marked in a.flags; launch_fix then recomputes those lags by direct
 // differences.
 
 // 1 / n for a positive integer n: hardware reciprocal refined by Newton's

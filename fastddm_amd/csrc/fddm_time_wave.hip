@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(wav
   // 5. D(d) = (psum(L - d) + psum(L) - psum(d) - 2 C(d)) / (L - d); lags at
   // or beyond L give values that nothing reads.  Compensated FP32: a lag
   // whose (L - d) D is small against sum |x|^2 marks the column for the
-  // direct recomputation (launch_wk_fix).
+  // direct recomputation (launch_fix).
   bool flag = false;
   {
     const double thr = ptot * kWkFlag;
