@@ -109,7 +109,10 @@ size_t in_bytes(int dtype) {
   }
 }
 
-// Radix plan: 2^a as 8s (two 4s or one 4 for the remainder), then 3s, 5s, 7s.
+// Radix plan: the 5s and 3s that take a factor 2 with them (5s first) as 10s
+// and 6s, the other odd factors, then the remaining power of two as 8s (two
+// 4s or one 4 for the remainder).  Every pass is a trip through LDS: the
+// fewest factors are paired that give the fewest passes.
 bool factorize(uint64_t n, FftDesc& d) {
   std::memset(&d, 0, sizeof(d));
   if (n == 0 || n > (1u << 20)) return false;
@@ -119,16 +122,6 @@ bool factorize(uint64_t n, FftDesc& d) {
   while (r % 2 == 0) {
     r /= 2;
     ++a;
-  }
-  d.c8 = a / 3;
-  const int rem = a % 3;
-  if (rem == 1 && d.c8 > 0) {
-    --d.c8;
-    d.c4 = 2;
-  } else if (rem == 1) {
-    d.c2 = 1;
-  } else if (rem == 2) {
-    d.c4 = 1;
   }
   while (r % 3 == 0) {
     r /= 3;
@@ -142,10 +135,28 @@ bool factorize(uint64_t n, FftDesc& d) {
     r /= 7;
     ++d.c7;
   }
+  int pairs = 0;
+  for (int m = 1; m <= std::min(a, d.c3 + d.c5); ++m)
+    if ((a - m + 2) / 3 < (a - pairs + 2) / 3) pairs = m;
+  a -= pairs;
+  d.c10 = std::min(pairs, d.c5);
+  d.c6 = pairs - d.c10;
+  d.c5 -= d.c10;
+  d.c3 -= d.c6;
+  d.c8 = a / 3;
+  const int rem = a % 3;
+  if (rem == 1 && d.c8 > 0) {
+    --d.c8;
+    d.c4 = 2;
+  } else if (rem == 1) {
+    d.c2 = 1;
+  } else if (rem == 2) {
+    d.c4 = 1;
+  }
   return r == 1;
 }
 
-// Per-pass twiddle tables in execution order (radix 8s, 4s, 2s, 3s, 5s, 7s):
+// Per-pass twiddle tables in the order of FftDesc:
 // pass with radix R after Ns points stores exp(-2 pi i r k / (Ns R)) at
 // k (R-1) + r - 1 for k < Ns, r = 1 .. R-1; n - 1 entries in all.  Evaluated
 // in long double and rounded once.
@@ -154,10 +165,10 @@ std::vector<T> twiddles(const FftDesc& d) {
   std::vector<T> w;
   w.reserve(2 * static_cast<size_t>(d.n));
   const long double two_pi = 6.283185307179586476925286766559005768L;
-  const int counts[6] = {d.c8, d.c4, d.c2, d.c3, d.c5, d.c7};
-  const int radix[6] = {8, 4, 2, 3, 5, 7};
+  const int counts[8] = {d.c7, d.c5, d.c3, d.c10, d.c6, d.c8, d.c4, d.c2};
+  const int radix[8] = {7, 5, 3, 10, 6, 8, 4, 2};
   long long ns = 1;
-  for (int g = 0; g < 6; ++g)
+  for (int g = 0; g < 8; ++g)
     for (int i = 0; i < counts[g]; ++i) {
       const int R = radix[g];
       for (long long k = 0; k < ns; ++k)

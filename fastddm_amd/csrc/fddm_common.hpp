@@ -33,10 +33,13 @@ enum OutDtype : int { OUT_F64 = 0, OUT_F32 = 1 };
 enum Mode : int { MODE_DIFF = 0, MODE_FFT = 1 };
 
 // Mixed-radix factorisation of one FFT length, passed to kernels by value:
-// n = 8^c8 4^c4 2^c2 3^c3 5^c5 7^c7, passes applied in that order.
+// n = 7^c7 5^c5 3^c3 10^c10 6^c6 8^c8 4^c4 2^c2, passes applied in that order.
+// A pass of radix R writes at a stride of its radix times the points so far:
+// an odd radix first keeps those strides off the LDS banks' powers of two
+// (radix 8 first, as a power of two: 8 lanes on a bank).
 struct FftDesc {
   int n;
-  int c8, c4, c2, c3, c5, c7;
+  int c7, c5, c3, c10, c6, c8, c4, c2;
 };
 
 // Elements of an LDS buffer holding n logical elements with one pad slot

@@ -12,7 +12,8 @@
 //
 // Butterflies: radix 2, 4, 8 in closed form; radix 3, 5, 7 from the
 // symmetric-pair form of the DFT,
-//   X_s = v_0 + sum_r (v_r + v_{R-r}) cos(2 pi r s / R) - i (v_r - v_{R-r}) sin(2 pi r s / R).
+//   X_s = v_0 + sum_r (v_r + v_{R-r}) cos(2 pi r s / R) - i (v_r - v_{R-r}) sin(2 pi r s / R);
+// radix 6 and 10 as 2 x 3 and 2 x 5 (Good-Thomas, no twiddles between).
 // Twiddles come from per-pass tables exp(-2 pi i r k / (Ns R)) built on the
 // host in extended precision and stored contiguously per butterfly.
 #pragma once
@@ -138,6 +139,23 @@ __device__ __forceinline__ void butterfly(cplx_t<T> (&v)[R]) {
     v[6] = csub(e2, w2);
     v[3] = cadd(e3, w3);
     v[7] = csub(e3, w3);
+  } else if constexpr (R == 6 || R == 10) {
+    // n = P n1 + 2 n2, k = P k1 + (P + 1) k2 (mod 2 P): w^(n k) splits into
+    // (-1)^(n1 k1) and the length-P DFT over n2
+    constexpr int P = R / 2;
+    C s[P], d[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      s[i] = cadd(v[2 * i], v[(P + 2 * i) % R]);
+      d[i] = csub(v[2 * i], v[(P + 2 * i) % R]);
+    }
+    butterfly_odd<T, P>(s);
+    butterfly_odd<T, P>(d);
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      v[(P + 1) * i % R] = s[i];
+      v[(P + (P + 1) * i) % R] = d[i];
+    }
   } else {
     butterfly_odd<T, R>(v);
   }
@@ -223,10 +241,10 @@ __device__ __forceinline__ void stockham_pass(cplx_t<T>* buf, int off, int n, in
 
 // Forward FFT (unnormalised) of nb transforms in LDS.  E bounds the elements
 // per thread: E * nthr >= n * nb.  `tw` is the plan's concatenated per-pass
-// twiddle table (pass order: 8s, 4s, 2s, 3s, 5s, 7s).  The caller
+// twiddle table (in the order of FftDesc).  The caller
 // synchronises before the call; the data are synchronised on return.  One
 // loop per radix (rather than a switch over a pass list) keeps the register
-// allocation of the six pass variants disjoint.
+// allocation of the eight pass variants disjoint.
 template <typename T, int E, bool TIF>
 __device__ void fft_lds(cplx_t<T>* buf, int off, const FftDesc& d, int nb, int lognb, int bstride,
                         int estride, const cplx_t<T>* __restrict__ tw, int tid, int nthr) {
@@ -239,12 +257,14 @@ __device__ void fft_lds(cplx_t<T>* buf, int off, const FftDesc& d, int nb, int l
     tw += ns * (RAD - 1);                                                                    \
     ns *= RAD;                                                                               \
   }
+  FDDM_PASSES(7, c7)
+  FDDM_PASSES(5, c5)
+  FDDM_PASSES(3, c3)
+  FDDM_PASSES(10, c10)
+  FDDM_PASSES(6, c6)
   FDDM_PASSES(8, c8)
   FDDM_PASSES(4, c4)
   FDDM_PASSES(2, c2)
-  FDDM_PASSES(3, c3)
-  FDDM_PASSES(5, c5)
-  FDDM_PASSES(7, c7)
 #undef FDDM_PASSES
 }
 

@@ -4,11 +4,12 @@
 // power-of-two persistent row kernel is:
 //
 //   * one wave per transform (rows: frames 2p and 2p+1 of one image row as
-//     one complex row; columns: one frame of the block), held in the wave's
+//     one complex row, short rows two or four to a wave; columns: one frame
+//     of the block), held in the wave's
 //     own LDS row and transformed with no workgroup barrier (runtime radix
-//     sequence 8s, 4s, 2s, 3s, 5s, 7s; each pass reads all of a lane's
-//     butterflies into registers before it writes, and the wave's LDS
-//     operations complete in order, so passes run in place);
+//     sequence, see FftDesc; each pass reads all of a lane's butterflies
+//     into registers before it writes, and the wave's LDS operations
+//     complete in order, so passes run in place);
 //   * the pass twiddles are copied into LDS once per workgroup, which then
 //     loops over items ((frame block, image row) or (kx, frame block));
 //   * pixels and window values come in 8-byte / 16-byte vector loads, all of
@@ -38,6 +39,14 @@ template <int KMAX, typename T>
 constexpr int mr_min_waves() {
   return KMAX <= kMrShort ? (sizeof(T) == 4 ? 8 : 4) : (sizeof(T) == 4 ? 3 : 2);
 }
+// (FP32 rows spill at 64 VGPRs: 6 waves; 480 x 640 x 997 0.75 -> 0.61 ms)
+template <int KMAX, typename T>
+constexpr int rows_min_waves() {
+  return KMAX <= kMrShort && sizeof(T) == 4 ? 6 : mr_min_waves<KMAX, T>();
+}
+// Rows of at most kMrHalf (kMrQuarter) points run two (four) to a wave, on
+// 32 (16) lanes each: a pass of radix R has n / R butterflies.
+constexpr int kMrHalf = 320, kMrQuarter = 160;
 
 // LDS slot of element e of a transform row.  FP32 rows are not padded:
 // those kernels spend most of their time issuing VALU instructions, and the
@@ -53,30 +62,31 @@ __device__ __forceinline__ int mr_pad(int e) {
 }
 
 // One radix-R Stockham pass (formulation of fddm_fft.hpp) of a length-n
-// transform held by one wave: element e at row[mr_pad<T>(e)], lane handles
-// butterflies j = lane + 64 b.  ns: product of the radices already applied;
+// transform held by P lanes of a wave: element e at row[mr_pad<T>(e)], lane
+// (0 .. P - 1) handles butterflies j = lane + P b.  ns: product of the radices already applied;
 // tw: this pass's table, tw[k (R-1) + r - 1] = exp(-2 pi i r k / (ns R)).
-template <typename T, int R, int KMAX>
+template <typename T, int R, int KMAX, int P>
 __device__ __forceinline__ void wave_pass(cplx_t<T>* row, int n, int ns, const cplx_t<T>* tw, int lane) {
   using C = cplx_t<T>;
-  constexpr int MB = (KMAX / R + 63) / 64;
+  constexpr int MB = (KMAX / R + P - 1) / P;
   // opaque lane index: the lane-derived address arithmetic stays in this
   // pass instead of being hoisted to the kernel entry and kept live
   asm volatile("" : "+v"(lane));
   const int m = n / R;
-  // k = j mod ns, advanced by 64 mod ns per item; ns is uniform, and a power
-  // of two for every pass before the first odd radix (a mask, not a division)
-  const bool p2ns = (ns & (ns - 1)) == 0;
-  int k = p2ns ? (lane & (ns - 1)) : lane % ns;
-  const int dk = p2ns ? (64 & (ns - 1)) : 64 % ns;
+  // k = j mod ns, advanced by P mod ns per item; ns is uniform.  The
+  // quotient by a 16-bit reciprocal: exact for lane <= 64, ns <= kMrLong.
+  const int rec = __builtin_amdgcn_readfirstlane(
+      static_cast<int>(65536.0f * __builtin_amdgcn_rcpf(static_cast<float>(ns))) + 1);
+  int k = lane - ns * ((lane * rec) >> 16);
+  const int dk = P - ns * ((P * rec) >> 16);
   C v[MB][R];
   int ob[MB];
 #pragma unroll
   for (int b = 0; b < MB; ++b) ob[b] = -1;
 #pragma unroll
   for (int b = 0; b < MB; ++b) {
-    const int j = lane + 64 * b;
-    if (64 * b < m && j < m) {  // (the first test is uniform)
+    const int j = lane + P * b;
+    if (P * b < m && j < m) {  // (the first test is uniform)
 #pragma unroll
       for (int r = 0; r < R; ++r) v[b][r] = row[mr_pad<T>(j + r * m)];
       if (ns > 1) {
@@ -100,37 +110,40 @@ __device__ __forceinline__ void wave_pass(cplx_t<T>* row, int n, int ns, const c
   p2::wave_lds_sync();
 }
 
-// Forward FFT (unnormalised) of one length-d.n row by one wave; passes in
-// the order of the twiddle table (8s, 4s, 2s, 3s, 5s, 7s).
-template <typename T, int KMAX>
+// Forward FFT (unnormalised) of one length-d.n row by P lanes; passes in the
+// order of FftDesc.
+template <typename T, int KMAX, int P>
 __device__ __forceinline__ void fft_wave_mr(cplx_t<T>* row, const FftDesc& d, const cplx_t<T>* tw, int lane) {
   const int n = d.n;
   int ns = 1;
 #define FDDM_WAVE_PASSES(RAD, COUNT)                  \
   for (int i = 0; i < d.COUNT; ++i) {                 \
-    wave_pass<T, RAD, KMAX>(row, n, ns, tw, lane);    \
+    wave_pass<T, RAD, KMAX, P>(row, n, ns, tw, lane); \
     tw += ns * (RAD - 1);                             \
     ns *= RAD;                                        \
   }
+  FDDM_WAVE_PASSES(7, c7)
+  FDDM_WAVE_PASSES(5, c5)
+  FDDM_WAVE_PASSES(3, c3)
+  FDDM_WAVE_PASSES(10, c10)
+  FDDM_WAVE_PASSES(6, c6)
   FDDM_WAVE_PASSES(8, c8)
   FDDM_WAVE_PASSES(4, c4)
   FDDM_WAVE_PASSES(2, c2)
-  FDDM_WAVE_PASSES(3, c3)
-  FDDM_WAVE_PASSES(5, c5)
-  FDDM_WAVE_PASSES(7, c7)
 #undef FDDM_WAVE_PASSES
 }
 
-// Row pass, Tb = 2 NP frames per block, NP waves.  rs: LDS slots per pair
-// row (lds_padded_size(nx)); vec: pixel rows start 8-byte aligned and the
-// loaded width is a multiple of the vector (host-checked).
-template <typename Tin, typename T, int NP, int KMAX>
-__global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(RowArgs a, uint32_t nitems, int rs, int vec) {
+// Row pass, Tb = 2 NP frames per block, NP waves; an item is the rows
+// y .. y + G - 1 of a frame block, G = 64 / P, wave p transforms the pair p of
+// each on P lanes.  rs: LDS slots per pair row; vec: pixel rows start 8-byte
+// aligned and the loaded width is a multiple of the vector (host-checked).
+template <typename Tin, typename T, int NP, int KMAX, int P>
+__global__ void __launch_bounds__(64 * NP, (rows_min_waves<KMAX, T>())) k_rows_mr(RowArgs a, uint32_t nitems, int rs, int vec) {
   using C = cplx_t<T>;
-  constexpr int NT = 64 * NP, TB = 2 * NP;
+  constexpr int NT = 64 * NP, TB = 2 * NP, G = 64 / P;
   constexpr int VX = sizeof(Tin) <= 4 ? 8 / static_cast<int>(sizeof(Tin)) : 1;
   // vectors per lane and frame row, at most (even: taken two at a time)
-  constexpr int KV = ((KMAX / VX + 63) / 64 + 1) & ~1;
+  constexpr int KV = ((KMAX / VX + P - 1) / P + 1) & ~1;
   struct alignas(8) Vec {
     Tin v[VX];
   };
@@ -139,10 +152,9 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
   };
   extern __shared__ __align__(16) unsigned char smem[];
   C* const buf = reinterpret_cast<C*>(smem);
-  C* const twl = buf + NP * rs;
+  C* const twl = buf + G * NP * rs;
   const int tid = threadIdx.x;
-  const int p = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's pair row (uniform)
-  C* const row = buf + p * rs;
+  const int p = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's pair (uniform)
   const int H = a.H, W = a.W, nx = a.nx, nxh = nx / 2 + 1;
   const int wl = W < nx ? W : nx;  // pixels loaded per row; x in [wl, nx) is zero padding
   const Tin* __restrict__ img = static_cast<const Tin*>(a.img);
@@ -151,7 +163,7 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
   const size_t plane = static_cast<size_t>(H) * W;
   const bool sub = a.subtract0 != 0;
   const T half_norm = static_cast<T>(0.5 * a.norm);
-  const uint32_t kstride = static_cast<uint32_t>(H) * TB;
+  const uint32_t kstride = static_cast<uint32_t>(H) * TB, hg = (static_cast<uint32_t>(H) + G - 1) / G;
   {
     const C* __restrict__ tw = static_cast<const C*>(a.twx);
     const int twn = nx > 1 ? nx - 1 : 1;
@@ -165,10 +177,18 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
   for (uint64_t item = x * per + (blockIdx.x >> 3); item < end; item += gridDim.x >> 3) {
     // thread-derived addresses are rebuilt per item rather than hoisted out
     // of the loop and kept live through the transform
-    int lane = tid & 63, tidi = tid;
+    int lane = tid & (P - 1), tidi = tid;
     asm volatile("" : "+v"(lane), "+v"(tidi));
-    const int y = static_cast<int>(static_cast<uint32_t>(item) % static_cast<uint32_t>(H));
-    const uint64_t tb = static_cast<uint32_t>(item) / static_cast<uint32_t>(H), ta = tb * TB + 2 * p;
+    const int y0 = static_cast<int>(static_cast<uint32_t>(item) % hg) * G;
+    const uint64_t tb = static_cast<uint32_t>(item) / hg, ta = tb * TB + 2 * p;
+    // this lane's image row (rows past the last repeat it and are not stored)
+    int y = y0;
+    C* row = buf + p * rs;
+    if constexpr (G > 1) {
+      const int g = (tidi & 63) / P;
+      y = min(y0 + g, H - 1);
+      row += g * NP * rs;
+    }
     // (uniform over the wave)
     const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
     const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
@@ -178,7 +198,7 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
     const Tin* __restrict__ r0 = img0 + yo;
     auto scalar_rows = [&]() {
 #pragma unroll 4
-      for (int x0 = lane; x0 < wl; x0 += 64) {
+      for (int x0 = lane; x0 < wl; x0 += P) {
         const T w = win ? win[yo + x0] : T(1);
         const Tin p0 = sub ? r0[x0] : Tin(0);
         const T fa = has_a ? sp::pixel_value<Tin, T>(ra[x0], p0, sub_a, w) : T(0);
@@ -192,12 +212,12 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
         // all issued before the first conversion
 #pragma unroll
         for (int k0 = 0; k0 < KV; k0 += 2) {
-          if (64 * k0 * VX < wl) {  // uniform
+          if (P * k0 * VX < wl) {  // uniform
             Vec va[2], vb[2], v0[2];
             WVec wv[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              const int x0 = min((lane + 64 * (k0 + h)) * VX, wl - VX);
+              const int x0 = min((lane + P * (k0 + h)) * VX, wl - VX);
               va[h] = has_a ? *reinterpret_cast<const Vec*>(ra + x0) : Vec{};
               vb[h] = has_b ? *reinterpret_cast<const Vec*>(rb + x0) : Vec{};
               v0[h] = sub ? *reinterpret_cast<const Vec*>(r0 + x0) : Vec{};
@@ -205,7 +225,7 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
             }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              const int x0 = (lane + 64 * (k0 + h)) * VX;
+              const int x0 = (lane + P * (k0 + h)) * VX;
               if (x0 < wl) {
 #pragma unroll
                 for (int v = 0; v < VX; ++v) {
@@ -224,21 +244,23 @@ __global__ void __launch_bounds__(64 * NP, (mr_min_waves<KMAX, T>())) k_rows_mr(
     } else {
       scalar_rows();
     }
-    for (int xp = wl + lane; xp < nx; xp += 64) row[mr_pad<T>(xp)] = C{0, 0};
+    for (int xp = wl + lane; xp < nx; xp += P) row[mr_pad<T>(xp)] = C{0, 0};
     p2::wave_lds_sync();
-    fft_wave_mr<T, KMAX>(row, a.dx, twl, lane);
+    fft_wave_mr<T, KMAX, P>(row, a.dx, twl, lane);
     __syncthreads();  // every pair row transformed
 
     // split into the two half spectra, store R[tb][k][y][ti] (ti fastest)
-    C* __restrict__ R = static_cast<C*>(a.R) + (tb * nxh * static_cast<size_t>(H) + y) * TB;
-    // thread tidi takes pair row pp = tidi mod NP and k = tidi / NP + 64 i
-    // (NT = 64 NP threads): the row is fixed and the address advances
+    // thread tidi takes pair pp = tidi mod NP of row y0 + g and k = kt + (64 / G) i
+    // (NT = 64 NP threads): the LDS row is fixed and the address advances
     {
-      const int pp = tidi & (NP - 1);
-      const C* const rp = buf + pp * rs;
-      C* dst = R + static_cast<uint32_t>(tidi / NP) * kstride + 2 * pp;
-      for (int k = tidi / NP; k < nxh; k += 64, dst += 64 * kstride)
-        sp::split_store<T>(dst, rp[mr_pad<T>(k)], rp[mr_pad<T>(k == 0 ? 0 : nx - k)], half_norm);
+      const int rr = tidi & (G * NP - 1), pp = rr & (NP - 1), g = rr / NP, kt = tidi / (G * NP);
+      if (G == 1 || y0 + g < H) {
+        const C* const rp = buf + rr * rs;
+        C* dst = static_cast<C*>(a.R) + (tb * nxh * static_cast<size_t>(H) + y0 + g) * TB +
+                 static_cast<uint32_t>(kt) * kstride + 2 * pp;
+        for (int k = kt; k < nxh; k += P, dst += P * kstride)
+          sp::split_store<T>(dst, rp[mr_pad<T>(k)], rp[mr_pad<T>(k == 0 ? 0 : nx - k)], half_norm);
+      }
     }
     __syncthreads();  // the LDS rows are rewritten by the next item
   }
@@ -301,7 +323,7 @@ __global__ void __launch_bounds__(64 * TB, (mr_min_waves<KMAX, T>())) k_cols_mr(
     }
     for (int y = hl + lane; y < ny; y += 64) col[mr_pad<T>(y)] = C{0, 0};
     __syncthreads();
-    fft_wave_mr<T, KMAX>(col, a.dy, twl, lane);
+    fft_wave_mr<T, KMAX, 64>(col, a.dy, twl, lane);
     __syncthreads();  // every transform done
     C* __restrict__ S = static_cast<C*>(a.S) + static_cast<size_t>(kx) * a.Lp + static_cast<size_t>(tb) * TB;
     // thread tidi stores frames 2 tp, 2 tp + 1 (tp = tidi mod TB/2) of the q
@@ -326,15 +348,49 @@ __global__ void __launch_bounds__(64 * TB, (mr_min_waves<KMAX, T>())) k_cols_mr(
   }
 }
 
+// LDS slots per transform row: the 256 bytes of banks split evenly over the
+// `rows` rows that neighbouring lanes step through in the slab writes of the
+// column pass and the split of the row pass, so that a row's run of
+// neighbouring elements starts where the previous row's ends.  With the odd
+// radices first and the pass pairs of factorize() (fddm_capi.hip): FP32
+// columns of 480 x 640 x 997 0.90 -> 0.62 ms (57 % of their cycles had been
+// bank conflicts), rows and columns of 1000^2 x 300 0.81 -> 0.65 and
+// 0.82 -> 0.72 ms.
+int mr_row_slots(int n, int rows, int precision) {
+  const int banks = precision == PREC_FP64 ? 16 : 32;  // slots in all banks
+  const int padded = precision == PREC_FP64 ? lds_padded_size(n) : n, step = banks / rows;
+  return padded + ((step - padded) & (banks - 1));
+}
+
+// Image rows per item of the row kernel.  Two or four short rows to a wave
+// where one to a wave needs several rounds of the chip (four workgroups to a
+// CU): 600 frames of 96^2 35.3 -> 18.3 us, of 150 x 200 60.7 -> 44.3 us, 271
+// of 147 x 201 in FP64 62.7 -> 37.2 us; a launch of one round only gets
+// longer (41 frames of 96^2 in FP64, 576 rows: 8.0 one to a wave, 9.8 us).
+int rows_mr_group(const RowArgs& a, int precision) {
+  if (a.Tb != (precision == PREC_FP64 ? 8 : 16)) return 1;  // (a smaller block: long columns)
+  if ((a.frames + a.Tb - 1) / a.Tb * static_cast<uint64_t>(a.H) <= 1024) return 1;
+  return a.nx <= kMrQuarter ? 4 : a.nx <= kMrHalf ? 2 : 1;
+}
+
 size_t rows_mr_lds(const RowArgs& a, int precision, int* rs) {
-  *rs = lds_padded_size(a.nx);
+  const int rows = a.Tb / 2 * rows_mr_group(a, precision);
+  *rs = mr_row_slots(a.nx, rows, precision);
   const size_t csz = precision == PREC_FP64 ? 16 : 8;
-  return csz * (static_cast<size_t>(a.Tb / 2) * *rs + std::max(a.nx - 1, 1));
+  return csz * (static_cast<size_t>(rows) * *rs + std::max(a.nx - 1, 1));
 }
 
 template <typename Tin, typename T, int NP>
-hipError_t rows_mr_np(const RowArgs& a, uint32_t items, size_t lds, int rs, int vec, hipStream_t s) {
-  auto kernel = a.nx <= kMrShort ? k_rows_mr<Tin, T, NP, kMrShort> : k_rows_mr<Tin, T, NP, kMrLong>;
+hipError_t rows_mr_np(const RowArgs& a, size_t lds, int rs, int vec, hipStream_t s) {
+  auto kernel = a.nx <= kMrShort ? k_rows_mr<Tin, T, NP, kMrShort, 64> : k_rows_mr<Tin, T, NP, kMrLong, 64>;
+  int group = 1;
+  if constexpr (NP == (sizeof(T) == 4 ? 8 : 4)) {
+    group = rows_mr_group(a, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32);
+    if (group == 2) kernel = k_rows_mr<Tin, T, NP, kMrHalf, 32>;
+    if (group == 4) kernel = k_rows_mr<Tin, T, NP, kMrQuarter, 16>;
+  }
+  const uint64_t nblocks = (a.frames + a.Tb - 1) / a.Tb;
+  const uint32_t items = static_cast<uint32_t>(nblocks * ((static_cast<uint64_t>(a.H) + group - 1) / group));
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
@@ -355,7 +411,7 @@ hipError_t rows_mr_np(const RowArgs& a, uint32_t items, size_t lds, int rs, int 
 }
 
 template <typename Tin, typename T>
-hipError_t rows_mr_in(const RowArgs& a, uint32_t items, size_t lds, int rs, hipStream_t s) {
+hipError_t rows_mr_in(const RowArgs& a, size_t lds, int rs, hipStream_t s) {
   int vec = 0;
   if constexpr (sizeof(Tin) <= 4) {
     constexpr int VX = 8 / sizeof(Tin);
@@ -365,31 +421,31 @@ hipError_t rows_mr_in(const RowArgs& a, uint32_t items, size_t lds, int rs, hipS
           reinterpret_cast<uintptr_t>(a.window) % 16 == 0;
   }
   switch (a.Tb) {
-    case 4: return rows_mr_np<Tin, T, 2>(a, items, lds, rs, vec, s);
-    case 8: return rows_mr_np<Tin, T, 4>(a, items, lds, rs, vec, s);
-    case 16: return rows_mr_np<Tin, T, 8>(a, items, lds, rs, vec, s);
+    case 4: return rows_mr_np<Tin, T, 2>(a, lds, rs, vec, s);
+    case 8: return rows_mr_np<Tin, T, 4>(a, lds, rs, vec, s);
+    case 16: return rows_mr_np<Tin, T, 8>(a, lds, rs, vec, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 template <typename T>
-hipError_t rows_mr_t(const RowArgs& a, uint32_t items, size_t lds, int rs, hipStream_t s) {
+hipError_t rows_mr_t(const RowArgs& a, size_t lds, int rs, hipStream_t s) {
   switch (a.in_dtype) {
-    case IN_U8: return rows_mr_in<uint8_t, T>(a, items, lds, rs, s);
-    case IN_I16: return rows_mr_in<int16_t, T>(a, items, lds, rs, s);
-    case IN_U16: return rows_mr_in<uint16_t, T>(a, items, lds, rs, s);
-    case IN_I32: return rows_mr_in<int32_t, T>(a, items, lds, rs, s);
-    case IN_U32: return rows_mr_in<uint32_t, T>(a, items, lds, rs, s);
-    case IN_I64: return rows_mr_in<int64_t, T>(a, items, lds, rs, s);
-    case IN_U64: return rows_mr_in<uint64_t, T>(a, items, lds, rs, s);
-    case IN_F32: return rows_mr_in<float, T>(a, items, lds, rs, s);
-    case IN_F64: return rows_mr_in<double, T>(a, items, lds, rs, s);
+    case IN_U8: return rows_mr_in<uint8_t, T>(a, lds, rs, s);
+    case IN_I16: return rows_mr_in<int16_t, T>(a, lds, rs, s);
+    case IN_U16: return rows_mr_in<uint16_t, T>(a, lds, rs, s);
+    case IN_I32: return rows_mr_in<int32_t, T>(a, lds, rs, s);
+    case IN_U32: return rows_mr_in<uint32_t, T>(a, lds, rs, s);
+    case IN_I64: return rows_mr_in<int64_t, T>(a, lds, rs, s);
+    case IN_U64: return rows_mr_in<uint64_t, T>(a, lds, rs, s);
+    case IN_F32: return rows_mr_in<float, T>(a, lds, rs, s);
+    case IN_F64: return rows_mr_in<double, T>(a, lds, rs, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 size_t cols_mr_lds(const ColArgs& a, int precision, int* rs) {
-  *rs = lds_padded_size(a.ny);
+  *rs = mr_row_slots(a.ny, a.Tb, precision);
   const size_t csz = precision == PREC_FP64 ? 16 : 8;
   return csz * (static_cast<size_t>(a.Tb) * *rs + std::max(a.ny - 1, 1));
 }
@@ -446,8 +502,7 @@ hipError_t launch_rows_mr(const RowArgs& a, int precision, hipStream_t s) {
   if (items > 0xfffffff0ull) return hipErrorInvalidValue;
   int rs = 0;
   const size_t lds = rows_mr_lds(a, precision, &rs);
-  return precision == PREC_FP64 ? rows_mr_t<double>(a, static_cast<uint32_t>(items), lds, rs, s)
-                                : rows_mr_t<float>(a, static_cast<uint32_t>(items), lds, rs, s);
+  return precision == PREC_FP64 ? rows_mr_t<double>(a, lds, rs, s) : rows_mr_t<float>(a, lds, rs, s);
 }
 
 bool cols_mr_ok(const ColArgs& a, int precision) {
