@@ -11,16 +11,21 @@
 // deviations are taken from the finished average, as the reference does).
 //
 // Work split (deterministic, no atomics).  Pixels are taken in flat q order
-// in tiles of 64 (one per wave instruction); a workgroup owns T consecutive
-// rows t and a contiguous range of tiles.  Each lane loads its pixel's bin
-// and weight once and the T values x_q(t0 .. t0+T-1) together, so T loads per
+// in tiles of 128 (two neighbours per lane); a workgroup owns T consecutive
+// rows t and a contiguous range of tiles.  Each lane loads its pixels' bins
+// and weights once and the T pairs x_q(t0 .. t0+T-1) together, so T loads per
 // lane are in flight.  Along one ky row the modulus |k| grows with kx, so the
-// key (row within the tile, bin) never decreases across a tile's lanes: runs
+// key (row within the tile, bin) never decreases across a tile's pixels: runs
 // of equal key are reduced with a segmented wave scan built from DPP row
-// shifts and row broadcasts, and the last lane of each run adds the run's sum
-// to the wave's own LDS accumulator.  Runs of one row have distinct bins, and
-// runs of different rows are added in separate steps, so no two lanes of one
-// LDS write share an address.  Waves' accumulators are summed in fixed order
+// shifts and row broadcasts over the lanes' second pixels (with the first
+// added where both share the key).  The lane where a run ends adds the run's
+// sum to the wave's own LDS accumulator: with its second pixel from the scan,
+// with its first from the scan of the lane before.  Runs of one row have
+// distinct bins, and runs of different rows, or ending at different pixels of
+// a lane, are added in separate steps, so no two lanes of one LDS write share
+// an address.  With one pixel per lane the scan's instructions held the pass
+// at 3.5 TB/s (502 rows of 512 x 257: 150 us, vector units 62 % busy; with two
+// 134 us, 3.9 TB/s, what reading alone reaches).  Waves' accumulators are summed in fixed order
 // into partial[t][chunk][bin]; a second kernel sums the chunks in order.
 #include <algorithm>
 #include <cmath>
@@ -39,6 +44,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
+constexpr int kTile = 128;  // pixels of a wave step
 constexpr int kMaxBins = 1024;
 constexpr int kTargetBlocks = 4096;  // workgroups aimed for per pass (256 CUs x 16)
 constexpr size_t kLdsBudget = 64 * 1024;
@@ -93,6 +99,23 @@ __device__ __forceinline__ double seg_scan(double v, unsigned f) {
   return v;
 }
 
+// Whether the lane before (its second pixel's key: kb) ends in the run of ka.
+__device__ __forceinline__ bool same_key_before(int kb, int ka) {
+  return __builtin_amdgcn_update_dpp(-1, kb, 0x138, 0xf, 0xf, false) == ka;
+}
+
+// A pixel's term; masked pixels add nothing, not even a NaN.
+template <bool SQ>
+__device__ __forceinline__ double weighted(double x, double w, double mean) {
+  if (w == 0.0) return 0.0;
+  if constexpr (SQ) {
+    const double d = x - mean;
+    return w * d * d;
+  } else {
+    return w * x;
+  }
+}
+
 // Pass 1 (SQ = false): sum w x.  Pass 2 (SQ = true): sum w (x - avg[b, t])^2.
 // LDS: acc[kWaves][T][nbins], then (SQ) mean[T][nbins].
 template <typename In, bool SQ, int T>
@@ -118,38 +141,51 @@ __global__ void __launch_bounds__(kThreads)
   const In* __restrict__ rowt[T];
 #pragma unroll
   for (int tt = 0; tt < T; ++tt) rowt[tt] = data + static_cast<size_t>(min(t0 + tt, rows - 1)) * nq;
-  const uint32_t tile_end = min(static_cast<uint32_t>(chunk + 1) * chunk_tiles * 64u, nq);
-  for (uint32_t q0 = (static_cast<uint32_t>(chunk) * chunk_tiles + wave) * 64u; q0 < tile_end; q0 += kWaves * 64u) {
-    const uint32_t qlast = min(q0 + 63u, tile_end - 1u);
-    const bool in = q0 + lane <= qlast;
-    const uint32_t q = in ? q0 + lane : qlast;  // lanes past the end repeat the last pixel with weight 0
-    In x[T];
+  const uint32_t tile0 = static_cast<uint32_t>(chunk) * chunk_tiles;
+  const uint32_t tile_end = min(tile0 + chunk_tiles, (nq - 1u) / kTile + 1u);
+  for (uint32_t tile = tile0 + wave; tile < tile_end; tile += kWaves) {
+    const uint32_t q0 = tile * kTile;
+    // lanes past the end repeat the last pixel with weight 0
+    const uint32_t qlast = min(q0 + (kTile - 1u), nq - 1u);
+    const uint32_t qa = min(q0 + 2u * lane, qlast), qb = min(q0 + 2u * lane + 1u, qlast);
+    In xa[T], xb[T];
+    if (qlast == q0 + (kTile - 1u)) {  // uniform: whole pairs, in one load of the element's alignment
 #pragma unroll
-    for (int tt = 0; tt < T; ++tt) x[tt] = rowt[tt][q];
-    const int b = bin[q];
-    const double wq = in ? w[q] : 0.0;
-    const int y0 = static_cast<int>(q0 / nxh), yrow = static_cast<int>(q / nxh) - y0;
+      for (int tt = 0; tt < T; ++tt) {
+        In v[2];
+        __builtin_memcpy(v, rowt[tt] + qa, sizeof(v));
+        xa[tt] = v[0];
+        xb[tt] = v[1];
+      }
+    } else {
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt) {
+        xa[tt] = rowt[tt][qa];
+        xb[tt] = rowt[tt][qb];
+      }
+    }
+    const int ba = bin[qa], bb = bin[qb];
+    const double wa = q0 + 2u * lane <= qlast ? w[qa] : 0.0, wb = q0 + 2u * lane + 1u <= qlast ? w[qb] : 0.0;
+    const int y0 = static_cast<int>(q0 / nxh), ya = static_cast<int>(qa / nxh) - y0, yb = static_cast<int>(qb / nxh) - y0;
     const int nrows = static_cast<int>(qlast / nxh) - y0 + 1;
-    const int key = yrow * kMaxBins + b;
-    const unsigned f = run_flags(key);
-    const int key_next = __shfl_down(key, 1, 64);  // every lane takes part
-    const bool run_end = (lane == 63) | (key_next != key);
+    const int ka = ya * kMaxBins + ba, kb = yb * kMaxBins + bb;
+    const unsigned f = run_flags(kb);
+    const bool one = ka == kb;  // both pixels in one run
+    const int ka_next = __shfl_down(ka, 1, 64);  // every lane takes part
+    const bool end_b = (lane == 63) | (ka_next != kb);
+    const bool join_a = same_key_before(kb, ka);
 #pragma unroll
     for (int tt = 0; tt < T; ++tt) {
-      double v = 0.0;
-      if (wq != 0.0) {  // masked pixels add nothing, not even a NaN
-        const double xv = static_cast<double>(x[tt]);
-        if constexpr (SQ) {
-          const double d = xv - mean[tt * nbins + b];
-          v = wq * d * d;
-        } else {
-          v = wq * xv;
-        }
-      }
-      v = seg_scan(v, f);
+      const double va = weighted<SQ>(static_cast<double>(xa[tt]), wa, SQ ? mean[tt * nbins + ba] : 0.0);
+      const double vb = weighted<SQ>(static_cast<double>(xb[tt]), wb, SQ ? mean[tt * nbins + bb] : 0.0);
+      const double sb = seg_scan(one ? va + vb : vb, f);
+      const double before = dpp_zero<0x138, 0xf>(sb);  // the lane before
+      const double sa = join_a ? before + va : va;
       if (tt < nt) {
-        for (int r = 0; r < nrows; ++r)
-          if (run_end && yrow == r) my[tt * nbins + b] += v;
+        for (int r = 0; r < nrows; ++r) {
+          if (!one && ya == r) my[tt * nbins + ba] += sa;
+          if (end_b && yb == r) my[tt * nbins + bb] += sb;
+        }
       }
     }
   }
@@ -275,9 +311,9 @@ extern "C" int fddm_azimuthal_average(const void* d_data, int data_f32, uint64_t
   std::vector<double> bias(nbins);
   for (int b = 0; b < nbins; ++b) bias[b] = sw[b] > 0 ? sw[b] - sw2[b] / sw[b] : 0.0;
 
-  // grid: T rows per workgroup, chunks of chunk_tiles tiles of 64 pixels
+  // grid: T rows per workgroup, chunks of chunk_tiles tiles of kTile pixels
   const int T = rows_per_block(nbins);
-  const uint64_t ntiles = (nq + 63) / 64, ttiles = (rows + T - 1) / T;
+  const uint64_t ntiles = (nq + kTile - 1) / kTile, ttiles = (rows + T - 1) / T;
   const uint64_t want = (ntiles * ttiles + kTargetBlocks - 1) / kTargetBlocks;
   const int chunk_tiles = static_cast<int>(std::min<uint64_t>(std::max<uint64_t>(want, kWaves), 1024));
   const int nchunks = static_cast<int>((ntiles + chunk_tiles - 1) / chunk_tiles);
