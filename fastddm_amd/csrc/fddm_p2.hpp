@@ -139,8 +139,19 @@ __device__ __forceinline__ void dft(cplx_t<T> (&v)[R]) {
   }
 }
 
-__device__ __forceinline__ int padi(int e) { return e + (e >> 5); }
-constexpr int cpad(int e) { return e + (e >> 5); }
+template <int SH = 5>
+__device__ __forceinline__ int padi(int e) {
+  return e + (e >> SH);
+}
+template <int SH = 5>
+constexpr int cpad(int e) {
+  return e + (e >> SH);
+}
+// Pad shift of rows transformed by one wave: a slot after each round of the
+// 64 banks (16 FP64, 32 FP32 elements), which spreads writes at a stride of 8
+// over all of them.
+template <typename T>
+constexpr int kWavePad = sizeof(T) == 8 ? 4 : 5;
 
 // One Stockham pass with compile-time parameters: nb transforms of N points,
 // radix R after NS points, worked on by NT threads (thread index `tid` in
@@ -150,7 +161,9 @@ constexpr int cpad(int e) { return e + (e >> 5); }
 // the butterfly index first (BS a multiple of 32).  Butterfly j reads
 // x[j + r M] and writes y[(j - k) R + k + r NS], k = j mod NS; with all sizes
 // powers of two both are one padded base per butterfly plus constant offsets.
-template <typename T, int N, int R, int NS, int NT, int NB = 1, bool TIF = false, int E = 1, int BS = 0>
+// TS: entries per k of the twiddle table, R or (without r = 0) R - 1; SH: pad
+// shift.
+template <typename T, int N, int R, int NS, int NT, int NB = 1, bool TIF = false, int E = 1, int BS = 0, int TS = R, int SH = 5>
 struct Pass {
   using C = cplx_t<T>;
   static constexpr int M = N / R;
@@ -179,12 +192,12 @@ struct Pass {
       if (ITEMS % NT != 0 && w >= ITEMS) break;
       int j, ti;
       item(w, j, ti);
-      const C* p = buf + padi(ti * BS + j * E);
+      const C* p = buf + padi<SH>(ti * BS + j * E);
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[b][r] = p[cpad(r * M * E)];
+      for (int r = 0; r < R; ++r) v[b][r] = p[cpad<SH>(r * M * E)];
       if constexpr (NS > 1) {
         const int k = j & (NS - 1);
-        const C* t = tw + k * R;
+        const C* t = tw + k * TS - (R - TS);
 #pragma unroll
         for (int r = 1; r < R; ++r) v[b][r] = cmul(v[b][r], t[r]);
       }
@@ -204,9 +217,9 @@ struct Pass {
       int j, ti;
       item(w, j, ti);
       const int k = j & (NS - 1);
-      C* p = buf + padi(ti * BS + ((j - k) * R + k) * E);
+      C* p = buf + padi<SH>(ti * BS + ((j - k) * R + k) * E);
 #pragma unroll
-      for (int r = 0; r < R; ++r) p[cpad(r * NS * E)] = v[b][r];
+      for (int r = 0; r < R; ++r) p[cpad<SH>(r * NS * E)] = v[b][r];
     }
   }
 };
@@ -268,13 +281,15 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // Whole forward transform of one length-N row in LDS by one wave (lane in
 // [0, 64)), three passes, no workgroup barriers: the row's LDS region is
-// this wave's own.
+// this wave's own.  tw: the two tables without their r = 0 column, so that
+// their rows (of 7, 3 entries) start on different LDS banks: neighbouring
+// lanes take neighbouring rows, and rows of 8 entries lay 8 lanes to a bank.
 template <typename T, int N, int R0, int R1, int R2>
 __device__ __forceinline__ void fft3_wave(cplx_t<T>* row, const cplx_t<T>* __restrict__ tw, int lane) {
   using C = cplx_t<T>;
-  using A0 = Pass<T, N, R0, 1, 64>;
-  using A1 = Pass<T, N, R1, R0, 64>;
-  using A2 = Pass<T, N, R2, R0 * R1, 64>;
+  using A0 = Pass<T, N, R0, 1, 64, 1, false, 1, 0, R0, kWavePad<T>>;
+  using A1 = Pass<T, N, R1, R0, 64, 1, false, 1, 0, R1 - 1, kWavePad<T>>;
+  using A2 = Pass<T, N, R2, R0 * R1, 64, 1, false, 1, 0, R2 - 1, kWavePad<T>>;
   {
     C v[A0::MB][R0];
     A0::compute(row, v, tw, lane);
@@ -289,7 +304,7 @@ __device__ __forceinline__ void fft3_wave(cplx_t<T>* row, const cplx_t<T>* __res
   }
   {
     C v[A2::MB][R2];
-    A2::compute(row, v, tw + R0 * R1, lane);
+    A2::compute(row, v, tw + R0 * (R1 - 1), lane);
     A2::store(row, v, lane);
   }
 }

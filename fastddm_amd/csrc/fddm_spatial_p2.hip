@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
   }
 }
 
-// Full-width rows (W == NX <= 512) of pixels of up to 4 bytes, FP32 and FP64
+// Full-width rows (W == NX <= 1024) of pixels of up to 4 bytes, FP32 and FP64
 // (held to 64 and 128 VGPRs): a persistent form of k_rows_p2 with one wave
 // per pair row.  Workgroup b takes items b,
 // b + grid, ... (item = tb * H + y); wave p loads, converts and transforms
@@ -146,13 +146,30 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
 // transform needed more than the 64 VGPRs of 8 waves per SIMD, and the
 // spill reloads waited (vmcnt) for every load and store in flight
 // (0.73 ms at 512^2 x 2000 with that prefetch, 0.68-0.69 ms without).
+//
+// LDS: pair row p starts at slot p rowslots, the banks' 256 bytes divided by
+// NP past the row before, so that the split's neighbouring lanes (the pairs)
+// read from different banks; twiddles as fft3_wave takes them.  With rows at
+// multiples of all banks and twiddle rows of 8 entries, conflicts took 46 %
+// (FP64) and 28 % (FP32) of the kernel's cycles: 512^2 x 1000 in FP64 0.86 ->
+// 0.74 ms.
+template <typename T, int LOGX, int NP>
+struct PersistLds {
+  static constexpr SpPlan P = sp_plan(LOGX);
+  static constexpr int banks = 256 / sizeof(cplx_t<T>), padded = cpad<kWavePad<T>>(1 << LOGX);
+  static constexpr int rowslots = padded + ((banks / NP - padded) & (banks - 1));
+  static constexpr int tw1 = P.r0 * (P.r1 - 1), tw2 = P.r0 * P.r1 * (P.r2 - 1);
+  static constexpr size_t bytes = sizeof(cplx_t<T>) * (NP * rowslots + tw1 + tw2);
+};
+
 template <typename Tin, typename T, int LOGX, int NP>
-__global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_persist(RowArgs a, uint32_t nitems) {
+__global__ void __launch_bounds__(64 * NP, (LOGX <= 9 ? 2 : 1) * (sizeof(T) == 8 ? 2 : 4)) k_rows_p2_persist(RowArgs a, uint32_t nitems) {
   using C = cplx_t<T>;
   constexpr int NT = 64 * NP;
   constexpr int NX = 1 << LOGX, NXH = NX / 2 + 1, TB = 2 * NP;
   constexpr SpPlan P = sp_plan(LOGX);
-  constexpr int TWN = P.r0 * P.r1 * (1 + P.r2);  // [k][r] tables of passes 1 and 2
+  using Lds = PersistLds<T, LOGX, NP>;
+  constexpr int SH = kWavePad<T>;
   constexpr int VX = 8 / sizeof(Tin), GV = NX / VX;
   constexpr int PER = GV / 64;  // 8-byte vectors per lane and frame row
   static_assert(GV % 64 == 0, "whole vectors per lane");
@@ -164,10 +181,10 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
   };
   extern __shared__ __align__(16) unsigned char smem[];
   C* const buf = reinterpret_cast<C*>(smem);
-  C* const twl = buf + lds_padded_size(NP * NX);
+  C* const twl = buf + NP * Lds::rowslots;
   const int tid = threadIdx.x, lane = tid & 63;
   const int p = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's pair row (uniform)
-  C* const row = buf + padi(p * NX);  // p NX is a multiple of 32: padded offsets add
+  C* const row = buf + p * Lds::rowslots;
   const int H = a.H;
   const Tin* __restrict__ img = static_cast<const Tin*>(a.img);
   const T* __restrict__ win = static_cast<const T*>(a.window);
@@ -176,7 +193,10 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
   const uint32_t kstride = static_cast<uint32_t>(H) * TB;
   {
     const C* __restrict__ tw = static_cast<const C*>(a.twx);
-    for (int i = tid; i < TWN; i += NT) twl[i] = tw[i];
+    // [k][r] tables of passes 1 and 2, r from 1
+    for (int i = tid; i < Lds::tw1; i += NT) twl[i] = tw[i / (P.r1 - 1) * P.r1 + i % (P.r1 - 1) + 1];
+    for (int i = tid; i < Lds::tw2; i += NT)
+      twl[Lds::tw1 + i] = tw[P.r0 * P.r1 + i / (P.r2 - 1) * P.r2 + i % (P.r2 - 1) + 1];
   }
 
   Vec va[PER], vb[PER], v0[PER];
@@ -199,6 +219,8 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
     }
   };
 
+  // (partial lines in launch order too: a contiguous share of the items per
+  // XCD was 3 % slower at 1024^2 x 1000)
   uint32_t item = blockIdx.x;
   __syncthreads();  // twiddles in LDS
   for (; item < nitems; item += gridDim.x) {
@@ -212,7 +234,7 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int x0 = (lane + 64 * k) * VX;
-      C* d = row + padi(x0);  // VX divides 32: the VX slots are contiguous
+      C* d = row + padi<SH>(x0);  // VX divides 16: the VX slots are contiguous
 #pragma unroll
       for (int v = 0; v < VX; ++v) {
         const T w = win ? wv[k].v[v] : T(1);
@@ -229,8 +251,9 @@ __global__ void __launch_bounds__(64 * NP, (sizeof(T) == 8 ? 4 : 8)) k_rows_p2_p
     C* __restrict__ R = static_cast<C*>(a.R) + (tb * NXH * static_cast<size_t>(H) + y) * TB;
     for (int w = tid; w < NXH * NP; w += NT) {
       const int pp = w & (NP - 1), k = w / NP;
-      split_store<T>(R + static_cast<uint32_t>(k) * kstride + 2 * pp, buf[padi(pp * NX + k)],
-                     buf[padi(pp * NX + ((NX - k) & (NX - 1)))], half_norm);
+      const C* const rp = buf + pp * Lds::rowslots;
+      split_store<T>(R + static_cast<uint32_t>(k) * kstride + 2 * pp, rp[padi<SH>(k)],
+                     rp[padi<SH>((NX - k) & (NX - 1))], half_norm);
     }
     __syncthreads();  // the LDS rows are rewritten by the next item
   }
@@ -321,13 +344,14 @@ hipError_t rows_np(const RowArgs& a, unsigned grid, hipStream_t s) {
   const size_t lds_rows = sizeof(cplx_t<T>) * lds_padded_size(NP * (1 << LOGX));
   const size_t lds = lds_rows;
   // persistent form (pixels of up to 4 bytes in whole 8-byte vectors per
-  // lane, full rows up to 512 wide, FP32 and FP64: 512^2 x 2000 fp64 rows
+  // lane, full rows up to 1024 wide, FP32 and FP64: 512^2 x 2000 fp64 rows
   // 1.75 -> 1.49 ms, uint8 fp32c 0.78 -> 0.61 ms, float32 fp64 1.07 -> 0.77
-  // ms at 1000 frames); as many workgroups as stay resident
-  if constexpr (sizeof(Tin) <= 4 && LOGX <= 9 && ((1 << LOGX) * sizeof(Tin) / 8) % 64 == 0) {
+  // ms at 1000 frames); as many workgroups as stay resident.  Rows of 1024
+  // need three (of 2 or 4 waves) to a CU and many rounds of the chip:
+  // 1024^2 x 1000 fp32c 2.06 -> 1.94 ms, FP64 x 300 1.42 -> 1.30 ms, but 8 frames (1.3 rounds) 14 -> 18 us.
+  if constexpr (sizeof(Tin) <= 4 && LOGX <= 10 && ((1 << LOGX) * sizeof(Tin) / 8) % 64 == 0) {
     if (a.W == (1 << LOGX)) {
-      constexpr SpPlan P = sp_plan(LOGX);
-      const size_t lds = lds_rows + sizeof(cplx_t<T>) * P.r0 * P.r1 * (1 + P.r2);  // + the LDS twiddles
+      constexpr size_t lds = PersistLds<T, LOGX, NP>::bytes;
       auto kernel = k_rows_p2_persist<Tin, T, LOGX, NP>;
       if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -341,8 +365,11 @@ hipError_t rows_np(const RowArgs& a, unsigned grid, hipStream_t s) {
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), 64 * NP, lds);
       if (e != hipSuccess) return e;
       const unsigned resident = static_cast<unsigned>(std::max(1, cus) * std::max(1, per_cu));
-      hipLaunchKernelGGL(kernel, dim3(std::min(grid, resident)), dim3(64 * NP), lds, s, a, static_cast<uint32_t>(grid));
-      return hipGetLastError();
+      if (LOGX <= 9 || (per_cu >= 3 && grid / 8 > resident)) {
+        hipLaunchKernelGGL(kernel, dim3(std::min(grid, resident)), dim3(64 * NP), lds, s, a,
+                           static_cast<uint32_t>(grid));
+        return hipGetLastError();
+      }
     }
   }
   auto kernel = k_rows_p2<Tin, T, LOGX, NP>;
