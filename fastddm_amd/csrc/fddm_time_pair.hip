@@ -351,7 +351,8 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 
     }
   }
   if constexpr (!F64) {
-    if (p == 0) total[1] = __ballot(flag) != 0 ? 1.0 : 0.0;
+    const bool any = __ballot(flag) != 0;  // (by every lane: outside the branch)
+    if (p == 0) total[1] = any ? 1.0 : 0.0;
   }
   OutT* __restrict__ out = static_cast<OutT*>(a.out);
   const size_t ldo = a.ldo;

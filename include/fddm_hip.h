@@ -191,9 +191,9 @@ int fddm_plan_execute_static(fddm_plan *plan, const void *d_img, void *d_out, vo
                              size_t errlen);
 /* Per-stage timing with HIP events on the execute stream: begin reserves
  * events for up to max_steps executes; end waits for them and writes the
- * summed milliseconds of the stages {frame-0 spectra, row pass, column pass,
- * time/diff kernel, FP64 edge correction (FP32C only)} to stage_ms[5] and the
- * number of timed executes. */
+ * summed milliseconds of the stages {frame-0 spectra (FP32C: with the FP64 edge
+ * spectra), row pass, column pass, time/diff kernel, FP64 edge correction (FP32C
+ * only)} to stage_ms[5] and the number of timed executes. */
 int fddm_plan_timing_begin(fddm_plan *plan, int max_steps, char *err, size_t errlen);
 int fddm_plan_timing_end(fddm_plan *plan, double *stage_ms, int *steps, char *err, size_t errlen);
 /* Test entry: spatial stages only; copies the q-major spectra (ny*(nx/2+1),

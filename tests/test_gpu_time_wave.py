@@ -31,3 +31,23 @@ def test_lengths_match_oracle(hip, L, precision):
         else:
             assert np.allclose(out, ref, rtol=1e-3, atol=0)
             assert np.median(onp.relative_error(out, ref)) <= 1e-5
+
+
+# series whose frames recur once, at a lag that any lane of either wave can hold
+RECURRENCES = [(100, 61), (250, 131), (600, 333), (1000, 701), (2000, 1101), (2200, 1101), (4000, 2005), (4000, 2500), (4000, 3901)]
+
+
+@pytest.mark.parametrize("L,lag", RECURRENCES)
+def test_one_small_lag_marks_the_column(hip, L, lag):
+    """D at the one lag of a recurrence is 1e-5 of the variance: far below
+    what the float transforms resolve, right only if the column is marked."""
+    rng = np.random.default_rng(lag)
+    base = rng.normal(10000.0, 1000.0, (lag, 8, 8))
+    img = np.concatenate([base, base[: L - lag]]) + rng.normal(0.0, 3.0, (L, 8, 8))
+    img = np.rint(img).astype(np.uint16)
+    ref = onp.ddm_diff(img, np.array([lag]), 8, 8, None)
+    assert np.median(ref[0] / ref[-1]) < 1e-4
+    for lags in (np.arange(1, L), np.array([lag])):
+        out = hip.ddm_fft(img, lags, 8, 8, next_fast_len(2 * L, "hip"), None, precision="fp32c")
+        got = out[lag - 1 if len(lags) > 1 else 0]
+        assert np.allclose(got, ref[0], rtol=1e-3, atol=0)
