@@ -25,8 +25,9 @@
 // a lane, are added in separate steps, so no two lanes of one LDS write share
 // an address.  With one pixel per lane the scan's instructions held the pass
 // at 3.5 TB/s (502 rows of 512 x 257: 150 us, vector units 62 % busy; with two
-// 134 us, 3.9 TB/s, what reading alone reaches).  Waves' accumulators are summed in fixed order
-// into partial[t][chunk][bin]; a second kernel sums the chunks in order.
+// 134 us, 3.9 TB/s, what reading alone reaches).  Waves' accumulators are
+// summed in fixed order into partial[t][chunk][bin]; a second kernel sums the
+// chunks in order.
 #include <algorithm>
 #include <cmath>
 #include <cstdarg>

@@ -5,11 +5,10 @@
 //
 //   * one wave per transform (rows: frames 2p and 2p+1 of one image row as
 //     one complex row, short rows two or four to a wave; columns: one frame
-//     of the block), held in the wave's
-//     own LDS row and transformed with no workgroup barrier (runtime radix
-//     sequence, see FftDesc; each pass reads all of a lane's butterflies
-//     into registers before it writes, and the wave's LDS operations
-//     complete in order, so passes run in place);
+//     of the block), held in the wave's own LDS row and transformed with no
+//     workgroup barrier (runtime radix sequence, see FftDesc; each pass reads
+//     all of a lane's butterflies into registers before it writes, and the
+//     wave's LDS operations complete in order, so passes run in place);
 //   * the pass twiddles are copied into LDS once per workgroup, which then
 //     loops over items ((frame block, image row) or (kx, frame block));
 //   * pixels and window values come in 8-byte / 16-byte vector loads, all of
@@ -30,10 +29,9 @@
 namespace fddm {
 namespace {
 
-// Longest transforms of the two kernel forms: up to kMrShort points the
-// FP32 kernels fit 64 VGPRs (8 waves per SIMD, the occupancy their LDS
-// allows); longer ones, up to kMrLong, hold fewer workgroups per CU anyway
-// (their LDS rows) and get the registers for it.
+// Longest transforms of the two kernel forms: up to kMrShort points the FP32
+// column kernel fits 64 VGPRs (8 waves per SIMD, the occupancy its LDS allows); longer ones, up to kMrLong, hold fewer workgroups per CU anyway (their LDS
+// rows) and get the registers for it.
 constexpr int kMrShort = 768, kMrLong = 2048;
 template <int KMAX, typename T>
 constexpr int mr_min_waves() {
