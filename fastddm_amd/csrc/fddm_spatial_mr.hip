@@ -30,8 +30,9 @@ namespace fddm {
 namespace {
 
 // Longest transforms of the two kernel forms: up to kMrShort points the FP32
-// column kernel fits 64 VGPRs (8 waves per SIMD, the occupancy its LDS allows); longer ones, up to kMrLong, hold fewer workgroups per CU anyway (their LDS
-// rows) and get the registers for it.
+// column kernel fits 64 VGPRs (8 waves per SIMD, the occupancy its LDS
+// allows); longer ones, up to kMrLong, hold fewer workgroups per CU anyway
+// (their LDS rows) and get the registers for it.
 constexpr int kMrShort = 768, kMrLong = 2048;
 template <int KMAX, typename T>
 constexpr int mr_min_waves() {
