@@ -285,14 +285,14 @@ __global__ void __launch_bounds__(kThreads) k_diff_short(TimeArgs a, int wg_per_
       }
     }
     for (int t0 = whole; t0 < L - d[0]; t0 += SEG) {
-      const int t = t0 + sl, tc = min(t, L - 1);
-      const C v = ser[tc];
+      const int t = t0 + sl;
+      const C v = ser[min(t, L - 1)];
       const Acc vx = static_cast<Acc>(v.x), vy = static_cast<Acc>(v.y);
 #pragma unroll
       for (int k = 0; k < K; ++k) {
-        const C u = ser[t + d[k] < L ? t + d[k] : tc];  // (a difference of zero beyond the series)
+        const C u = ser[min(t + d[k], L - 1)];
         const Acc dr = static_cast<Acc>(u.x) - vx, di = static_cast<Acc>(u.y) - vy;
-        acc[k] += dr * dr + di * di;
+        acc[k] += t + d[k] < L ? dr * dr + di * di : Acc(0);  // (not a product: the frames may hold NaN)
       }
     }
     // the four sums of every segment, traded while adding; k: the lag this lane ends with
