@@ -49,7 +49,7 @@ struct PairLay {
   // sample chunks of R2: 16 bytes of padding each; prefix sums: two doubles
   static constexpr int XC = R2 + 16 / sizeof(C), CS = R2 + 2;
   static_assert(128 * XC * sizeof(C) <= 2 * REG * 8 && 128 * CS <= 2 * REG, "REG");
-  static constexpr int EXTRA = kEdge * sizeof(C) / 8 + 2;  // last samples, total, flag
+  static constexpr int EXTRA = kLast * sizeof(C) / 8 + 2;  // last samples, total, flag
   static constexpr size_t bytes = sizeof(double) * W * (REG + EXTRA);
   // tables: W_M^(p k1), W_M^(p (k1 + 1/2)), second stage; the same of FFT_H
   // (even only); (cos, sin)(2 pi d / M), (2 pi d / N), (6 pi d / N) for d < M / 4;
@@ -60,7 +60,7 @@ struct PairLay {
 };
 
 template <int PAD, int R>
-__device__ __forceinline__ int padded(int t) {
+__host__ __device__ __forceinline__ int padded(int t) {
   constexpr int LR = R == 32 ? 5 : 4;
   static_assert(R == 1 << LR, "R");
   return t + (t >> LR) * PAD;
@@ -240,27 +240,15 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 
     __syncthreads();
     {
       C* const last = reinterpret_cast<C*>(extra);
-      if (p < kEdge) last[p] = xs[padded<XP, R2>(L - kEdge + p)];
+      static_assert(kLast == 64, "one per lane");
+      last[p] = p < kEdge ? xs[padded<XP, R2>(L - kEdge + p)] : C{0, 0};
       wave_sync();
-      const int n = ch / 4 + 1, s0 = ch % 4;
-      const C* const u = last + kEdge - n + s0;
-      constexpr int B = 4;  // pairs in flight
-#pragma nounroll
-      for (int i = 0; i < kEdge; i += 4 * B) {
-        C x1[B], x0[B];
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-          x1[b] = u[i + 4 * b];
-          x0[b] = xs[s0 + 4 * b + padded<XP, R2>(i)];
-        }
-        issued();
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-          const double dr = static_cast<double>(x1[b].x) - static_cast<double>(x0[b].x);
-          const double di = static_cast<double>(x1[b].y) - static_cast<double>(x0[b].y);
-          de += i + 4 * b + s0 < n ? dr * dr + di * di : 0.0;
-        }
-      }
+      few_pairs<4, 4>(de, ch / 4 + 1, ch % 4, kEdge, static_cast<const C*>(last), static_cast<const C*>(xs),
+                      [](int t0) { return padded<XP, R2>(t0); }, [](C u, C w) {
+                        const double dr = static_cast<double>(u.x) - static_cast<double>(w.x);
+                        const double di = static_cast<double>(u.y) - static_cast<double>(w.y);
+                        return dr * dr + di * di;
+                      });
       de += __shfl_xor(de, 1, 64);
       de += __shfl_xor(de, 2, 64);
     }

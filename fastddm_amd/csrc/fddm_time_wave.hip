@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(wav
   double* const wlds = reinterpret_cast<double*>(smem) + wave * Lay::WAVE;
   double* const xlds = wlds + g * Lay::GS;  // exchange
   double* const clds = wlds + g * Lay::CG;  // chunks
-  double* const tlds = wlds + Lay::BUF + g * kEdge;  // last samples
+  double* const tlds = wlds + Lay::BUF + g * kLast;  // last samples
 
   // samples t = p + P r, zero from L on.  L > M / 2 except at the smallest M, so the first half needs no check.
   constexpr int FULL = M > 128 ? R / 2 : 0;
@@ -178,9 +178,6 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(wav
   {
     double s[R];
     center(x, m_r, m_i);
-    // adds the squared differences of one component, or of both: sample
-    // L - n + t sits in place kEdge - n + t of the copied last ones, t < n in
-    // the first chunks
     auto reciprocals = [&] {
 #pragma unroll
       for (int r = 0; r < R / 2; ++r) {
@@ -189,27 +186,16 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(wav
       }
       issued();
     };
+    // adds the squared differences of one component, or of both (eight pairs in
+    // flight: a block of t from a multiple of 8 on shares a chunk)
     auto direct = [&](const auto* first, auto* last, auto square) {
-      for (int i = p; i < kEdge; i += P) last[i] = first[chunk_pos<R>(max(L - kEdge + i, 0))];
+      for (int i = p; i < kLast; i += P)
+        last[i] = i < kEdge ? first[chunk_pos<R>(max(L - kEdge + i, 0))] : std::decay_t<decltype(*last)>{};
       wave_sync();
 #pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        const int n = p / SPL + e * P + 1, s0 = p % SPL;
-        const auto* const u = last + kEdge - n + s0;
-        constexpr int B = 8;  // pairs in flight
-#pragma nounroll
-        for (int t0 = 0; t0 < min((e + 1) * P, kEdge); t0 += B * SPL) {
-          std::decay_t<decltype(*first)> x1[B], x0[B];
-#pragma unroll
-          for (int b = 0; b < B; ++b) {  // (t0 a multiple of 8: B pairs share a chunk)
-            x1[b] = u[t0 + b * SPL];
-            x0[b] = first[s0 + b * SPL + chunk_pos<R>(t0)];
-          }
-          issued();
-#pragma unroll
-          for (int b = 0; b < B; ++b) de[e] += t0 + b * SPL + s0 < n ? square(x1[b], x0[b]) : 0.0;
-        }
-      }
+      for (int e = 0; e < NE; ++e)
+        few_pairs<SPL, 8>(de[e], p / SPL + e * P + 1, p % SPL, min((e + 1) * P, kEdge), last, first,
+                          [](int t0) { return chunk_pos<R>(t0); }, square);
     };
 #pragma unroll
     for (int e = 0; e < NE; ++e) de[e] = 0;

@@ -26,6 +26,13 @@ using namespace p2;
 
 constexpr int kEdge = 32;  // lags of at most this many pairs: direct sums
 
+// The last kEdge samples as the direct sums read them: sample L - n + t, the
+// later one of pair t < n of the lag with n pairs, is in place late_place(n, t).
+// The sums run over the same t for every lag and drop t >= n, so they read up
+// to place late_place(1, kEdge - 1); the places from kEdge on hold zeros.
+constexpr int kLast = 2 * kEdge;
+__host__ __device__ constexpr int late_place(int n, int t) { return kEdge - n + t; }
+
 // Shape and LDS layout of M = P R.  Elements are 8 bytes: a float complex
 // value, or one component of a double one (exchanged one after the other).
 template <int R_, int P_, int W_ = 4>
@@ -47,8 +54,8 @@ struct WaveLay {
   static constexpr int CS = R + 2, CG = P * CS;
   static constexpr int NB = P >= R ? 1 : R / P;  // register rows per chunk, where a chunk is longer than a row
   static constexpr int chunk_row(int r) { return P >= R ? r * (P / R) * CS : (r / NB) * CS + (r % NB) * P; }
-  // the exchange buffer or the chunks, then the last kEdge samples of each group
-  static constexpr int BUF = GROUPS * (GS > CG ? GS : CG), WAVE = BUF + GROUPS * kEdge;
+  // the exchange buffer or the chunks, then the last samples of each group
+  static constexpr int BUF = GROUPS * (GS > CG ? GS : CG), WAVE = BUF + GROUPS * kLast;
   static constexpr size_t bytes = sizeof(double) * W * WAVE;
   // tables, complex of the compute type: W_M^(p k1) at [k1][p],
   // W_M^(p (k1 + 1/2)) at [k1][p], then W_P^j (j < R; LANE2) or W_P^(p0 k2) at
@@ -65,7 +72,7 @@ struct WaveLay {
 
 // Position of sample t in the chunk layout.
 template <int R>
-__device__ __forceinline__ int chunk_pos(int t) {
+__host__ __device__ __forceinline__ int chunk_pos(int t) {
   constexpr int LR = R == 32 ? 5 : R == 16 ? 4 : 3;
   static_assert(R == 1 << LR, "R");
   return t + ((t >> LR) << 1);
@@ -128,6 +135,29 @@ __device__ __forceinline__ double group_last(double v) {
 // left alone, the scheduler sinks each load to its use to save registers and
 // waits for them one by one.
 __device__ __forceinline__ void issued() { __builtin_amdgcn_sched_barrier(0); }
+
+// Adds the squared differences of the pairs t = s0, s0 + STEP, ... of the lag
+// with n pairs, t < end and t < n, B pairs in flight: sample t of a block from
+// t0 on is early[t - t0 + pos(t0)].  late and early are arrays, or stand-ins
+// that check their indices (the test of the ranges).
+template <int STEP, int B, typename Late, typename Early, typename Pos, typename F>
+__host__ __device__ __forceinline__ void few_pairs(double& sum, int n, int s0, int end, const Late& late, const Early& early,
+                                                   Pos&& pos, F&& square) {
+#pragma nounroll
+  for (int t0 = 0; t0 < end; t0 += B * STEP) {
+    std::decay_t<decltype(late[0])> x1[B], x0[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      x1[b] = late[late_place(n, s0) + t0 + b * STEP];
+      x0[b] = early[s0 + b * STEP + pos(t0)];
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    issued();
+#endif
+#pragma unroll
+    for (int b = 0; b < B; ++b) sum += t0 + b * STEP + s0 < n ? square(x1[b], x0[b]) : 0.0;
+  }
+}
 
 // Element i + p of a table (i the same for all lanes).
 template <typename E>
