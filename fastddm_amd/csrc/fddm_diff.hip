@@ -373,8 +373,20 @@ hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
   if (csz * pitch * kWaves * 2 <= 40 * 1024) return segments(k_diff_short<T, OutT, PREC, 32>, 2);
   const size_t lds = csz * a.L + 3 * 16 * sizeof(double);
   if (lds <= 159 * 1024) {
-    const int wpx = per_xcd(1);
-    return launch(k_diff<T, OutT, PREC>, 8u * wpx, lds <= 40 * 1024 ? 256 : lds <= 80 * 1024 ? 512 : 1024, lds, s, a, wpx);
+    const unsigned threads = lds <= 40 * 1024 ? 256 : lds <= 80 * 1024 ? 512 : 1024;
+    // a launch holds less than 2^32 threads: larger planes (16.7 M columns of
+    // 256 threads) in several
+    const int64_t most = static_cast<int64_t>((uint64_t(1) << 32) / threads) - 8;
+    for (int64_t c = 0; c < nq; c += most) {
+      TimeArgs part = a;
+      part.c0 += static_cast<int>(c);
+      part.cols = static_cast<int>(std::min<int64_t>(most, nq - c));
+      if (a.local) part.out = static_cast<OutT*>(a.out) + c;  // (stored by column of the launch)
+      const int wpx = (part.cols + 7) / 8;
+      const hipError_t e = launch(k_diff<T, OutT, PREC>, 8u * wpx, threads, lds, s, part, wpx);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
   }
   const int wpx = per_xcd(kWaves);
   return launch(k_diff_long<T, OutT, PREC>, 8u * wpx, kThreads, 0, s, a, wpx);
