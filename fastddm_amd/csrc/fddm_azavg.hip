@@ -205,33 +205,41 @@ __global__ void __launch_bounds__(kThreads)
 // divides by sum_w, pass 2 by the bias factor and takes the square root.
 // Output [b][t].  A chain of loads per output: with one thread for all chunks
 // 98 workgroups waited for 66 loads each (502 rows of 50 bins: 31 us).
+// Workgroups take further outputs in turn beyond kFinishGrid of them: a launch
+// holds less than 2^32 threads.
 constexpr int kFinishLanes = 8, kFinishOut = kThreads / kFinishLanes;
+constexpr uint64_t kFinishGrid = uint64_t(1) << 20;
 template <bool SQ>
 __global__ void __launch_bounds__(kThreads)
     k_azavg_finish(const double* __restrict__ partial, int rows, int nchunks, int nbins,
                    const double* __restrict__ denom, double* __restrict__ out) {
   __shared__ double sums[kFinishLanes][kFinishOut];
   const int lane = threadIdx.x / kFinishOut, o = threadIdx.x % kFinishOut;
-  const size_t i = static_cast<size_t>(blockIdx.x) * kFinishOut + o;
-  const bool in = i < static_cast<size_t>(rows) * nbins;
-  const int t = in ? static_cast<int>(i / nbins) : 0, b = in ? static_cast<int>(i - static_cast<size_t>(t) * nbins) : 0;
-  const double* p = partial + static_cast<size_t>(t) * nchunks * nbins + b;
-  double s = 0.0;
+  const size_t total = static_cast<size_t>(rows) * nbins;
+  for (size_t i0 = static_cast<size_t>(blockIdx.x) * kFinishOut; i0 < total; i0 += static_cast<size_t>(gridDim.x) * kFinishOut) {
+    const size_t i = i0 + o;
+    const bool in = i < total;
+    const int t = in ? static_cast<int>(i / nbins) : 0, b = in ? static_cast<int>(i - static_cast<size_t>(t) * nbins) : 0;
+    const double* p = partial + static_cast<size_t>(t) * nchunks * nbins + b;
+    double s = 0.0;
 #pragma unroll 4
-  for (int c = lane; c < nchunks; c += kFinishLanes) s += p[static_cast<size_t>(c) * nbins];
-  sums[lane][o] = s;
-  __syncthreads();
-  if (lane != 0 || !in) return;
+    for (int c = lane; c < nchunks; c += kFinishLanes) s += p[static_cast<size_t>(c) * nbins];
+    sums[lane][o] = s;
+    __syncthreads();
+    if (lane == 0 && in) {
 #pragma unroll
-  for (int l = 1; l < kFinishLanes; ++l) s += sums[l][o];
-  const double d = denom[b];
-  double r;
-  if constexpr (SQ) {
-    r = sqrt(s / d);  // 0/0 -> NaN, x/0 -> inf, as numpy
-  } else {
-    r = s / d;
+      for (int l = 1; l < kFinishLanes; ++l) s += sums[l][o];
+      const double d = denom[b];
+      double r;
+      if constexpr (SQ) {
+        r = sqrt(s / d);  // 0/0 -> NaN, x/0 -> inf, as numpy
+      } else {
+        r = s / d;
+      }
+      out[static_cast<size_t>(b) * rows + t] = r;
+    }
+    __syncthreads();  // the sums are rewritten by the next outputs
   }
-  out[static_cast<size_t>(b) * rows + t] = r;
 }
 
 // Rows per workgroup: the largest of 8, 4, 2, 1 whose accumulators (and, in
@@ -356,7 +364,7 @@ extern "C" int fddm_azimuthal_average(const void* d_data, int data_f32, uint64_t
   auto* d_bias = static_cast<double*>(carve(b_den));
   int rc = FDDM_OK;
   const unsigned grid1 = static_cast<unsigned>(ttiles * nchunks);
-  const unsigned grid2 = static_cast<unsigned>((rows * nbins + kFinishOut - 1) / kFinishOut);
+  const unsigned grid2 = static_cast<unsigned>(std::min<uint64_t>((rows * nbins + kFinishOut - 1) / kFinishOut, kFinishGrid));
   auto pass = [&](auto sq) {
     constexpr bool SQ = decltype(sq)::value;
     const size_t lds = static_cast<size_t>(kWaves + (SQ ? 1 : 0)) * T * nbins * sizeof(double);

@@ -1,10 +1,12 @@
-"""Planes of more columns than one launch of a workgroup each can hold
-(2^32 threads), on real hardware: every column is written, with its value."""
+"""Work beyond what one launch holds (2^32 threads), on real hardware: planes
+of more columns, averages of more rows and bins.  Every output is written,
+with its value."""
 
 import numpy as np
 import pytest
 
 from fastddm_amd import next_fast_len
+from fastddm_amd.azimuthalaverage import _reduce
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +52,16 @@ def test_diff_columns_beyond_one_launch(hip):
     finally:
         hip.set_memory_budget(0)
     assert np.array_equal(pieces, out)
+
+
+def test_azimuthal_outputs_beyond_one_launch(hip):
+    # 2^29 averages and a few more, eight threads each
+    rows, nq, nbins = 2**19 + 9, 64, 1024
+    data = np.random.default_rng(5).standard_normal((rows, nq)).astype(np.float32)
+    d_data = hip.DeviceBuffer.from_array(data)
+    bins = np.arange(nq, dtype=np.int32)  # a pixel to a bin: each average is that pixel
+    avg, _ = _reduce(d_data.ptr, True, rows, 1, nq, bins, np.ones(nq), None, nbins, False)
+    d_data.free()
+    hip.release_cache()
+    assert np.array_equal(avg[:nq], data.T.astype(np.float64))
+    assert np.isnan(avg[nq:]).all()
