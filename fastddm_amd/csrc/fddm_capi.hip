@@ -56,9 +56,13 @@ struct fddm_plan {
   // Compensated FP32: child FP64 plan over the first and last kEdgeFrames
   // frames; the lags from index edge_i0 on have at most kEdgeFrames pairs.
   // The child also transforms the raw first frame (its frame raw_at), whose
-  // spectrum PS needs; without a child the plan does that itself (S0).
+  // spectrum PS needs; without a child the plan does that itself (S0).  Its R
+  // and S are the workspace's last pieces.  With two frames to a block (columns
+  // above 2560) they would take more than the frame-0 spectra they replace, so
+  // there its rows use this plan's R, before or after the other frames'
+  // (bytes_edge_R = 0; bytes_R is the larger of the two).
   fddm_plan* edge = nullptr;
-  uint64_t edge_frames = 0, bytes_edge_ws = 0;
+  uint64_t edge_frames = 0, bytes_edge_R = 0, bytes_edge_S = 0;
   uint64_t raw_at = 0;  // child plan: index of the raw first frame (0: none)
   int edge_i0 = 0;
   // timing
@@ -447,7 +451,6 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     p->long_slot = long_slot_bytes(p->logn_t, precision, L);
     p->bytes_long = align256(p->long_slot * static_cast<uint64_t>(p->long_slots));
   }
-  p->ws_bytes = p->bytes_R + p->bytes_S + p->bytes_S0 + p->bytes_flags + p->bytes_long;
   if (has_edge) {
     // FP64 spectra of the edge frames for the lags with few pairs
     const uint64_t E = kEdgeFrames;
@@ -462,12 +465,17 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     c->bytes_R = align256(c->nblocks * c->nxh * H * c->Tb * 16);
     c->bytes_S = align256(c->nq * c->Lp * 16);
     c->bytes_S0 = 0;
-    c->ws_bytes = c->bytes_R + c->bytes_S;
-    p->bytes_edge_ws = c->ws_bytes;
-    p->ws_bytes += p->bytes_edge_ws;
+    // (one R for both costs 64 x 128^2 1.4 %: not where the memory is there)
+    if (p->Tb == 2) {
+      p->bytes_R = std::max(p->bytes_R, c->bytes_R);
+    } else {
+      p->bytes_edge_R = c->bytes_R;
+    }
+    p->bytes_edge_S = c->bytes_S;
     p->edge_i0 = static_cast<int>(nl);
     while (p->edge_i0 > 0 && L - lags[p->edge_i0 - 1] <= E) --p->edge_i0;
   }
+  p->ws_bytes = p->bytes_R + p->bytes_S + p->bytes_S0 + p->bytes_flags + p->bytes_long + p->bytes_edge_R + p->bytes_edge_S;
   *out = p;
   return FDDM_OK;
 }
@@ -547,8 +555,8 @@ int spatial_frames(const fddm_plan* p, const void* img, const void* img0, uint64
 // F(0) of the raw first frame, for PS: in the edge child's spectra, with the
 // edge frames, or by the plan itself into S0.  edge_src: the first and last
 // kEdgeFrames frames, or with in_stack the whole stack (from which the child's
-// rows read them).
-int frame0_stage(fddm_plan* p, const void* frame0, const void* edge_src, bool in_stack, void* R, void* S0, void* edge_ws,
+// rows read them).  R: bytes_R that no other work on the stream needs meanwhile.
+int frame0_stage(fddm_plan* p, const void* frame0, const void* edge_src, bool in_stack, void* R, void* S0, void* edge_S,
                  hipStream_t s, char* err, size_t errlen) {
   if (!p->subtract0) return FDDM_OK;
   if (!p->edge) return spatial_frames(p, frame0, frame0, 1, 0, R, S0, p->Tb, s, err, errlen);
@@ -564,22 +572,27 @@ int frame0_stage(fddm_plan* p, const void* frame0, const void* edge_src, bool in
     ra.gap = p->L - c->L;
   }
   ra.subtract0 = 1;
-  ra.R = edge_ws;
+  ra.R = R;
   FDDM_HIP(ra.logn ? launch_rows_p2(ra, c->precision, s) : launch_rows(ra, c->precision, s));
   ColArgs ca = col_args(c);
-  ca.R = edge_ws;
+  ca.R = R;
   ca.nblocks = c->nblocks;
   ca.Lp = c->Lp;
-  ca.S = static_cast<unsigned char*>(edge_ws) + c->bytes_R;
+  ca.S = edge_S;
   FDDM_HIP(ca.logn ? launch_cols_p2(ca, c->precision, s) : launch_cols(ca, c->precision, s));
   return FDDM_OK;
 }
 
+// The R of frame0_stage in a workspace.
+unsigned char* first_R(const fddm_plan* p, unsigned char* ws) {
+  return p->bytes_edge_R ? ws + p->ws_bytes - p->bytes_edge_S - p->bytes_edge_R : ws;
+}
+
 // Where the time stage finds F(0).
-void set_frame0(const fddm_plan* p, TimeArgs& ta, const void* S0, const void* edge_ws) {
+void set_frame0(const fddm_plan* p, TimeArgs& ta, const void* S0, const void* edge_S) {
   if (!p->subtract0) return;
   if (p->edge) {
-    ta.S0 = static_cast<const unsigned char*>(edge_ws) + p->edge->bytes_R + p->edge->raw_at * 16;
+    ta.S0 = static_cast<const unsigned char*>(edge_S) + p->edge->raw_at * 16;
     ta.s0_stride = p->edge->Lp;
     ta.s0_f64 = 1;
   } else {
@@ -588,8 +601,8 @@ void set_frame0(const fddm_plan* p, TimeArgs& ta, const void* S0, const void* ed
   }
 }
 
-hipError_t fix_lags(const fddm_plan* p, const TimeArgs& ta, const void* edge_S64, hipStream_t s) {
-  return launch_fix(ta, edge_S64, p->edge ? p->edge->Lp : 0, kEdgeFrames, p->edge_i0, p->out_dtype, s);
+hipError_t fix_lags(const fddm_plan* p, const TimeArgs& ta, const void* edge_S, hipStream_t s) {
+  return launch_fix(ta, p->edge ? edge_S : nullptr, p->edge ? p->edge->Lp : 0, kEdgeFrames, p->edge_i0, p->out_dtype, s);
 }
 
 // Spatial stage of the whole stack into the workspace (R, S); the timing
@@ -633,10 +646,10 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
   if (const int rc = check_alignment(p, d_img, d_out, ws, err, errlen)) return rc;
   auto* base = static_cast<unsigned char*>(ws);
   unsigned char* const S0 = base + p->bytes_R + p->bytes_S;
-  unsigned char* const ews = base + p->ws_bytes - p->bytes_edge_ws;
+  unsigned char* const edge_S = base + p->ws_bytes - p->bytes_edge_S;
   int rc;
   if ((rc = record(p, 0, s, err, errlen))) return rc;
-  if ((rc = frame0_stage(p, d_img, d_img, true, base, S0, ews, s, err, errlen))) return rc;
+  if ((rc = frame0_stage(p, d_img, d_img, true, first_R(p, base), S0, edge_S, s, err, errlen))) return rc;
   if ((rc = record(p, 1, s, err, errlen))) return rc;
   if ((rc = run_spatial(p, d_img, ws, s, err, errlen))) return rc;
   TimeArgs ta{};
@@ -645,7 +658,7 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
   ta.L = static_cast<int>(p->L);
   ta.ny = static_cast<int>(p->ny);
   ta.nxh = static_cast<int>(p->nxh);
-  set_frame0(p, ta, S0, ews);
+  set_frame0(p, ta, S0, edge_S);
   ta.lags = static_cast<const uint32_t*>(p->d_lags);
   ta.nl = static_cast<int>(p->nl);
   ta.dt = p->dt;
@@ -665,7 +678,7 @@ int plan_execute(fddm_plan* p, const void* d_img, void* d_out, void* ws, hipStre
   if ((rc = record(p, 4, s, err, errlen))) return rc;
   // compensated FP32 corrections: marked Wiener-Khinchin lags, and the lags
   // with at most kEdgeFrames pairs from FP64 spectra
-  FDDM_HIP(fix_lags(p, ta, p->edge ? ews + p->edge->bytes_R : nullptr, s));
+  FDDM_HIP(fix_lags(p, ta, edge_S, s));
   if ((rc = record(p, 5, s, err, errlen))) return rc;
   if (p->timing_cap > 0 && p->timing_steps < p->timing_cap) ++p->timing_steps;
   return FDDM_OK;
@@ -835,7 +848,7 @@ bool plan_chunks(const fddm_plan* p, uint64_t budget, ChunkPlan* cp) {
   const uint64_t row_out = p->nxh * (p->nl + 2) * osz;
   const uint64_t edge_in = p->edge ? align256(p->edge_frames * frame_b) : 0;
   const uint64_t fixed = align256(frame_b) + p->bytes_S0 + p->bytes_flags + p->bytes_long + edge_in +
-                         p->bytes_edge_ws + 8 * 256;
+                         p->bytes_edge_S + 8 * 256;
   for (int mode = 1; mode <= 2; ++mode) {
     const uint64_t fx = fixed + (mode == 1 ? p->bytes_S : 0);
     if (fx >= budget) continue;
@@ -844,19 +857,20 @@ bool plan_chunks(const fddm_plan* p, uint64_t budget, ChunkPlan* cp) {
     const uint64_t per_row = row_out + (mode == 2 ? p->nxh * p->Lp * csz : 0);
     const uint64_t nb = std::min<uint64_t>(avail / per_block, p->nblocks);
     const uint64_t rows = std::min<uint64_t>(avail / per_row, p->ny);
-    if (nb == 0 || rows == 0) continue;
+    const uint64_t edge_R = p->edge ? p->edge->bytes_R : 0;  // between the frame and the time chunks
+    if (nb == 0 || rows == 0 || edge_R > avail) continue;
     cp->mode = mode;
     cp->frames_per = nb * p->Tb;
     cp->rows_per = rows;
     cp->fixed = fx;
-    cp->work = std::max(nb * per_block, rows * per_row) + 4 * 256;
+    cp->work = std::max({nb * per_block, rows * per_row, edge_R}) + 4 * 256;
     return true;
   }
   return false;
 }
 
 // Time stage and corrections of one launch range (ta.c0, ta.cols, ...).
-int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* edge_S64, hipStream_t s, char* err,
+int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* edge_S, hipStream_t s, char* err,
                 size_t errlen) {
   if (p->mode == MODE_FFT && p->long_t) {
     FDDM_HIP(launch_time_long(ta, p->logn_t, p->precision, p->out_dtype, lng, p->long_slot, p->long_slots, s));
@@ -865,7 +879,7 @@ int time_launch(const fddm_plan* p, const TimeArgs& ta, void* lng, const void* e
   } else {
     FDDM_HIP(launch_diff(ta, p->precision, p->out_dtype, s));
   }
-  FDDM_HIP(fix_lags(p, ta, edge_S64, s));
+  FDDM_HIP(fix_lags(p, ta, edge_S, s));
   return FDDM_OK;
 }
 
@@ -935,23 +949,21 @@ PlanInfo fddm::plan_info(const fddm_plan* p) {
 int finish_from_spectra(fddm_plan* p, const void* frame0, const void* img, const void* edge_in, void* ws,
                         void* d_out, int cols_per, hipStream_t s, char* err, size_t errlen) {
   auto* base = static_cast<unsigned char*>(ws);
-  unsigned char* R = base;
   unsigned char* S = base + p->bytes_R;
   unsigned char* S0 = S + p->bytes_S;
   unsigned char* flags = S0 + p->bytes_S0;
   unsigned char* lng = flags + p->bytes_flags;
   const int nq = static_cast<int>(p->nq);
-  unsigned char* const ews = base + p->ws_bytes - p->bytes_edge_ws;
+  unsigned char* const edge_S = base + p->ws_bytes - p->bytes_edge_S;
   int rc;
-  if ((rc = frame0_stage(p, frame0, edge_in ? edge_in : img, !edge_in, R, S0, ews, s, err, errlen))) return rc;
-  const void* S64 = p->edge ? ews + p->edge->bytes_R : nullptr;
+  if ((rc = frame0_stage(p, frame0, edge_in ? edge_in : img, !edge_in, first_R(p, base), S0, edge_S, s, err, errlen))) return rc;
   TimeArgs ta{};
   ta.S = S;
   ta.Lp = p->Lp;
   ta.L = static_cast<int>(p->L);
   ta.ny = static_cast<int>(p->ny);
   ta.nxh = static_cast<int>(p->nxh);
-  set_frame0(p, ta, S0, ews);
+  set_frame0(p, ta, S0, edge_S);
   ta.lags = static_cast<const uint32_t*>(p->d_lags);
   ta.nl = static_cast<int>(p->nl);
   ta.dt = p->dt;
@@ -963,7 +975,7 @@ int finish_from_spectra(fddm_plan* p, const void* frame0, const void* img, const
   for (int c0 = 0; c0 < nq; c0 += cols_per) {
     ta.c0 = c0;
     ta.cols = std::min(cols_per, nq - c0);
-    if ((rc = time_launch(p, ta, lng, S64, s, err, errlen))) return rc;
+    if ((rc = time_launch(p, ta, lng, edge_S, s, err, errlen))) return rc;
   }
   return FDDM_OK;
 }
@@ -1022,7 +1034,7 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
   unsigned char* flags = take(p->bytes_flags);
   unsigned char* lng = take(p->bytes_long);
   unsigned char* ein = take(p->edge ? p->edge_frames * frame_b : 0);
-  unsigned char* ews = take(p->bytes_edge_ws);
+  unsigned char* edge_S = take(p->bytes_edge_S);
   unsigned char* S = cp.mode == 1 ? take(p->bytes_S) : nullptr;
   unsigned char* work = at;
   std::vector<unsigned char> hostS;
@@ -1065,7 +1077,7 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
       FDDM_HIP(hipMemcpyAsync(ein, img, p->L * frame_b, hipMemcpyHostToDevice, s));
     }
   }
-  if ((rc = frame0_stage(p, frame0, ein, false, work, S0, ews, s, err, errlen))) return rc;
+  if ((rc = frame0_stage(p, frame0, ein, false, work, S0, edge_S, s, err, errlen))) return rc;
   FDDM_HIP(hipStreamSynchronize(s));  // the work region is reused by the time chunks
 
   // time stage in chunks of whole ky rows, local (unshifted) pieces
@@ -1074,14 +1086,13 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
   ta.L = static_cast<int>(p->L);
   ta.ny = static_cast<int>(p->ny);
   ta.nxh = static_cast<int>(p->nxh);
-  set_frame0(p, ta, S0, ews);
+  set_frame0(p, ta, S0, edge_S);
   ta.lags = static_cast<const uint32_t*>(p->d_lags);
   ta.nl = static_cast<int>(p->nl);
   ta.dt = p->dt;
   ta.twt = p->d_twt;
   ta.flags = p->bytes_flags ? flags : nullptr;
   ta.local = 1;
-  const void* S64 = p->edge ? ews + p->edge->bytes_R : nullptr;
   const uint64_t ny = p->ny, nxh = p->nxh, kyw = ny - ny / 2;  // rows ky >= kyw wrap to the top
   uint64_t qchunks = 0;
   for (uint64_t ky0 = 0; ky0 < ny; ky0 += cp.rows_per, ++qchunks) {
@@ -1101,7 +1112,7 @@ int host_path_chunked(fddm_plan* p, HostPathCache& c, const ChunkPlan& cp, const
     ta.cols = static_cast<int>(cols);
     ta.ldo = cols;
     ta.out = opiece;
-    if ((rc = time_launch(p, ta, lng, S64, s, err, errlen))) return rc;
+    if ((rc = time_launch(p, ta, lng, edge_S, s, err, errlen))) return rc;
     // rows ky -> output rows (ky + ny/2) mod ny: at most two contiguous runs
     for (int part = 0; part < 2; ++part) {
       const uint64_t a0 = part == 0 ? ky0 : std::max(ky0, kyw), a1 = part == 0 ? std::min(ky1, kyw) : ky1;
