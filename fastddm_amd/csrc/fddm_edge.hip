@@ -30,18 +30,19 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// One thread per output column o (y-shifted q): for every lag index i >= i0
-// (those with n = L - lags[i] <= E), D = sum_{t < n} |F(t + dt) - F(t)|^2 / n
-// from the FP64 edge spectra S64[q][c] (row pitch lp), where frame f sits in
-// column f if f < E or the stack is short (L <= 2E), else f - (L - 2E).
-// For E = kEdgeFrames and L > 2E the 2E values are loaded once (16 loads in
-// flight) and D depends on n alone: frame t + dt = L - n + t sits in column
-// 2E - n + t, so the E sums run over registers with compile-time indices
-// and are then stored to the lag rows they belong to (same order of
-// additions as the general loop, so the same values).
+// Two threads per output column o (y-shifted q), comp = 0 and 1: for every lag
+// index i >= i0 (those with n = L - lags[i] <= E), D = sum_{t < n}
+// |F(t + dt) - F(t)|^2 / n from the FP64 edge spectra S64[q][c] (row pitch lp),
+// where frame f sits in column f if f < E or the stack is short (L <= 2E), else
+// f - (L - 2E).  For E = kEdgeFrames and L > 2E the 2E values are loaded once
+// (16 loads in flight) and D depends on n alone: frame t + dt = L - n + t sits
+// in column 2E - n + t, so the E sums run over registers with compile-time
+// indices, a thread taking one component, and are then stored to the lag rows
+// they belong to, the two threads in turn.  (One thread for both components
+// took 98 VGPRs, which left the marked columns 4 waves per SIMD.)
 template <typename OutT>
 __device__ __forceinline__ void edge_fix(const TimeArgs& a, const double2* __restrict__ S64, uint64_t lp, int E, int i0,
-                                         int c) {
+                                         int c, int comp) {
   const int q = col_q(a, c), L = a.L, nl = a.nl;
   const uint32_t* __restrict__ lags = a.lags;
   OutT* __restrict__ out = static_cast<OutT*>(a.out);
@@ -49,33 +50,32 @@ __device__ __forceinline__ void edge_fix(const TimeArgs& a, const double2* __res
   const double2* __restrict__ f = S64 + static_cast<size_t>(q) * lp;
   if (E == kEdgeFrames && L > 2 * kEdgeFrames) {
     constexpr int EE = kEdgeFrames;
-    double2 v[2 * EE];
+    const double* __restrict__ fc = reinterpret_cast<const double*>(f) + comp;
+    double v[2 * EE];
 #pragma unroll
-    for (int k = 0; k < 2 * EE; ++k) v[k] = f[k];
-    double dn[EE];  // dn[n - 1]: D of the lag with n pairs
+    for (int k = 0; k < 2 * EE; ++k) v[k] = fc[2 * k];
+    double dn[EE] = {};  // dn[n - 1]: n D of the lag with n pairs
 #pragma unroll
-    for (int n = 1; n <= EE; ++n) {
-      double acc = 0.0;
+    for (int t = 0; t < EE; ++t)
 #pragma unroll
-      for (int t = 0; t < n; ++t) {
-        const double2 x = v[2 * EE - n + t], y = v[t];
-        const double dr = x.x - y.x, di = x.y - y.y;
-        acc += dr * dr + di * di;
+      for (int n = t + 1; n <= EE; ++n) {
+        const double d = v[2 * EE - n + t] - v[t];
+        dn[n - 1] += d * d;
       }
-      dn[n - 1] = acc / n;
-    }
-    for (int i = i0; i < nl; ++i) {
+#pragma unroll
+    for (int n = 0; n < EE; ++n) dn[n] += __shfl_xor(dn[n], 1, 64);
+    for (int i = i0 + comp; i < nl; i += 2) {
       const int n = L - static_cast<int>(lags[i]);  // 1 <= n <= EE
       double D = dn[0];
 #pragma unroll
       for (int k = 1; k < EE; ++k)
         if (n == k + 1) D = dn[k];
-      out[static_cast<size_t>(i) * ldo + o] = static_cast<OutT>(D);
+      out[static_cast<size_t>(i) * ldo + o] = static_cast<OutT>(D / n);
     }
     return;
   }
   const int shift = L <= 2 * E ? 0 : L - 2 * E;
-  for (int i = i0; i < nl; ++i) {
+  for (int i = i0 + comp; i < nl; i += 2) {
     const int d = static_cast<int>(lags[i]), n = L - d;
     double acc = 0.0;
     for (int t = 0; t < n; ++t) {
@@ -92,11 +92,11 @@ __device__ __forceinline__ void edge_fix(const TimeArgs& a, const double2* __res
 // Both corrections in one launch: they write different lags (at most E pairs;
 // more than 32).  S64 null: no edge lags; a.flags null: no marked columns.
 template <typename OutT>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, 8)
     k_fix(TimeArgs a, const double2* __restrict__ S64, uint64_t lp, int E, int i0) {
-  if (S64)
-    for (int c = blockIdx.x * kThreads + threadIdx.x; c < a.cols; c += gridDim.x * kThreads)
-      edge_fix<OutT>(a, S64, lp, E, i0, c);
+  if (S64)  // (both threads of a column are inside or outside the loop)
+    for (int c = static_cast<int>((blockIdx.x * kThreads + threadIdx.x) / 2); c < a.cols; c += static_cast<int>(gridDim.x) * (kThreads / 2))
+      edge_fix<OutT>(a, S64, lp, E, i0, c, threadIdx.x & 1);
   if (!a.flags) return;
   // workgroup g owns the columns g + m G (G workgroups); their flags are read
   // at once, one per thread, the marked columns listed in LDS, and the
@@ -159,9 +159,10 @@ __global__ void __launch_bounds__(kThreads)
 hipError_t launch_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype, hipStream_t s) {
   if (i0 >= a.nl) S64 = nullptr;
   if (a.nl <= 0 || a.cols <= 0 || (!S64 && !a.flags)) return hipSuccess;
-  // a column per thread for the edge lags; up to 2048 workgroups share the marked columns
-  const unsigned edge = (a.cols + kThreads - 1) / kThreads;
-  const dim3 grid(a.flags ? std::max(edge, static_cast<unsigned>(std::min(a.cols, 2048))) : edge);
+  // two threads per column for the edge lags; 2048 workgroups, which the chip
+  // holds at once, share the marked columns (and the edge lags then)
+  const unsigned edge = (static_cast<unsigned>(a.cols) + kThreads / 2 - 1) / (kThreads / 2);
+  const dim3 grid(a.flags ? static_cast<unsigned>(std::min(a.cols, 2048)) : edge);
   if (out_dtype == OUT_F32) {
     hipLaunchKernelGGL(k_fix<float>, grid, dim3(kThreads), 0, s, a, static_cast<const double2*>(S64), lp, E, i0);
   } else {
