@@ -214,15 +214,85 @@ __device__ __forceinline__ A add_mirrored(A a, A b, int lane) {
 }
 constexpr int kRowMirror = 0x140, kHalfMirror = 0x141, kQuadSwap1 = 0xb1, kQuadSwap2 = 0x4e;
 
-// A wave works on 64 / SEG columns, one per segment of SEG lanes; lane l of a
-// segment takes t = l, l + SEG, ...; four lags at a time (at the end of the
-// list the last lag stands in for the missing ones).
+// The segment's last lane ends with its sum.
+template <int SEG, typename A>
+__device__ __forceinline__ A segment_scan(A v) {
+  v = row_scan(v);
+  if constexpr (SEG == 32) v += wave::dpp_zero<wave::kRowBcast15, 0xa>(v);
+  return v;
+}
+
+// Lags i0 .. i0 + K - 1 of a segment's series; lane l of a segment takes
+// t = l, l + SEG, ...
+template <typename C, typename Acc, typename OutT, int SEG, int K>
+__device__ __forceinline__ void segment_lags(const TimeArgs& a, const C* ser, int i0, size_t oq, int lane, bool valid) {
+  const int L = a.L, sl = lane & (SEG - 1);
+  const C* const p = ser + sl;
+  OutT* __restrict__ const out = static_cast<OutT*>(a.out) + oq;
+  int d[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) d[k] = __builtin_amdgcn_readfirstlane(static_cast<int>(a.lags[i0 + k]));
+  Acc acc[K] = {};
+  const int whole = (L - d[K - 1]) & ~(SEG - 1);  // (lags ascend) t below it: inside the series for every lag
+#pragma unroll 2
+  for (int t = 0; t < whole; t += SEG) {
+    const C v = p[t];
+    C u[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) u[k] = p[t + d[k]];
+    const Acc vx = static_cast<Acc>(v.x), vy = static_cast<Acc>(v.y);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const Acc dr = static_cast<Acc>(u[k].x) - vx, di = static_cast<Acc>(u[k].y) - vy;
+      acc[k] += dr * dr + di * di;
+    }
+  }
+  for (int t0 = whole; t0 < L - d[0]; t0 += SEG) {
+    const int t = t0 + sl;
+    const C v = ser[min(t, L - 1)];
+    const Acc vx = static_cast<Acc>(v.x), vy = static_cast<Acc>(v.y);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const C u = ser[min(t + d[k], L - 1)];
+      const Acc dr = static_cast<Acc>(u.x) - vx, di = static_cast<Acc>(u.y) - vy;
+      acc[k] += t + d[k] < L ? dr * dr + di * di : Acc(0);  // (not a product: the frames may hold NaN)
+    }
+  }
+  if constexpr (K == 4) {
+    // the four sums of every segment, traded while adding; k: the lag this lane ends with
+    Acc s;
+    int k;
+    if constexpr (SEG == 16) {
+      s = add_mirrored<kHalfMirror, 4>(add_mirrored<kRowMirror, 8>(acc[0], acc[1], lane),
+                                       add_mirrored<kRowMirror, 8>(acc[2], acc[3], lane), lane);
+      k = ((lane >> 3) & 1) | ((lane >> 1) & 2);
+    } else {
+      s = add_mirrored<kRowMirror, 8>(add_traded<true>(acc[0], acc[1]), add_traded<true>(acc[2], acc[3]), lane);
+      s += wave::dpp_zero<kHalfMirror, 0xf>(s);
+      k = ((lane >> 4) & 1) | ((lane >> 2) & 2);
+    }
+    s += wave::dpp_zero<kQuadSwap1, 0xf>(s);
+    s += wave::dpp_zero<kQuadSwap2, 0xf>(s);
+    const int dk = k == 0 ? d[0] : k == 1 ? d[1] : k == 2 ? d[2] : d[3];
+    const bool writer = SEG == 16 ? (lane & 3) == 0 : (lane & 7) == 0;
+    if (writer && valid)
+      out[static_cast<size_t>(i0 + k) * a.ldo] = static_cast<OutT>(s / static_cast<Acc>(L - dk));
+  } else {
+    static_assert(K == 1, "batches of four, the rest one by one");
+    const Acc s = segment_scan<SEG>(acc[0]);
+    if (valid && sl == SEG - 1) out[static_cast<size_t>(i0) * a.ldo] = static_cast<OutT>(s / static_cast<Acc>(L - d[0]));
+  }
+}
+
+// A wave works on 64 / SEG columns, one per segment of SEG lanes, four lags at
+// a time and the rest one by one (with stand-ins for a last batch of four, one
+// lag took as long as four: 300 x 512^2 in compensated FP32 113 us, now 95).
 template <typename T, typename OutT, int PREC, int SEG>
 __global__ void __launch_bounds__(kThreads) k_diff_short(TimeArgs a, int wg_per_xcd, int pitch) {
   using C = cplx_t<T>;
   using Acc = acc_t<PREC>;
   static_assert(SEG == 16 || SEG == 32, "segment");
-  constexpr int QPW = 64 / SEG, K = kLagBatch;
+  constexpr int QPW = 64 / SEG;
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int sl = lane & (SEG - 1), seg = lane / SEG;
@@ -252,68 +322,15 @@ __global__ void __launch_bounds__(kThreads) k_diff_short(TimeArgs a, int wg_per_
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  auto segment_scan = [](Acc v) {  // the segment's last lane ends with its sum
-    v = row_scan(v);
-    if constexpr (SEG == 32) v += wave::dpp_zero<wave::kRowBcast15, 0xa>(v);
-    return v;
-  };
-  sr = segment_scan(sr);
-  si = segment_scan(si);
-  s2 = segment_scan(s2);
+  sr = segment_scan<SEG>(sr);
+  si = segment_scan<SEG>(si);
+  s2 = segment_scan<SEG>(s2);
   const size_t oq = col_out(a, c);
   if (valid && sl == SEG - 1) store_moments<Acc, C, OutT>(a, q, oq, sr, si, s2);
 
-  const C* const p = ser + sl;
-  OutT* __restrict__ const out = static_cast<OutT*>(a.out) + oq;
-  for (int i0 = 0; i0 < nl; i0 += K) {
-    int d[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) d[k] = __builtin_amdgcn_readfirstlane(static_cast<int>(a.lags[min(i0 + k, nl - 1)]));
-    Acc acc[K] = {};
-    const int whole = (L - d[K - 1]) & ~(SEG - 1);  // (lags ascend) t below it: inside the series for every lag
-#pragma unroll 2
-    for (int t = 0; t < whole; t += SEG) {
-      const C v = p[t];
-      C u[K];
-#pragma unroll
-      for (int k = 0; k < K; ++k) u[k] = p[t + d[k]];
-      const Acc vx = static_cast<Acc>(v.x), vy = static_cast<Acc>(v.y);
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const Acc dr = static_cast<Acc>(u[k].x) - vx, di = static_cast<Acc>(u[k].y) - vy;
-        acc[k] += dr * dr + di * di;
-      }
-    }
-    for (int t0 = whole; t0 < L - d[0]; t0 += SEG) {
-      const int t = t0 + sl;
-      const C v = ser[min(t, L - 1)];
-      const Acc vx = static_cast<Acc>(v.x), vy = static_cast<Acc>(v.y);
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const C u = ser[min(t + d[k], L - 1)];
-        const Acc dr = static_cast<Acc>(u.x) - vx, di = static_cast<Acc>(u.y) - vy;
-        acc[k] += t + d[k] < L ? dr * dr + di * di : Acc(0);  // (not a product: the frames may hold NaN)
-      }
-    }
-    // the four sums of every segment, traded while adding; k: the lag this lane ends with
-    Acc s;
-    int k;
-    if constexpr (SEG == 16) {
-      s = add_mirrored<kHalfMirror, 4>(add_mirrored<kRowMirror, 8>(acc[0], acc[1], lane),
-                                       add_mirrored<kRowMirror, 8>(acc[2], acc[3], lane), lane);
-      k = ((lane >> 3) & 1) | ((lane >> 1) & 2);
-    } else {
-      s = add_mirrored<kRowMirror, 8>(add_traded<true>(acc[0], acc[1]), add_traded<true>(acc[2], acc[3]), lane);
-      s += wave::dpp_zero<kHalfMirror, 0xf>(s);
-      k = ((lane >> 4) & 1) | ((lane >> 2) & 2);
-    }
-    s += wave::dpp_zero<kQuadSwap1, 0xf>(s);
-    s += wave::dpp_zero<kQuadSwap2, 0xf>(s);
-    const int dk = k == 0 ? d[0] : k == 1 ? d[1] : k == 2 ? d[2] : d[3];
-    const bool writer = SEG == 16 ? (lane & 3) == 0 : (lane & 7) == 0;
-    if (writer && valid && i0 + k < nl)
-      out[static_cast<size_t>(i0 + k) * a.ldo] = static_cast<OutT>(s / static_cast<Acc>(L - dk));
-  }
+  const int nb = nl / kLagBatch;
+  for (int b = 0; b < nb; ++b) segment_lags<C, Acc, OutT, SEG, kLagBatch>(a, ser, b * kLagBatch, oq, lane, valid);
+  for (int i = nb * kLagBatch; i < nl; ++i) segment_lags<C, Acc, OutT, SEG, 1>(a, ser, i, oq, lane, valid);
 }
 
 // Series too long for the LDS: one column per wave, read from L2.
@@ -356,7 +373,9 @@ hipError_t launch(K kernel, unsigned grid, unsigned threads, size_t lds, hipStre
 }
 
 // Four or two columns per wave while their series leave four workgroups per
-// CU; then a column per workgroup, with as many waves as keep 16 per CU or
+// CU, or eight for four columns and a few lags, where loading the series is
+// most of the time (300 x 512^2 in compensated FP32: one lag 105 -> 95 us, five
+// 124 -> 118, six 129 -> 138); then a column per workgroup, with as many waves as keep 16 per CU or
 // more beside the series' LDS; beyond the LDS, a wave per column.
 template <typename T, typename OutT, int PREC>
 hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
@@ -369,7 +388,7 @@ hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
     const int wpx = per_xcd(kWaves * qpw);
     return launch(kernel, 8u * wpx, kThreads, csz * pitch * kWaves * qpw, s, a, wpx, pitch);
   };
-  if (csz * pitch * kWaves * 4 <= 40 * 1024) return segments(k_diff_short<T, OutT, PREC, 16>, 4);
+  if (csz * pitch * kWaves * 4 <= (a.nl < 6 ? 20 : 40) * 1024) return segments(k_diff_short<T, OutT, PREC, 16>, 4);
   if (csz * pitch * kWaves * 2 <= 40 * 1024) return segments(k_diff_short<T, OutT, PREC, 32>, 2);
   const size_t lds = csz * a.L + 3 * 16 * sizeof(double);
   if (lds <= 159 * 1024) {
