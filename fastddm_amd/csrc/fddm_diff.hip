@@ -12,9 +12,10 @@
 // and in compensated FP32 VALU issue (6.5 instructions per difference,
 // widening included).
 //
-// k_diff_short: four or two columns per wave, one per 16 or 32 lanes, each
-// series in its own LDS slice: with short series fewer lanes per column leave
-// less of them idle in the last step over t and share one reduction.
+// k_diff_short: four, two or one column per wave, one per 16, 32 or 64 lanes,
+// each series in its own LDS slice: with short series fewer lanes per column
+// leave less of them idle in the last step over t and share one reduction, and
+// with few lags a workgroup works on four columns or more at once.
 //
 // k_diff_long: one column per wave, for series beyond the LDS.
 //
@@ -151,7 +152,7 @@ __device__ __forceinline__ void wave_lags(const TimeArgs& a, const C* ser, int i
 }
 
 template <typename T, typename OutT, int PREC>
-__global__ void __launch_bounds__(1024) k_diff(TimeArgs a, int wg_per_xcd) {
+__global__ void __launch_bounds__(1024) k_diff(TimeArgs a, int wg_per_xcd, int nb) {
   using C = cplx_t<T>;
   using Acc = acc_t<PREC>;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -198,7 +199,6 @@ __global__ void __launch_bounds__(1024) k_diff(TimeArgs a, int wg_per_xcd) {
     }
     store_moments<Acc, C, OutT>(a, q, oq, sr, si, s2);
   }
-  const int nb = a.nl / kLagBatch;
   for (int b = wid; b < nb; b += NW) wave_lags<C, Acc, OutT, kLagBatch>(a, ser, b * kLagBatch, oq, lane);
   // the remaining lags, one by one, on the waves that had a batch less
   for (int i = nb * kLagBatch + (wid - nb % NW + NW) % NW; i < a.nl; i += NW)
@@ -217,6 +217,7 @@ constexpr int kRowMirror = 0x140, kHalfMirror = 0x141, kQuadSwap1 = 0xb1, kQuadS
 // The segment's last lane ends with its sum.
 template <int SEG, typename A>
 __device__ __forceinline__ A segment_scan(A v) {
+  if constexpr (SEG == 64) return wave::incl_scan(v);
   v = row_scan(v);
   if constexpr (SEG == 32) v += wave::dpp_zero<wave::kRowBcast15, 0xa>(v);
   return v;
@@ -287,11 +288,12 @@ __device__ __forceinline__ void segment_lags(const TimeArgs& a, const C* ser, in
 // A wave works on 64 / SEG columns, one per segment of SEG lanes, four lags at
 // a time and the rest one by one (with stand-ins for a last batch of four, one
 // lag took as long as four: 300 x 512^2 in compensated FP32 113 us, now 95).
+// Nothing of one column waits for another wave.
 template <typename T, typename OutT, int PREC, int SEG>
 __global__ void __launch_bounds__(kThreads) k_diff_short(TimeArgs a, int wg_per_xcd, int pitch) {
   using C = cplx_t<T>;
   using Acc = acc_t<PREC>;
-  static_assert(SEG == 16 || SEG == 32, "segment");
+  static_assert(SEG == 16 || SEG == 32 || SEG == 64, "segment");
   constexpr int QPW = 64 / SEG;
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -301,7 +303,9 @@ __global__ void __launch_bounds__(kThreads) k_diff_short(TimeArgs a, int wg_per_
   if (cw >= a.cols) return;  // whole waves: nothing below synchronises the workgroup
   const bool valid = cw + seg < a.cols;
   const int c = valid ? cw + seg : a.cols - 1;  // (idle segments repeat the last column and store nothing)
-  const int q = col_q(a, c), L = a.L, nl = a.nl;
+  int q = col_q(a, c);
+  if constexpr (SEG == 64) q = __builtin_amdgcn_readfirstlane(q);
+  const int L = a.L, nl = a.nl;
   const C* __restrict__ src = static_cast<const C*>(a.S) + static_cast<size_t>(q - a.s_q0) * a.Lp;
   C* const ser = reinterpret_cast<C*>(smem) + static_cast<size_t>(wid * QPW + seg) * pitch;
   Acc sr = 0, si = 0, s2 = 0;
@@ -329,8 +333,13 @@ __global__ void __launch_bounds__(kThreads) k_diff_short(TimeArgs a, int wg_per_
   if (valid && sl == SEG - 1) store_moments<Acc, C, OutT>(a, q, oq, sr, si, s2);
 
   const int nb = nl / kLagBatch;
-  for (int b = 0; b < nb; ++b) segment_lags<C, Acc, OutT, SEG, kLagBatch>(a, ser, b * kLagBatch, oq, lane, valid);
-  for (int i = nb * kLagBatch; i < nl; ++i) segment_lags<C, Acc, OutT, SEG, 1>(a, ser, i, oq, lane, valid);
+  if constexpr (SEG == 64) {
+    for (int b = 0; b < nb; ++b) wave_lags<C, Acc, OutT, kLagBatch>(a, ser, b * kLagBatch, oq, lane);
+    for (int i = nb * kLagBatch; i < nl; ++i) wave_lags<C, Acc, OutT, 1>(a, ser, i, oq, lane);
+  } else {
+    for (int b = 0; b < nb; ++b) segment_lags<C, Acc, OutT, SEG, kLagBatch>(a, ser, b * kLagBatch, oq, lane, valid);
+    for (int i = nb * kLagBatch; i < nl; ++i) segment_lags<C, Acc, OutT, SEG, 1>(a, ser, i, oq, lane, valid);
+  }
 }
 
 // Series too long for the LDS: one column per wave, read from L2.
@@ -373,10 +382,21 @@ hipError_t launch(K kernel, unsigned grid, unsigned threads, size_t lds, hipStre
 }
 
 // Four or two columns per wave while their series leave four workgroups per
-// CU, or eight for four columns and a few lags, where loading the series is
-// most of the time (300 x 512^2 in compensated FP32: one lag 105 -> 95 us, five
-// 124 -> 118, six 129 -> 138); then a column per workgroup, with as many waves as keep 16 per CU or
-// more beside the series' LDS; beyond the LDS, a wave per column.
+// CU, or eight with a few lags, where loading the series is most of the time
+// (300 x 512^2 in compensated FP32: one lag 105 -> 95 us, five 124 -> 118, six
+// 129 -> 138; 500 x 256^2, four lags: two columns per wave 54 us, one 48).  Plain
+// FP32, with the least work per value read, takes eight and six (300 x 256^2,
+// 24 lags: four columns 55 us, two 44; 500 x 256^2: two 79, one 69).
+// Then, with few lags, a column per wave: a workgroup per column leaves most of
+// its waves without a lag (256^2 columns, kernel time with a workgroup and with
+// a wave per column: 700 samples in compensated FP32, 1 lag 66 and 50 us, 24
+// lags 175 and 161, 60 lags 302 and 301; 400 in FP64, 1 lag 65 and 49 us, 24 lags
+// 119 and 100; longer series want more waves per LDS: 1200 in compensated FP32, 1
+// lag 86 and 99 us).
+// Then a column per workgroup, with as many waves as keep 16 per CU or more
+// beside the series' LDS, every lag by itself where there is a wave for each
+// (4000 samples, 4 lags: as one batch 1145 us in FP64, by themselves 457);
+// beyond the LDS, a wave per column.
 template <typename T, typename OutT, int PREC>
 hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
   constexpr size_t csz = sizeof(cplx_t<T>);
@@ -388,13 +408,18 @@ hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
     const int wpx = per_xcd(kWaves * qpw);
     return launch(kernel, 8u * wpx, kThreads, csz * pitch * kWaves * qpw, s, a, wpx, pitch);
   };
-  if (csz * pitch * kWaves * 4 <= (a.nl < 6 ? 20 : 40) * 1024) return segments(k_diff_short<T, OutT, PREC, 16>, 4);
-  if (csz * pitch * kWaves * 2 <= 40 * 1024) return segments(k_diff_short<T, OutT, PREC, 32>, 2);
+  constexpr bool plain = PREC == PREC_FP32;
+  const size_t lds1 = csz * pitch * kWaves;  // of a workgroup with one column per wave
+  const bool few = a.nl < 6;
+  if (4 * lds1 <= (few || plain ? 20 : 40) << 10) return segments(k_diff_short<T, OutT, PREC, 16>, 4);
+  if (2 * lds1 <= (few ? 20 : plain ? 28 : 40) << 10) return segments(k_diff_short<T, OutT, PREC, 32>, 2);
+  if (lds1 <= (csz == 16 ? 34 : 28) << 10 && a.nl < 32) return segments(k_diff_short<T, OutT, PREC, 64>, 1);
   const size_t lds = csz * a.L + 3 * 16 * sizeof(double);
   if (lds <= 159 * 1024) {
     const unsigned threads = lds <= 40 * 1024 ? 256 : lds <= 80 * 1024 ? 512 : 1024;
     // a launch holds less than 2^32 threads: larger planes (16.7 M columns of
     // 256 threads) in several
+    const int nb = a.nl <= static_cast<int>(threads / 64) ? 0 : a.nl / kLagBatch;
     const int64_t most = static_cast<int64_t>((uint64_t(1) << 32) / threads) - 8;
     for (int64_t c = 0; c < nq; c += most) {
       TimeArgs part = a;
@@ -402,7 +427,7 @@ hipError_t diff_l(const TimeArgs& a, hipStream_t s) {
       part.cols = static_cast<int>(std::min<int64_t>(most, nq - c));
       if (a.local) part.out = static_cast<OutT*>(a.out) + c;  // (stored by column of the launch)
       const int wpx = (part.cols + 7) / 8;
-      const hipError_t e = launch(k_diff<T, OutT, PREC>, 8u * wpx, threads, lds, s, part, wpx);
+      const hipError_t e = launch(k_diff<T, OutT, PREC>, 8u * wpx, threads, lds, s, part, wpx, nb);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 def test_diff_columns_beyond_one_launch(hip):
-    L, H, W, lag = 641, 8, 8, 320  # a column per workgroup of 256 threads
+    L, H, W, lag = 897, 8, 8, 448  # a column per workgroup of 256 threads
     nx, ny = 8192, 4116
     nxh = nx // 2 + 1
     assert nxh * ny > 2**24 and next_fast_len(ny, "hip") == ny
