@@ -566,10 +566,10 @@ int frame0_stage(fddm_plan* p, const void* frame0, const void* edge_src, bool in
   ra.img0 = edge_src;
   ra.L = c->L;
   ra.frames = c->raw_at + 1;
-  ra.raw = c->raw_at;
+  ra.raw = static_cast<uint32_t>(c->raw_at);
   if (in_stack && p->L > c->L) {
     ra.split = kEdgeFrames;
-    ra.gap = p->L - c->L;
+    ra.gap = static_cast<uint32_t>(p->L - c->L);
   }
   ra.subtract0 = 1;
   ra.R = R;

@@ -84,17 +84,17 @@ __global__ void __launch_bounds__(kThreads) k_rows(RowArgs a) {
   C* __restrict__ R = static_cast<C*>(a.R);
   const C* __restrict__ tw = static_cast<const C*>(a.twx);
 
+  const sp::BlockFrames<sizeof(T) == 8> fr(a, t0, Tb, plane);
+  const bool sub = a.subtract0 != 0;
   for (int g0 = 0; g0 < Tb / 2; g0 += G) {
     for (int w = tid; w < G * nx; w += kThreads) {
       const int p = w / nx, x = w - p * nx;
       T va = 0, vb = 0;
       if (x < W) {
-        const uint64_t ta = t0 + 2 * (g0 + p), tb2 = ta + 1;
+        const int ka = 2 * (g0 + p), kb = ka + 1;
         const size_t i0 = static_cast<size_t>(y) * W + x;
-        if (sp::frame_here(a, ta))
-          va = load_pixel<Tin, T>(img, ref, sp::frame_src(a, ta) * plane + i0, i0, sp::frame_sub(a, ta));
-        if (sp::frame_here(a, tb2))
-          vb = load_pixel<Tin, T>(img, ref, sp::frame_src(a, tb2) * plane + i0, i0, sp::frame_sub(a, tb2));
+        if (fr.here(ka)) va = load_pixel<Tin, T>(img, ref, fr.at(ka, plane) + i0, i0, sub && !fr.is_raw(ka));
+        if (kb < fr.n) vb = load_pixel<Tin, T>(img, ref, fr.first + kb * plane + i0, i0, sub);
         if (win) {
           const T wv = win[i0];
           va *= wv;

@@ -13,16 +13,15 @@ namespace fddm {
 // `window` (H*W of T) may be null.  subtract0: use I(t) - I0 in place of I(t),
 // where I0 is the frame at img0 (the stack's frame 0; img itself when the
 // launch starts at frame 0).  `frames` limits how many leading frames are
-// transformed (>= 1).  Frames t >= split come from frame t + gap of img, and
-// frame t == raw (> 0; none: 0) is frame 0 of img without the subtraction
-// (frame_src, frame_here, frame_sub in fddm_spatial.hpp).
+// transformed (>= 1).  In FP64 frames t >= split (a multiple of Tb) come from
+// frame t + gap of img, and frame t == raw (even; none: 2^32 - 1) is frame 0 of
+// img without the subtraction (BlockFrames in fddm_spatial.hpp).
 struct RowArgs {
   const void* img;
   const void* img0;
   int in_dtype;
   uint64_t L;       // frames present (t < L; besides raw)
   uint64_t frames;  // frames to transform
-  uint64_t split, gap, raw;
   int H, W, nx, Tb, G;
   int logn;  // > 0: power-of-two kernel for nx = 2^logn (twx holds its tables)
   const void* window;
@@ -32,6 +31,7 @@ struct RowArgs {
   const void* twx;
   void* R;
   int generic;  // 1: the generic workgroup kernel even where k_rows_mr applies
+  uint32_t split = 0, gap = 0, raw = ~uint32_t(0);
 };
 
 // Stage (a) column pass + q-major store: R -> S[q][t], q = ky * nxh + kx,

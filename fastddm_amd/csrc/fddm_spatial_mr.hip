@@ -136,7 +136,7 @@ __device__ __forceinline__ void fft_wave_mr(cplx_t<T>* row, const FftDesc& d, co
 // y .. y + G - 1 of a frame block, G = 64 / P, wave p transforms the pair p of
 // each on P lanes.  rs: LDS slots per pair row; vec: pixel rows start 8-byte
 // aligned and the loaded width is a multiple of the vector (host-checked).
-template <typename Tin, typename T, int NP, int KMAX, int P>
+template <typename Tin, typename T, int NP, int KMAX, int P, bool EDGES = false>
 __global__ void __launch_bounds__(64 * NP, (rows_min_waves<KMAX, T>())) k_rows_mr(RowArgs a, uint32_t nitems, int rs, int vec) {
   using C = cplx_t<T>;
   constexpr int NT = 64 * NP, TB = 2 * NP, G = 64 / P;
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(64 * NP, (rows_min_waves<KMAX, T>())) k_rows_m
     int lane = tid & (P - 1), tidi = tid;
     asm volatile("" : "+v"(lane), "+v"(tidi));
     const int y0 = static_cast<int>(static_cast<uint32_t>(item) % hg) * G;
-    const uint64_t tb = static_cast<uint32_t>(item) / hg, ta = tb * TB + 2 * p;
+    const uint64_t tb = static_cast<uint32_t>(item) / hg;
     // this lane's image row (rows past the last repeat it and are not stored)
     int y = y0;
     C* row = buf + p * rs;
@@ -189,11 +189,11 @@ __global__ void __launch_bounds__(64 * NP, (rows_min_waves<KMAX, T>())) k_rows_m
       row += g * NP * rs;
     }
     // (uniform over the wave)
-    const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
-    const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
+    const sp::BlockFrames<EDGES> fr(a, tb * TB, TB, plane);
+    const bool has_a = fr.here(2 * p), has_b = 2 * p + 1 < fr.n, sub_a = sub && !fr.is_raw(2 * p);
     const size_t yo = static_cast<size_t>(y) * W;
-    const Tin* __restrict__ ra = img + sp::frame_src(a, ta) * plane + yo;
-    const Tin* __restrict__ rb = img + sp::frame_src(a, ta + 1) * plane + yo;
+    const Tin* __restrict__ ra = img + fr.at(2 * p, plane) + yo;
+    const Tin* __restrict__ rb = img + fr.first + (2 * p + 1) * plane + yo;
     const Tin* __restrict__ r0 = img0 + yo;
     auto scalar_rows = [&]() {
 #pragma unroll 4
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(64 * NP, (rows_min_waves<KMAX, T>())) k_rows_m
         const T w = win ? win[yo + x0] : T(1);
         const Tin p0 = sub ? r0[x0] : Tin(0);
         const T fa = has_a ? sp::pixel_value<Tin, T>(ra[x0], p0, sub_a, w) : T(0);
-        const T fb = has_b ? sp::pixel_value<Tin, T>(rb[x0], p0, sub_b, w) : T(0);
+        const T fb = has_b ? sp::pixel_value<Tin, T>(rb[x0], p0, sub, w) : T(0);
         row[mr_pad<T>(x0)] = C{fa, fb};
       }
     };
@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(64 * NP, (rows_min_waves<KMAX, T>())) k_rows_m
                 for (int v = 0; v < VX; ++v) {
                   const T w = win ? wv[h].v[v] : T(1);
                   const T fa = has_a ? sp::pixel_value<Tin, T>(va[h].v[v], v0[h].v[v], sub_a, w) : T(0);
-                  const T fb = has_b ? sp::pixel_value<Tin, T>(vb[h].v[v], v0[h].v[v], sub_b, w) : T(0);
+                  const T fb = has_b ? sp::pixel_value<Tin, T>(vb[h].v[v], v0[h].v[v], sub, w) : T(0);
                   row[mr_pad<T>(x0 + v)] = C{fa, fb};
                 }
               }
@@ -381,12 +381,19 @@ size_t rows_mr_lds(const RowArgs& a, int precision, int* rs) {
 
 template <typename Tin, typename T, int NP>
 hipError_t rows_mr_np(const RowArgs& a, size_t lds, int rs, int vec, hipStream_t s) {
-  auto kernel = a.nx <= kMrShort ? k_rows_mr<Tin, T, NP, kMrShort, 64> : k_rows_mr<Tin, T, NP, kMrLong, 64>;
   int group = 1;
-  if constexpr (NP == (sizeof(T) == 4 ? 8 : 4)) {
-    group = rows_mr_group(a, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32);
-    if (group == 2) kernel = k_rows_mr<Tin, T, NP, kMrHalf, 32>;
-    if (group == 4) kernel = k_rows_mr<Tin, T, NP, kMrQuarter, 16>;
+  if constexpr (NP == (sizeof(T) == 4 ? 8 : 4)) group = rows_mr_group(a, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32);
+  auto pick = [&](auto edges) {
+    constexpr bool E = decltype(edges)::value;
+    if constexpr (NP == (sizeof(T) == 4 ? 8 : 4)) {
+      if (group == 2) return k_rows_mr<Tin, T, NP, kMrHalf, 32, E>;
+      if (group == 4) return k_rows_mr<Tin, T, NP, kMrQuarter, 16, E>;
+    }
+    return a.nx <= kMrShort ? k_rows_mr<Tin, T, NP, kMrShort, 64, E> : k_rows_mr<Tin, T, NP, kMrLong, 64, E>;
+  };
+  auto kernel = pick(std::false_type{});
+  if constexpr (sizeof(T) == 8 && NP <= 4) {  // (edge frames: FP64, blocks of at most 8)
+    if (a.raw != ~uint32_t(0)) kernel = pick(std::true_type{});
   }
   const uint64_t nblocks = (a.frames + a.Tb - 1) / a.Tb;
   const uint32_t items = static_cast<uint32_t>(nblocks * ((static_cast<uint64_t>(a.H) + group - 1) / group));

@@ -68,6 +68,8 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
   const C* __restrict__ tw = static_cast<const C*>(a.twx);
   const Tin* __restrict__ row0 = img + static_cast<size_t>(y) * W;  // first frame of the launch, row y
   const Tin* __restrict__ ref0 = static_cast<const Tin*>(a.img0) + static_cast<size_t>(y) * W;  // subtracted frame
+  const sp::BlockFrames<sizeof(T) == 8> fr(a, t0, TB, plane);
+  const bool sub = a.subtract0 != 0;
 
   // pairs (2p, 2p+1) -> LDS, element (p, x) at logical p NX + x
   if (W == NX && (static_cast<size_t>(W) * sizeof(Tin)) % 8 == 0) {
@@ -81,14 +83,12 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
     };
     for (int e = tid; e < NP * G; e += kThreads) {
       const int p = e / G, g = e - p * G, x0 = g * VX;
-      const uint64_t ta = t0 + 2 * p;
-      const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
-      const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
+      const bool has_a = fr.here(2 * p), has_b = 2 * p + 1 < fr.n, sub_a = sub && !fr.is_raw(2 * p);
       Vec va{}, vb{}, v0{};
       WVec wv;
-      if (has_a) va = *reinterpret_cast<const Vec*>(row0 + sp::frame_src(a, ta) * plane + x0);
-      if (has_b) vb = *reinterpret_cast<const Vec*>(row0 + sp::frame_src(a, ta + 1) * plane + x0);
-      if (sub_a || sub_b) v0 = *reinterpret_cast<const Vec*>(ref0 + x0);
+      if (has_a) va = *reinterpret_cast<const Vec*>(row0 + fr.at(2 * p, plane) + x0);
+      if (has_b) vb = *reinterpret_cast<const Vec*>(row0 + fr.first + (2 * p + 1) * plane + x0);
+      if (sub) v0 = *reinterpret_cast<const Vec*>(ref0 + x0);
       // the VX window values in one or two vector loads issued with the
       // pixels (one load per value: row pass 9.3 ms at 1024^2 x 4000, this
       // way 7.9 ms)
@@ -98,22 +98,19 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
       for (int v = 0; v < VX; ++v) {
         const T w = win ? wv.v[v] : T(1);
         const T fa = has_a ? pixel_value<Tin, T>(va.v[v], v0.v[v], sub_a, w) : T(0);
-        const T fb = has_b ? pixel_value<Tin, T>(vb.v[v], v0.v[v], sub_b, w) : T(0);
+        const T fb = has_b ? pixel_value<Tin, T>(vb.v[v], v0.v[v], sub, w) : T(0);
         d[v] = C{fa, fb};
       }
     }
   } else {
     for (int e = tid; e < NP * NX; e += kThreads) {
       const int p = e >> LOGX, x = e & (NX - 1);
-      const uint64_t ta = t0 + 2 * p;
       T fa = 0, fb = 0;
       if (x < W) {
         const T w = win ? win[static_cast<size_t>(y) * W + x] : T(1);
-        const Tin x0v = a.subtract0 ? ref0[x] : Tin(0);
-        if (sp::frame_here(a, ta))
-          fa = pixel_value<Tin, T>(row0[sp::frame_src(a, ta) * plane + x], x0v, sp::frame_sub(a, ta), w);
-        if (sp::frame_here(a, ta + 1))
-          fb = pixel_value<Tin, T>(row0[sp::frame_src(a, ta + 1) * plane + x], x0v, sp::frame_sub(a, ta + 1), w);
+        const Tin x0v = sub ? ref0[x] : Tin(0);
+        if (fr.here(2 * p)) fa = pixel_value<Tin, T>(row0[fr.at(2 * p, plane) + x], x0v, sub && !fr.is_raw(2 * p), w);
+        if (2 * p + 1 < fr.n) fb = pixel_value<Tin, T>(row0[fr.first + (2 * p + 1) * plane + x], x0v, sub, w);
       }
       buf[padi(e)] = C{fa, fb};
     }
@@ -189,6 +186,7 @@ __global__ void __launch_bounds__(64 * NP, (LOGX <= 9 ? 2 : 1) * (sizeof(T) == 8
   const Tin* __restrict__ img = static_cast<const Tin*>(a.img);
   const T* __restrict__ win = static_cast<const T*>(a.window);
   const size_t plane = static_cast<size_t>(H) * NX;
+  const bool sub = a.subtract0 != 0;
   const T half_norm = static_cast<T>(0.5 * a.norm);
   const uint32_t kstride = static_cast<uint32_t>(H) * TB;
   {
@@ -201,20 +199,18 @@ __global__ void __launch_bounds__(64 * NP, (LOGX <= 9 ? 2 : 1) * (sizeof(T) == 8
 
   Vec va[PER], vb[PER], v0[PER];
   WVec wv[PER];
-  auto load = [&](uint32_t item) {
-    const int y = static_cast<int>(item % H);
-    const uint64_t ta = static_cast<uint64_t>(item / H) * TB + 2 * p;
+  auto load = [&](const sp::BlockFrames<sizeof(T) == 8>& fr, int y) {
     const Tin* __restrict__ row0 = img + static_cast<size_t>(y) * NX;
     const Tin* __restrict__ ref0 = static_cast<const Tin*>(a.img0) + static_cast<size_t>(y) * NX;
-    const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
-    const Tin* __restrict__ rowa = row0 + sp::frame_src(a, ta) * plane;
-    const Tin* __restrict__ rowb = row0 + sp::frame_src(a, ta + 1) * plane;
+    const bool has_a = fr.here(2 * p), has_b = 2 * p + 1 < fr.n;
+    const Tin* __restrict__ rowa = row0 + fr.at(2 * p, plane);
+    const Tin* __restrict__ rowb = row0 + fr.first + (2 * p + 1) * plane;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int x0 = (lane + 64 * k) * VX;
       va[k] = has_a ? *reinterpret_cast<const Vec*>(rowa + x0) : Vec{};
       vb[k] = has_b ? *reinterpret_cast<const Vec*>(rowb + x0) : Vec{};
-      v0[k] = a.subtract0 ? *reinterpret_cast<const Vec*>(ref0 + x0) : Vec{};
+      v0[k] = sub ? *reinterpret_cast<const Vec*>(ref0 + x0) : Vec{};
       if (win) wv[k] = *reinterpret_cast<const WVec*>(win + static_cast<size_t>(y) * NX + x0);
     }
   };
@@ -224,12 +220,12 @@ __global__ void __launch_bounds__(64 * NP, (LOGX <= 9 ? 2 : 1) * (sizeof(T) == 8
   uint32_t item = blockIdx.x;
   __syncthreads();  // twiddles in LDS
   for (; item < nitems; item += gridDim.x) {
-    load(item);
     const int y = static_cast<int>(item % H);
-    const uint64_t tb = item / H, ta = tb * TB + 2 * p;
+    const uint64_t tb = item / H;
+    const sp::BlockFrames<sizeof(T) == 8> fr(a, tb * TB, TB, plane);
+    load(fr, y);
     // (uniform over the wave)
-    const bool has_a = sp::frame_here(a, ta), has_b = sp::frame_here(a, ta + 1);
-    const bool sub_a = sp::frame_sub(a, ta), sub_b = sp::frame_sub(a, ta + 1);
+    const bool has_a = fr.here(2 * p), has_b = 2 * p + 1 < fr.n, sub_a = sub && !fr.is_raw(2 * p);
     // registers -> this wave's row: frames (2p, 2p+1) as one complex row
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
@@ -239,7 +235,7 @@ __global__ void __launch_bounds__(64 * NP, (LOGX <= 9 ? 2 : 1) * (sizeof(T) == 8
       for (int v = 0; v < VX; ++v) {
         const T w = win ? wv[k].v[v] : T(1);
         const T fa = has_a ? pixel_value<Tin, T>(va[k].v[v], v0[k].v[v], sub_a, w) : T(0);
-        const T fb = has_b ? pixel_value<Tin, T>(vb[k].v[v], v0[k].v[v], sub_b, w) : T(0);
+        const T fb = has_b ? pixel_value<Tin, T>(vb[k].v[v], v0[k].v[v], sub, w) : T(0);
         d[v] = C{fa, fb};
       }
     }
