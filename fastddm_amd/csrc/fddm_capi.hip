@@ -18,6 +18,7 @@
 #include <mutex>
 #include <new>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "fddm_copy_pool.hpp"
@@ -160,30 +161,37 @@ bool factorize(uint64_t n, FftDesc& d) {
   return r == 1;
 }
 
-// Per-pass twiddle tables in the order of FftDesc:
+// Per-pass twiddle tables in the two orders of FftDesc:
 // pass with radix R after Ns points stores exp(-2 pi i r k / (Ns R)) at
-// k (R-1) + r - 1 for k < Ns, r = 1 .. R-1; n - 1 entries in all.  Evaluated
-// in long double and rounded once.
+// k (R-1) + r - 1 for k < Ns, r = 1 .. R-1; n - 1 entries in all.  Picked from
+// the n roots of unity, evaluated in long double and rounded once.
 template <typename T>
 std::vector<T> twiddles(const FftDesc& d) {
-  std::vector<T> w;
-  w.reserve(2 * static_cast<size_t>(d.n));
   const long double two_pi = 6.283185307179586476925286766559005768L;
-  const int counts[8] = {d.c7, d.c5, d.c3, d.c10, d.c6, d.c8, d.c4, d.c2};
-  const int radix[8] = {7, 5, 3, 10, 6, 8, 4, 2};
-  long long ns = 1;
-  for (int g = 0; g < 8; ++g)
-    for (int i = 0; i < counts[g]; ++i) {
-      const int R = radix[g];
-      for (long long k = 0; k < ns; ++k)
-        for (int r = 1; r < R; ++r) {
-          const long double ang = -two_pi * static_cast<long double>(r * k) / static_cast<long double>(ns * R);
-          w.push_back(static_cast<T>(cosl(ang)));
-          w.push_back(static_cast<T>(sinl(ang)));
-        }
-      ns *= R;
-    }
-  if (w.empty()) w.assign(2, T(0));
+  std::vector<T> root(2 * static_cast<size_t>(d.n)), w;
+  for (long long j = 0; j < d.n; ++j) {
+    const long double ang = -two_pi * static_cast<long double>(j) / static_cast<long double>(d.n);
+    root[2 * j] = static_cast<T>(cosl(ang));
+    root[2 * j + 1] = static_cast<T>(sinl(ang));
+  }
+  w.reserve(4 * static_cast<size_t>(fft_table(d.n)));
+  const std::pair<int, int> plans[2][8] = {
+      {{7, d.c7}, {5, d.c5}, {3, d.c3}, {10, d.c10}, {6, d.c6}, {8, d.c8}, {4, d.c4}, {2, d.c2}},
+      {{10, d.c10}, {8, d.c8}, {7, d.c7}, {6, d.c6}, {5, d.c5}, {4, d.c4}, {3, d.c3}, {2, d.c2}}};
+  for (const auto& plan : plans) {
+    long long ns = 1;
+    for (const auto& [R, count] : plan)
+      for (int i = 0; i < count; ++i) {
+        for (long long k = 0; k < ns; ++k)
+          for (int r = 1; r < R; ++r) {
+            const T* const z = &root[2 * (r * k * (d.n / (ns * R)))];
+            w.push_back(z[0]);
+            w.push_back(z[1]);
+          }
+        ns *= R;
+      }
+    if (d.n <= 1) w.insert(w.end(), 2, T(0));
+  }
   return w;
 }
 

@@ -33,14 +33,19 @@ enum OutDtype : int { OUT_F64 = 0, OUT_F32 = 1 };
 enum Mode : int { MODE_DIFF = 0, MODE_FFT = 1 };
 
 // Mixed-radix factorisation of one FFT length, passed to kernels by value:
-// n = 7^c7 5^c5 3^c3 10^c10 6^c6 8^c8 4^c4 2^c2, passes applied in that order.
-// A pass of radix R writes at a stride of its radix times the points so far:
-// an odd radix first keeps those strides off the LDS banks' powers of two
-// (radix 8 first, as a power of two: 8 lanes on a bank).
+// n = 7^c7 5^c5 3^c3 10^c10 6^c6 8^c8 4^c4 2^c2.  The kernels with a transform
+// to a wave (fddm_spatial_mr.hip) apply the passes in that order: a pass of
+// radix R writes at a stride of its radix times the points so far, and an odd
+// radix first keeps those strides off the LDS banks' powers of two (radix 8
+// first, as a power of two: 8 lanes on a bank).  The workgroup engine
+// (fddm_fft.hpp) applies them in descending order: its first pass, which has no
+// twiddles to read and multiply by, is then the widest.  The twiddle tables of
+// both orders lie one after the other, n - 1 entries each (fft_table).
 struct FftDesc {
   int n;
   int c7, c5, c3, c10, c6, c8, c4, c2;
 };
+__host__ __device__ constexpr int fft_table(int n) { return n > 1 ? n - 1 : 1; }
 
 // Elements of an LDS buffer holding n logical elements with one pad slot
 // every 32 (see lds_pad in fddm_fft.hpp).

@@ -240,15 +240,16 @@ __device__ __forceinline__ void stockham_pass(cplx_t<T>* buf, int off, int n, in
 }
 
 // Forward FFT (unnormalised) of nb transforms in LDS.  E bounds the elements
-// per thread: E * nthr >= n * nb.  `tw` is the plan's concatenated per-pass
-// twiddle table (in the order of FftDesc).  The caller
+// per thread: E * nthr >= n * nb.  `tw`: the plan's twiddle tables (FftDesc),
+// the second of which is this engine's.  The caller
 // synchronises before the call; the data are synchronised on return.  One
 // loop per radix (rather than a switch over a pass list) keeps the register
 // allocation of the eight pass variants disjoint.
-template <typename T, int E, bool TIF>
+template <typename T, int E, bool TIF, bool PAIRS = true>
 __device__ void fft_lds(cplx_t<T>* buf, int off, const FftDesc& d, int nb, int lognb, int bstride,
                         int estride, const cplx_t<T>* __restrict__ tw, int tid, int nthr) {
   const int n = d.n;
+  tw += fft_table(n);
   int ns = 1;
 #define FDDM_PASSES(RAD, COUNT)                                                              \
   for (int i = 0; i < d.COUNT; ++i) {                                                        \
@@ -257,13 +258,17 @@ __device__ void fft_lds(cplx_t<T>* buf, int off, const FftDesc& d, int nb, int l
     tw += ns * (RAD - 1);                                                                    \
     ns *= RAD;                                                                               \
   }
-  FDDM_PASSES(7, c7)
-  FDDM_PASSES(5, c5)
-  FDDM_PASSES(3, c3)
-  FDDM_PASSES(10, c10)
-  FDDM_PASSES(6, c6)
+  if constexpr (PAIRS) {
+    FDDM_PASSES(10, c10)
+  }
   FDDM_PASSES(8, c8)
+  FDDM_PASSES(7, c7)
+  if constexpr (PAIRS) {
+    FDDM_PASSES(6, c6)
+  }
+  FDDM_PASSES(5, c5)
   FDDM_PASSES(4, c4)
+  FDDM_PASSES(3, c3)
   FDDM_PASSES(2, c2)
 #undef FDDM_PASSES
 }
