@@ -195,6 +195,21 @@ std::vector<T> twiddles(const FftDesc& d) {
   return w;
 }
 
+// Columns up to which series of a short transform take the workgroup kernel
+// (fddm_time_p2.hip).  It gives a column 64 or 128 threads of its own and looks
+// at the requested lags only; the register kernel (fddm_time_wave.hip) puts two
+// or four columns on a wave, whose one long chain of instructions an empty chip
+// does not hide.  Kernel time of the register and the workgroup kernel in
+// compensated FP32: 200 x 32^2, all lags 14.4 and 12.6 us, 200 x 64^2 15.1 and
+// 15.1; with 20 lags 14.6 and 12.6, 200 x 128^2 23.2 and 21.3; in FP64 200 x 32^2
+// 16.0 and 14.5 us, 500 x 40^2 with 20 lags 18.2 and 15.6, 500 x 52^2 18.9 and 19.0.
+uint64_t short_columns(int logn, int precision, uint64_t nl, uint64_t L) {
+  const bool few = nl <= L / 8;
+  if (logn > kShortMaxLog) return 0;
+  if (precision != PREC_FP64) return few ? 8400 : logn == 10 ? 850 : 1100;
+  return logn == 8 ? (few ? 8400 : 1100) : logn == 9 ? (few ? 1400 : 1100) : logn == 10 ? 850 : 0;
+}
+
 // Twiddles of the power-of-two time plans: passes 1 .. np-1 of p2_plan, then
 // of p2_half_plan (length N/2), each [k][r] = exp(-2 pi i r k / (NS R)), then
 // (cos, sin)(2 pi k / N) for k < N/2.
@@ -370,7 +385,7 @@ int fddm::plan_create_ex(fddm_plan** out, int mode, int dtype, uint64_t L, uint6
     if (nt < 2 * L - 1) return fail(set_err(err, errlen, FDDM_ERR_ARG, "nt must be >= 2*length-1"));
     int logn = kTimeMinLog;
     while ((1ull << logn) < 2 * L - 1) ++logn;
-    if (logn - 1 <= time_pair_log(precision)) {
+    if (p->nq > short_columns(logn, precision, nl, L) && logn - 1 <= time_pair_log(precision)) {
       p->wave_t = logn - 1;
     } else if (logn > time_p2_log(precision)) {
       // longer series: four-step transform through device scratch
@@ -502,7 +517,7 @@ int record(fddm_plan* p, int slot, hipStream_t s, char* err, size_t errlen) {
 
 // Time kernel of series that need no device scratch.
 hipError_t launch_time(const fddm_plan* p, const TimeArgs& ta, hipStream_t s) {
-  if (!p->wave_t) return launch_time_p2(ta, p->precision, p->out_dtype, s);
+  if (!p->wave_t) return launch_time_p2(ta, p->logn_t, p->precision, p->out_dtype, s);
   if (p->wave_t <= time_wave_max_log(p->precision))
     return launch_time_wave(ta, p->wave_t, p->precision, p->out_dtype, s);
   return launch_time_pair(ta, p->precision, p->out_dtype, s);

@@ -51,16 +51,22 @@ __host__ __device__ constexpr int fft_table(int n) { return n > 1 ? n - 1 : 1; }
 // every 32 (see lds_pad in fddm_fft.hpp).
 __host__ __device__ constexpr int lds_padded_size(int n) { return n + (n >> 5) + 1; }
 
-// Time-axis plans of the workgroup kernel (fddm_time_p2.hip), N = 2^14 in FP32
-// and 2^13 in FP64: threads per transform, number of passes (3 or 4) and the
-// radices of the first transform in order; the first and last passes have a
-// whole number of butterflies per thread.  FP64 takes three passes on 256
-// threads, which measured faster than four at its register and LDS footprint.
+// Time-axis plans of the workgroup kernel (fddm_time_p2.hip), N = 2^8 to 2^11
+// (kShortMaxLog), and 2^14 in FP32 and 2^13 in FP64: threads per transform, number
+// of passes (3 or 4) and the radices of the first transform in order; the first
+// and last passes have a whole number of butterflies per thread.  FP64 takes
+// three passes on 256 threads at 2^13, which measured faster than four at its
+// register and LDS footprint.
 struct P2Plan {
   int threads, np, r0, r1, r2, r3;
 };
 __host__ __device__ constexpr P2Plan p2_plan(int logn) {
-  return logn == 13 ? P2Plan{256, 3, 16, 16, 32, 1} : P2Plan{1024, 4, 16, 8, 8, 16};
+  return logn == 8    ? P2Plan{64, 4, 4, 4, 4, 4}
+         : logn == 9  ? P2Plan{64, 3, 8, 8, 8, 1}
+         : logn == 10 ? P2Plan{64, 3, 16, 16, 4, 1}
+         : logn == 11 ? P2Plan{128, 3, 16, 16, 8, 1}
+         : logn == 13 ? P2Plan{256, 3, 16, 16, 32, 1}
+                      : P2Plan{1024, 4, 16, 8, 8, 16};
 }
 __host__ __device__ constexpr int p2_radix(const P2Plan& P, int i) {
   return i == 0 ? P.r0 : i == 1 ? P.r1 : i == 2 ? P.r2 : P.r3;
@@ -70,7 +76,12 @@ __host__ __device__ constexpr int p2_radix(const P2Plan& P, int i) {
 // same threads (passes with fewer butterflies than threads leave whole waves
 // idle), followed by a per-lag untangling step.
 __host__ __device__ constexpr P2Plan p2_half_plan(int logn) {
-  return logn == 13 ? P2Plan{256, 3, 16, 16, 16, 1} : P2Plan{1024, 4, 16, 8, 8, 8};
+  return logn == 8    ? P2Plan{64, 4, 4, 4, 4, 2}
+         : logn == 9  ? P2Plan{64, 3, 8, 8, 4, 1}
+         : logn == 10 ? P2Plan{64, 3, 8, 8, 8, 1}
+         : logn == 11 ? P2Plan{128, 3, 16, 16, 4, 1}
+         : logn == 13 ? P2Plan{256, 3, 16, 16, 16, 1}
+                      : P2Plan{1024, 4, 16, 8, 8, 8};
 }
 // Points already combined before pass i (product of the earlier radices).
 __host__ __device__ constexpr int p2_ns(const P2Plan& P, int i) { return i == 0 ? 1 : p2_ns(P, i - 1) * p2_radix(P, i - 1); }
@@ -88,6 +99,7 @@ __host__ __device__ constexpr int p2_tw_h(int logn, int i) {
 }
 __host__ __device__ constexpr int p2_tw_post(int logn) { return p2_tw_h(logn, p2_half_plan(logn).np); }
 constexpr int kTimeMinLog = 8;  // shortest time transform
+constexpr int kShortMaxLog = 11;  // longest of the workgroup kernel's short plans
 
 template <typename T> struct Cplx;
 template <> struct Cplx<float> { using type = float2; };

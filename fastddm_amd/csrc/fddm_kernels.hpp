@@ -105,9 +105,10 @@ __device__ __forceinline__ C frame0_spectrum(const TimeArgs& a, int q) {
 hipError_t launch_rows(const RowArgs& a, int precision, hipStream_t s);
 hipError_t launch_cols(const ColArgs& a, int precision, hipStream_t s);
 hipError_t launch_diff(const TimeArgs& a, int precision, int out_dtype, hipStream_t s);
-// Time kernel with one column per workgroup (fddm_time_p2.hip), N = 2^time_p2_log.
+// Time kernel with a column's transforms in LDS (fddm_time_p2.hip), N = 2^logn,
+// logn in [kTimeMinLog, kShortMaxLog] or time_p2_log.
 int time_p2_log(int precision);
-hipError_t launch_time_p2(const TimeArgs& a, int precision, int out_dtype, hipStream_t s);
+hipError_t launch_time_p2(const TimeArgs& a, int logn, int precision, int out_dtype, hipStream_t s);
 // Time kernel with every transform in the registers of one wave
 // (fddm_time_wave.hip): M = 2^logm samples (zero-padded, M >= L), logm in
 // [7, time_wave_max_log].  time_wave_tables: the tables it reads from a.twt.

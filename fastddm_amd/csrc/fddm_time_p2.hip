@@ -1,26 +1,28 @@
-// Stage (c) + (e), fft mode, for series of 4097 to 8192 frames (FP32) and 2049
-// to 4096 (FP64): one column per workgroup, its transforms in LDS.  (Shorter
-// series run in registers: fddm_time_wave.hip, fddm_time_pair.hip; longer ones
-// through device scratch: fddm_time_long.hip.)
+// Stage (c) + (e), fft mode, with a column's transforms in LDS: for series of
+// 4097 to 8192 frames (FP32) and 2049 to 4096 (FP64), one column per workgroup,
+// and for up to 1024 frames in planes of few columns (short_columns in
+// fddm_capi.hip), two or four per workgroup.  (Other series run in registers:
+// fddm_time_wave.hip, fddm_time_pair.hip; longer ones through device scratch:
+// fddm_time_long.hip.)
 //
 // D(q, dt) does not depend on the zero-padded transform length N as long as
 // N >= 2L - 1, so the time stage runs at N = 2^ceil(log2(2L - 1)), here 2^14
-// (FP32) or 2^13 (FP64), with plans fixed at compile time (p2_plan in
-// fddm_common.hpp): three or four passes per transform with radix 8..32
+// (FP32), 2^13 (FP64) or 2^8 to 2^11, with plans fixed at compile time (p2_plan
+// in fddm_common.hpp): three or four passes per transform with radix 4..32
 // butterflies, all strides and LDS offsets known to the compiler, and padded
 // LDS addresses (one slot per 32 elements) that stay linear in the butterfly
 // index.
 //
-// Per q, the workgroup of T threads:
+// Per q, the workgroup, or one of its groups, of T threads:
 //   1. loads its first-pass inputs F(t), t = u + b T + r N/R0, straight from
 //      HBM (t >= N/2 >= L is the zero padding and is never read);
 //   2. compensated paths: subtracts the temporal mean (one group reduction);
 //   3. FFT1 (radices R0 .. RL); the last pass stays in registers, |G|^2 is
 //      formed there and written to LDS as z(n) = P(2n) + i P(2n+1);
 //   4. forms the prefix sums of |F(t)|^2 (double on the compensated paths)
-//      and keeps the first and last kEdge samples: in FP64 from the first
-//      pass's registers before step 3 (wave scans per segment of the register
-//      layout, held in registers until a buffer half is free), in FP32, whose
+//      and keeps the first and last kEdge samples: from the first pass's
+//      registers before step 3 (wave scans per segment of the register layout,
+//      held in registers until a buffer half is free), at 2^14, where the
 //      registers are full, from a second (cache-resident) read of the series
 //      with contiguous segments per thread and one group scan;
 //   5. the second forward transform of the real P runs as one complex
@@ -31,9 +33,10 @@
 //      PS and VAR, and stores them fftshifted along y.
 //
 // The output is lag-major, so each lag store of one q writes one value into
-// its own line.  The compensated paths run steps 1-6 for two neighbouring
-// output columns in turn, keep the first column's D in registers and store
-// each lag's two values together.
+// its own line.  Workgroups of several q interleave them across lanes; on the
+// long plans the compensated paths run steps 1-6 for two neighbouring output
+// columns in turn, keep the first column's D in registers and store each lag's
+// two values together.
 #include <type_traits>
 #include <utility>
 
@@ -45,6 +48,7 @@ namespace fddm {
 namespace {
 using namespace p2;
 
+constexpr int kMinThreads = 256;  // workgroup size of plans with fewer threads (several q each)
 constexpr int kEdge = 32;
 // Compensated FP32: the float transforms leave an absolute error of at most
 // about 3e-7 x sum_t |G|^2 in (L - dt) D (measured worst case over 2 x 10^9
@@ -100,32 +104,40 @@ typedef float OutPairF __attribute__((ext_vector_type(2)));
 template <typename O>
 using OutPair = std::conditional_t<sizeof(O) == 8, OutPairD, OutPairF>;
 
-// Workgroup shape and LDS layout of the time kernel at N = 2^LOGN.
+// Workgroup shape and LDS layout of the time kernel at N = 2^LOGN.  Plans of
+// fewer than kMinThreads threads put G = kMinThreads / TPT q in a workgroup:
+// neighbours, whose lags the lag loop interleaves across lanes, so each lag
+// store covers G adjacent output values.
 template <int LOGN, typename T, bool SUB>
 struct P2Lds {
   static constexpr P2Plan P = p2_plan(LOGN);
   static constexpr int N = 1 << LOGN, TPT = P.threads, WPT = TPT / 64;
-  using Acc = std::conditional_t<SUB, double, float>;
+  // (sums in double wherever fddm_time_wave.hip, which takes the larger planes
+  // of these lengths, has them)
+  using Acc = std::conditional_t<SUB || LOGN <= kShortMaxLog, double, float>;
   static constexpr size_t csz = sizeof(cplx_t<T>);
   static constexpr int S = N / 2 / TPT;  // first-pass segments of TPT samples below N/2
   // Prefix sums formed from the first pass's registers (no second read of the
   // series) where the registers allow it; at N = 16384 the series is read
   // again from cache.
   static constexpr bool REG = LOGN <= 13;
-  // wave totals (REG: by segment and wave, then their offsets) and, last, their sum
+  // Lags of at most kEdge pairs: direct sums.
+  static constexpr bool DIRECT = SUB || LOGN <= kShortMaxLog;
+  // per q: wave totals (REG: by segment and wave, then their offsets) and, last, their sum
   static constexpr int CH = (REG ? S : 1) * WPT + 1;
-  // The LDS holds one q and leaves registers free: the workgroup transforms
-  // the q of two neighbouring output columns one after the other and keeps
-  // the first one's D in registers (KMAX lag iterations per thread), so each
-  // lag store writes both columns at once.  (Plain FP32 would spill.)
-  static constexpr int SEQ = SUB ? 2 : 1;
-  static constexpr int KMAX = (N / 2 + TPT - 1) / TPT;
+  static constexpr int NT = TPT < kMinThreads ? kMinThreads : TPT, G = NT / TPT;
+  // The long plans' LDS holds one q and leaves registers free: the workgroup
+  // transforms the q of two neighbouring output columns one after the other
+  // and keeps the first one's D in registers (KMAX lag iterations per thread),
+  // so each lag store writes both columns at once.  (Plain FP32 would spill.)
+  static constexpr int SEQ = SUB && G == 1 ? 2 : 1;
+  static constexpr int KMAX = (N / 2 + NT - 1) / NT;
   // Register bound: FP32 gets the 4 waves per SIMD its LDS allows.
   static constexpr int kMinWaves = SEQ > 1 && sizeof(T) == 4 ? 4 : 1;
-  static constexpr size_t buf = static_cast<size_t>(lds_padded_size(N)) * csz;
-  static constexpr size_t edge = static_cast<size_t>(2) * kEdge * csz;
-  static constexpr size_t red = 2 * WPT * sizeof(double);
-  static constexpr size_t chunk = static_cast<size_t>(CH) * sizeof(Acc);
+  static constexpr size_t buf = static_cast<size_t>(G) * lds_padded_size(N) * csz;
+  static constexpr size_t edge = static_cast<size_t>(G) * 2 * kEdge * csz;
+  static constexpr size_t red = 2 * (NT / 64) * sizeof(double);
+  static constexpr size_t chunk = static_cast<size_t>(G) * CH * sizeof(Acc);
   static constexpr size_t bytes = buf + edge + red + chunk;
 };
 
@@ -151,13 +163,13 @@ __device__ __forceinline__ void p2_passes(cplx_t<T>* buf, const cplx_t<T>* __res
 }
 
 template <typename T, typename OutT, int LOGN, bool SUB>
-__global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SUB>::kMinWaves))
+__global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::NT), (P2Lds<LOGN, T, SUB>::kMinWaves))
     k_time_p2(TimeArgs a, int wg_per_xcd, int nq) {
   using C = cplx_t<T>;
   using Lay = P2Lds<LOGN, T, SUB>;
   using Acc = typename Lay::Acc;
   constexpr P2Plan P = Lay::P;
-  constexpr int N = 1 << LOGN, TPT = P.threads, WPT = Lay::WPT, NP = P.np;
+  constexpr int N = 1 << LOGN, TPT = P.threads, G = Lay::G, WPT = Lay::WPT, NP = P.np;
   constexpr bool F64 = sizeof(T) == 8;
   constexpr int R0 = P.r0, RL = p2_radix(P, NP - 1), NH = N / 2;
   using A0 = Pass<T, N, R0, 1, TPT>;                          // first pass (registers)
@@ -174,7 +186,8 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
   // output columns share its L2.
   constexpr int SEQ = Lay::SEQ;
   const int wgi = (blockIdx.x & 7) * wg_per_xcd + (blockIdx.x >> 3);
-  if (SEQ * wgi >= nq) return;  // whole workgroup: before any barrier
+  const int cbase = SEQ * G * wgi;  // first column of this workgroup (nq: columns of the launch)
+  if (cbase >= nq) return;  // whole workgroup: before any barrier
   const int L = a.L;
   const C* __restrict__ tw = static_cast<const C*>(a.twt);
   OutT* __restrict__ out = static_cast<OutT*>(a.out);
@@ -188,12 +201,15 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
     // across the loop (the thread index is opaque to the optimiser there)
     int tid = threadIdx.x;
     if constexpr (SEQ > 1) asm volatile("" : "+v"(tid));
-    const int u = tid, lane = tid & 63, wg = u >> 6;
-    C* const buf = reinterpret_cast<C*>(smem);
-    C* const edge = reinterpret_cast<C*>(smem + Lay::buf);
+    const int g = G > 1 ? tid / TPT : 0, u = tid - g * TPT, lane = tid & 63, wg = u >> 6;
+    C* const buf0 = reinterpret_cast<C*>(smem);
+    C* const edge0 = reinterpret_cast<C*>(smem + Lay::buf);
     double* const red = reinterpret_cast<double*>(smem + Lay::buf + Lay::edge);
-    Acc* const chunk = reinterpret_cast<Acc*>(smem + Lay::buf + Lay::edge + Lay::red);
-    const int c = SEQ * wgi + sq;  // column of the launch (of nq)
+    Acc* const chunk0 = reinterpret_cast<Acc*>(smem + Lay::buf + Lay::edge + Lay::red);
+    C* const buf = buf0 + g * lds_padded_size(N);
+    C* const edge = edge0 + g * 2 * kEdge;
+    Acc* const chunk = chunk0 + g * Lay::CH;
+    const int c = cbase + (SEQ > 1 ? sq : g);  // column of the launch
     const bool active = c < nq;
     const int q = active ? col_q(a, c) : a.s_q0;
     const C* __restrict__ src = static_cast<const C*>(a.S) + static_cast<size_t>(q - a.s_q0) * a.Lp;
@@ -263,7 +279,7 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
         for (int r = 0; r < RH; ++r) {
           const int sg = b + r * MB0, t = sg * TPT + u;
           const C f = v0[b][r];  // zero for t >= L and for an inactive column
-          if constexpr (SUB) {
+          if constexpr (Lay::DIRECT) {
             if (t < kEdge && t < L) edge[t] = f;
             if (t >= L - kEdge && t < L) edge[t - L + 2 * kEdge] = f;
           }
@@ -373,26 +389,32 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
       p2_passes<T, LOGN, true, 0, NPH>(buf, tw, u);
     }
 
-    // 6. lags: thread u serves lag indices nl - 1 - u, stepping by TPT.  Lags in
-    // reverse order: the largest lags (direct sums, longest loops) all fall in
-    // the first wave(s).
+    // 6. lags: thread tid serves q group h = tid mod G and lag indices nl - 1 - v,
+    // v = tid / G, stepping by TPT, so neighbouring lanes store the same lag of
+    // neighbouring q.  Lags in reverse order: the largest lags (direct sums,
+    // longest loops) all fall in the first wave(s).
     {
-      {
+      const int h = tid % G, v = tid / G, ch = SEQ > 1 ? c : cbase + h;
+      if (SEQ > 1 || ch < nq) {
+        const C* const hbuf = buf0 + h * lds_padded_size(N);  // Z
+        const Acc* const htail = reinterpret_cast<const Acc*>(hbuf + padi(NH));
+        const C* const hedge = edge0 + h * 2 * kEdge;
+        const Acc* const hchunk = chunk0 + h * Lay::CH;
         bool flag = false;  // some lag of this q needs the direct recomputation
         Acc hptot = 0;  // psum(L)
         if constexpr (Lay::REG) {
-          hptot = chunk[S * WPT];
+          hptot = hchunk[S * WPT];
         } else {
 #pragma unroll
-          for (int w = 0; w < WPT; ++w) hptot += chunk[w];
+          for (int w = 0; w < WPT; ++w) hptot += hchunk[w];
         }
-        // This thread's lag iterations k (index nl - 1 - u - k STEP, at most KL
-        // of them since nl < N/2).  Where registers are to spare (two columns)
-        // their lag values and (cos, sin) entries are loaded first, so those
+        // This thread's lag iterations k (index nl - 1 - v - k STEP, at most KL
+        // of them since nl < N/2).  Where registers are to spare (two columns,
+        // or FP64, whose LDS allows at most 4 waves per SIMD) their lag values and (cos, sin) entries are loaded first, so those
         // loads overlap instead of opening every iteration.
         constexpr int STEP = TPT;
         constexpr int KL = (NH + STEP - 1) / STEP;
-        constexpr bool PRE = SEQ > 1;
+        constexpr bool PRE = SEQ > 1 || F64;
         // (cos, sin)(2 pi d / N) of lag d: unsigned 32-bit indices, so each
         // entry address is one 64-bit shift-add from this base
         const C* __restrict__ const twp = tw + TWP;
@@ -401,7 +423,7 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
         if constexpr (PRE) {
 #pragma unroll
           for (int k = 0; k < KL; ++k) {
-            const int i = a.nl - 1 - u - k * STEP;
+            const int i = a.nl - 1 - v - k * STEP;
             dk[k] = i >= 0 ? static_cast<int>(a.lags[static_cast<uint32_t>(i)]) : 1;
           }
 #pragma unroll
@@ -409,23 +431,23 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
         }
         auto lag_value = [&](int d, C cs) -> Acc {
           Acc D;
-          if (SUB && L - d <= kEdge) {
+          if (Lay::DIRECT && L - d <= kEdge) {
             Acc acc = 0;
             for (int t = 0; t < L - d; ++t) {
               const int e = t + d;
-              const C x = e < kEdge ? edge[e] : edge[e - L + 2 * kEdge];
-              const C y = edge[t];
+              const C x = e < kEdge ? hedge[e] : hedge[e - L + 2 * kEdge];
+              const C y = hedge[t];
               const Acc dr = static_cast<Acc>(x.x) - static_cast<Acc>(y.x);
               const Acc di = static_cast<Acc>(x.y) - static_cast<Acc>(y.y);
               acc += dr * dr + di * di;
             }
             D = acc * recip<Acc>(L - d);
           } else {
-            const Acc head = tail[L - d - 1];   // psum(L - d)
-            const Acc tl = hptot - tail[d - 1];  // psum(L) - psum(d)
+            const Acc head = htail[L - d - 1];   // psum(L - d)
+            const Acc tl = hptot - htail[d - 1];  // psum(L) - psum(d)
             // N C(d) = Re FFT_N(P)(d) from A = Z(d), B = Z(N/2 - d) and
             // (c, s) = (cos, sin)(2 pi d / N): 2 Re X = A.x + B.x + c (A.y + B.y) - s (A.x - B.x)
-            const C za = buf[padi(d)], zb = buf[padi((NH - d) & (NH - 1))];
+            const C za = hbuf[padi(d)], zb = hbuf[padi((NH - d) & (NH - 1))];
             const Acc ax = za.x, ay = za.y, bx = zb.x, by = zb.y;
             const Acc re = (ax + bx) + static_cast<Acc>(cs.x) * (ay + by) - static_cast<Acc>(cs.y) * (ax - bx);
             const Acc c = re * (Acc(0.5) * inv_n);
@@ -439,12 +461,12 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
           // the second column stores both values (one access where the pair is
           // aligned: the first column is even, so that needs an even row
           // length and an aligned base)
-          const size_t o0 = col_out(a, SEQ * wgi);
+          const size_t o0 = col_out(a, cbase);
           const bool vec = ((nqs | o0) & 1) == 0 && reinterpret_cast<uintptr_t>(out) % sizeof(OutPair<OutT>) == 0;
           static_assert(Lay::KMAX == KL, "one lag iteration count");
 #pragma unroll
           for (int k = 0; k < KL; ++k) {
-            const int i = a.nl - 1 - u - k * STEP;
+            const int i = a.nl - 1 - v - k * STEP;
             if (i < 0) break;
             const Acc D = lag_value(dk[k], csk[k]);
             if (sq == 0) {
@@ -460,14 +482,23 @@ __global__ void __launch_bounds__((P2Lds<LOGN, T, SUB>::TPT), (P2Lds<LOGN, T, SU
             }
           }
         } else {
-          const size_t oq = col_out(a, c);
-          for (int i = a.nl - 1 - u; i >= 0; i -= STEP) {
-            const int d = static_cast<int>(a.lags[i]);
-            out[static_cast<size_t>(i) * nqs + oq] = static_cast<OutT>(lag_value(d, twp[static_cast<uint32_t>(d)]));
+          const size_t oq = col_out(a, ch);
+          if constexpr (PRE) {
+#pragma unroll
+            for (int k = 0; k < KL; ++k) {
+              const int i = a.nl - 1 - v - k * STEP;
+              if (i < 0) break;
+              out[static_cast<size_t>(i) * nqs + oq] = static_cast<OutT>(lag_value(dk[k], csk[k]));
+            }
+          } else {
+            for (int i = a.nl - 1 - v; i >= 0; i -= STEP) {
+              const int d = static_cast<int>(a.lags[i]);
+              out[static_cast<size_t>(i) * nqs + oq] = static_cast<OutT>(lag_value(d, twp[static_cast<uint32_t>(d)]));
+            }
           }
         }
         if constexpr (SUB && !F64) {
-          if (flag && a.flags && active) a.flags[q] = 1;
+          if (flag && a.flags && (SEQ == 1 || active)) a.flags[SEQ > 1 ? q : col_q(a, ch)] = 1;
         }
       }
     }
@@ -507,8 +538,8 @@ hipError_t launch_one(const TimeArgs& a, hipStream_t s) {
   using Lay = P2Lds<LOGN, T, SUB>;
   const int nq = a.cols;
   // two-column plans keep at most KMAX lags per thread in registers (nl < L <= N/2 fits)
-  if (Lay::SEQ > 1 && a.nl > Lay::KMAX * Lay::TPT) return hipErrorInvalidValue;
-  const int wgs = (nq + Lay::SEQ - 1) / Lay::SEQ;
+  if (Lay::SEQ > 1 && a.nl > Lay::KMAX * Lay::NT) return hipErrorInvalidValue;
+  const int wgs = (nq + Lay::G * Lay::SEQ - 1) / (Lay::G * Lay::SEQ);
   const int wpx = (wgs + 7) / 8;
   const size_t lds = Lay::bytes;
   auto kernel = k_time_p2<T, OutT, LOGN, SUB>;
@@ -517,20 +548,36 @@ hipError_t launch_one(const TimeArgs& a, hipStream_t s) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kernel, dim3(8u * wpx), dim3(Lay::TPT), lds, s, a, wpx, nq);
+  hipLaunchKernelGGL(kernel, dim3(8u * wpx), dim3(Lay::NT), lds, s, a, wpx, nq);
   return hipGetLastError();
+}
+
+template <typename T, typename OutT, bool SUB>
+hipError_t launch_logn(const TimeArgs& a, int logn, hipStream_t s) {
+  constexpr int LONG = sizeof(T) == 8 ? 13 : 14;
+  static_assert(kTimeMinLog == 8 && kShortMaxLog == 11, "the short plans");
+  switch (logn) {
+    case 8: return launch_one<T, OutT, 8, SUB>(a, s);
+    case 9: return launch_one<T, OutT, 9, SUB>(a, s);
+    case 10: return launch_one<T, OutT, 10, SUB>(a, s);
+    case 11:
+      if constexpr (sizeof(T) == 4) return launch_one<T, OutT, 11, SUB>(a, s);  // (FP64: in registers)
+      return hipErrorInvalidValue;
+    case LONG: return launch_one<T, OutT, LONG, SUB>(a, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace
 
 int time_p2_log(int precision) { return precision == PREC_FP64 ? 13 : 14; }
 
-hipError_t launch_time_p2(const TimeArgs& a, int precision, int out_dtype, hipStream_t s) {
+hipError_t launch_time_p2(const TimeArgs& a, int logn, int precision, int out_dtype, hipStream_t s) {
   const bool f32 = out_dtype == OUT_F32;
   switch (precision) {
-    case PREC_FP64: return f32 ? launch_one<double, float, 13, true>(a, s) : launch_one<double, double, 13, true>(a, s);
-    case PREC_FP32: return f32 ? launch_one<float, float, 14, false>(a, s) : launch_one<float, double, 14, false>(a, s);
-    case PREC_FP32C: return f32 ? launch_one<float, float, 14, true>(a, s) : launch_one<float, double, 14, true>(a, s);
+    case PREC_FP64: return f32 ? launch_logn<double, float, true>(a, logn, s) : launch_logn<double, double, true>(a, logn, s);
+    case PREC_FP32: return f32 ? launch_logn<float, float, false>(a, logn, s) : launch_logn<float, double, false>(a, logn, s);
+    case PREC_FP32C: return f32 ? launch_logn<float, float, true>(a, logn, s) : launch_logn<float, double, true>(a, logn, s);
     default: return hipErrorInvalidValue;
   }
 }
