@@ -200,14 +200,14 @@ std::vector<T> twiddles(const FftDesc& d) {
 // at the requested lags only; the register kernel (fddm_time_wave.hip) puts two
 // or four columns on a wave, whose one long chain of instructions an empty chip
 // does not hide.  Kernel time of the register and the workgroup kernel in
-// compensated FP32: 200 x 32^2, all lags 14.4 and 12.6 us, 200 x 64^2 15.1 and
-// 15.1; with 20 lags 14.6 and 12.6, 200 x 128^2 23.2 and 21.3; in FP64 200 x 32^2
+// compensated FP32: 200 x 32^2, all lags 14.4 and 12.6 us, 200 x 52^2 14.8 and
+// 13.8, 200 x 64^2 15.1 and 15.1, 500 x 45^2 17.4 and 18.7, 700 x 45^2 22.3 and 22.1; with 20 lags 14.6 and 12.6, 200 x 128^2 23.2 and 21.3; in FP64 200 x 32^2
 // 16.0 and 14.5 us, 500 x 40^2 with 20 lags 18.2 and 15.6, 500 x 52^2 18.9 and 19.0.
 uint64_t short_columns(int logn, int precision, uint64_t nl, uint64_t L) {
   const bool few = nl <= L / 8;
   if (logn > kShortMaxLog) return 0;
-  if (precision != PREC_FP64) return few ? 8400 : logn == 10 ? 850 : 1100;
-  return logn == 8 ? (few ? 8400 : 1100) : logn == 9 ? (few ? 1400 : 1100) : logn == 10 ? 850 : 0;
+  if (precision != PREC_FP64) return few ? 8400 : logn <= 9 ? 1500 : logn == 10 ? 850 : 1100;
+  return logn == 8 ? (few ? 8400 : 1100) : logn == 9 ? (few ? 1500 : 1100) : logn == 10 ? 850 : 0;
 }
 
 // Twiddles of the power-of-two time plans: passes 1 .. np-1 of p2_plan, then

@@ -25,8 +25,8 @@ def _check(out, ref, precision):
         assert np.median(onp.relative_error(out, ref)) <= 1e-4
 
 
-# 3, 819, 910, 1092 and 1170 columns: around 850 and 1100
-PLANES = [(3, 1), (63, 24), (70, 24), (84, 24), (90, 24)]
+# 3, 819, 910, 1092, 1170, 1456 and 1560 columns: around 850, 1100 and 1500
+PLANES = [(3, 1), (63, 24), (70, 24), (84, 24), (90, 24), (112, 24), (120, 24)]
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c", "fp32"])
@@ -42,7 +42,7 @@ def test_every_lag(hip, H, W, precision):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32c", "fp32"])
-@pytest.mark.parametrize("H,W", [(5, 9), (54, 50), (120, 140)])  # 25, 1404 and 8520 columns
+@pytest.mark.parametrize("H,W", [(5, 9), (60, 50), (120, 140)])  # 25, 1560 and 8520 columns
 def test_few_lags(hip, H, W, precision):
     ny, nx = next_fast_len(H, "hip"), next_fast_len(W, "hip")
     for L in (20, 128, 129, 256, 300, 512, 600):
@@ -63,7 +63,7 @@ def test_one_small_lag_marks_every_column(hip, L, lag):
     """Frames that recur once: D at that lag is 1e-5 of the variance, right only
     if the column is marked."""
     rng = np.random.default_rng(lag)
-    H, W = 36, 64  # 1188 columns
+    H, W = 48, 64  # 1584 columns
     base = rng.normal(10000.0, 1000.0, (lag, H, W))
     img = np.concatenate([base, base[: L - lag]]) + rng.normal(0.0, 3.0, (L, H, W))
     img = np.rint(img).astype(np.uint16)
