@@ -345,6 +345,14 @@ hipError_t rows_np(const RowArgs& a, unsigned grid, hipStream_t s) {
   // ms at 1000 frames); as many workgroups as stay resident.  Rows of 1024
   // need three (of 2 or 4 waves) to a CU and many rounds of the chip:
   // 1024^2 x 1000 fp32c 2.06 -> 1.94 ms, FP64 x 300 1.42 -> 1.30 ms, but 8 frames (1.3 rounds) 14 -> 18 us.
+  // In FP32 their runs of R are half lines, which the one-item kernel writes in
+  // neighbouring pairs on one XCD; in launch order they meet only in the caches.
+  // What that costs grows with the launch and shows where little is done per
+  // byte read: 4-byte pixels (1024^2 x 600 plain FP32 1.18 ms, persistent 1.54),
+  // 2-byte pixels without a window and frame 0 to subtract (x 160 0.27 and 0.25
+  // ms, x 300 0.52 and 0.53, x 1500 2.61 and 2.99) or with one of the two (x 600
+  // 1.16 and 1.15, x 1500 2.89 and 2.99), not with both (x 1500 3.07 and 2.96) or 1-byte
+  // pixels (x 1500 2.55 and 2.47).
   if constexpr (sizeof(Tin) <= 4 && LOGX <= 10 && ((1 << LOGX) * sizeof(Tin) / 8) % 64 == 0) {
     if (a.W == (1 << LOGX)) {
       constexpr size_t lds = PersistLds<T, LOGX, NP>::bytes;
@@ -361,7 +369,12 @@ hipError_t rows_np(const RowArgs& a, unsigned grid, hipStream_t s) {
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), 64 * NP, lds);
       if (e != hipSuccess) return e;
       const unsigned resident = static_cast<unsigned>(std::max(1, cus) * std::max(1, per_cu));
-      if (LOGX <= 9 || (per_cu >= 3 && grid / 8 > resident)) {
+      bool persist = LOGX <= 9 || (per_cu >= 3 && grid / 8 > resident);
+      if constexpr (LOGX == 10 && sizeof(T) == 4) {
+        const int work = (a.window != nullptr) + (a.subtract0 != 0);
+        if (sizeof(Tin) == 4 || (sizeof(Tin) == 2 && work < 2 && grid > (work ? 80000u : 25000u))) persist = false;
+      }
+      if (persist) {
         hipLaunchKernelGGL(kernel, dim3(std::min(grid, resident)), dim3(64 * NP), lds, s, a,
                            static_cast<uint32_t>(grid));
         return hipGetLastError();

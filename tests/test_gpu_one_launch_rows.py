@@ -48,6 +48,17 @@ def test_rows_of_1024(hip, L, precision, dtype):
     _check(_run(hip, img, lags, W, H, precision), onp.ddm_diff(img, lags, W, H, None), precision)
 
 
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.float32])
+@pytest.mark.parametrize("precision", ["fp32", "fp32c"])
+def test_rows_of_1024_same_in_pieces(hip, precision, dtype):
+    """Launches of any size give the same bits, whichever kernel they take."""
+    L, H, W = 200, 1024, 1024  # 25600 rows in one launch
+    img = np.random.default_rng(7).integers(0, 255, (L, H, W)).astype(dtype)
+    lags = np.array([1, 100])
+    whole = _run(hip, img, lags, W, H, precision)
+    assert np.array_equal(hip.ddm_diff(img, lags, W, H, None, precision=precision), whole)
+
+
 # width -> transform length: 4 rows to a wave up to 160, 2 up to 320, 1 above
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 @pytest.mark.parametrize("W", [63, 96, 150, 160, 162, 201, 315, 320, 324, 768, 784])
