@@ -86,8 +86,9 @@ __global__ void __launch_bounds__(kThreads) k_rows_p2(RowArgs a, uint32_t nitems
       const bool has_a = fr.here(2 * p), has_b = 2 * p + 1 < fr.n, sub_a = sub && !fr.is_raw(2 * p);
       Vec va{}, vb{}, v0{};
       WVec wv;
-      if (has_a) va = *reinterpret_cast<const Vec*>(row0 + fr.at(2 * p, plane) + x0);
-      if (has_b) vb = *reinterpret_cast<const Vec*>(row0 + fr.first + (2 * p + 1) * plane + x0);
+      const Tin* const pa = row0 + fr.first + static_cast<uint32_t>(2 * p) * plane;
+      if (has_a) va = *reinterpret_cast<const Vec*>((fr.is_raw(2 * p) ? row0 : pa) + x0);
+      if (has_b) vb = *reinterpret_cast<const Vec*>(pa + plane + x0);
       if (sub) v0 = *reinterpret_cast<const Vec*>(ref0 + x0);
       // the VX window values in one or two vector loads issued with the
       // pixels (one load per value: row pass 9.3 ms at 1024^2 x 4000, this
