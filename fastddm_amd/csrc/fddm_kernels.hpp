@@ -125,12 +125,12 @@ bool p2_spatial_ok(int logn);
 int p2_spatial_plan(int logn, bool cols, int* r0, int* r1, int* r2);
 hipError_t launch_rows_p2(const RowArgs& a, int precision, hipStream_t s);
 hipError_t launch_cols_p2(const ColArgs& a, int precision, hipStream_t s);
-// Mixed-radix row kernel (one wave per frame pair, nx <= 768, Tb 4, 8 or
-// 16); launch_rows uses it where rows_mr_ok holds.
+// Mixed-radix row kernel (a frame pair's row on a wave, a half or a quarter of
+// one, 2 <= nx <= 2048, Tb 4, 8 or 16); launch_rows uses it where rows_mr_ok holds.
 bool rows_mr_ok(const RowArgs& a, int precision);
 hipError_t launch_rows_mr(const RowArgs& a, int precision, hipStream_t s);
-// Mixed-radix column kernel (one wave per frame of the block, ny <= 768);
-// launch_cols uses it where cols_mr_ok holds.
+// Mixed-radix column kernel (one wave per frame of the block, 256 <= ny <= 2048,
+// in FP64 up to 768); launch_cols uses it where cols_mr_ok holds.
 bool cols_mr_ok(const ColArgs& a, int precision);
 hipError_t launch_cols_mr(const ColArgs& a, int precision, hipStream_t s);
 hipError_t launch_fft_test(void* data, int n, int batch, const FftDesc& d, const void* tw,
@@ -147,6 +147,12 @@ hipError_t launch_copy_out(void* dst, const void* src, uint64_t n, hipStream_t s
 // kWkFlag L VAR and L - dt > 32 by direct differences of the float series
 // S[q][t] (pitch Lp) in double.
 constexpr int kEdgeFrames = 8;
+// What the float transforms leave in (L - dt) D, against direct differences of
+// the same float spectra: at most 1.4e-7 sum |G|^2 on white noise (8e8 cells) and
+// 5.6e-7 on slow speckle (1.2e8 cells, 120 to 4000 frames), with transforms in
+// registers (fddm_time_wave.hip, fddm_time_pair.hip) as in LDS (fddm_time_p2.hip:
+// 6.2e-7).  So a lag that is not marked is off by 2.8e-4 at most; 1.7e-4 was the
+// largest found.
 constexpr double kWkFlag = 2e-3;
 hipError_t launch_fix(const TimeArgs& a, const void* S64, uint64_t lp, int E, int i0, int out_dtype, hipStream_t s);
 

@@ -51,12 +51,10 @@ using namespace p2;
 constexpr int kMinThreads = 256;  // workgroup size of plans with fewer threads (several q each)
 constexpr int kEdge = 32;
 // Compensated FP32: the float transforms leave an absolute error of at most
-// about 3e-7 x sum_t |G|^2 in (L - dt) D (measured worst case over 2 x 10^9
-// cells at N = 8192).  A q with a lag whose (L - dt) D falls below
-// kWkFlag x sum |G|^2 (2e-3: a relative error bound above ~1.5e-4) -- slow
-// low-q modes at short lags, chance near-recurrences at large lags -- is
-// marked in a.flags; launch_fix then recomputes those lags by direct
-// differences.
+// about 6e-7 x sum_t |G|^2 in (L - dt) D (kWkFlag in fddm_kernels.hpp).  A q with
+// a lag whose (L - dt) D falls below kWkFlag x sum |G|^2 -- slow low-q modes at
+// short lags, chance near-recurrences at large lags -- is marked in a.flags;
+// launch_fix then recomputes those lags by direct differences.
 
 // 1 / n for a positive integer n: hardware reciprocal refined by Newton's
 // iteration r <- r (2 - n r), twice for double (error below 2 ulp).
