@@ -161,19 +161,45 @@ bool factorize(uint64_t n, FftDesc& d) {
   return r == 1;
 }
 
+// exp(-2 pi i j / n) for j < n, evaluated in long double and rounded once.  The
+// long double functions are most of what a plan costs on the host, so the first
+// eighth (or half, if n is no multiple of 8) gives the others by reflection.
+template <typename T>
+std::vector<T> roots(long long n) {
+  const long double two_pi = 6.283185307179586476925286766559005768L;
+  std::vector<T> w(2 * static_cast<size_t>(n));
+  auto direct = [&](long long j, T* z) {
+    const long double ang = two_pi * static_cast<long double>(j) / static_cast<long double>(n);
+    z[0] = static_cast<T>(cosl(ang));
+    z[1] = static_cast<T>(-sinl(ang));
+  };
+  const long long e = n % 8 == 0 ? n / 8 : n / 2, q = n / 4;
+  for (long long j = 0; j <= e && j < n; ++j) direct(j, &w[2 * j]);
+  if (n % 8 != 0) {
+    for (long long j = e + 1; j < n; ++j) {
+      w[2 * j] = w[2 * (n - j)];
+      w[2 * j + 1] = -w[2 * (n - j) + 1];
+    }
+    return w;
+  }
+  for (long long j = e + 1; j <= q; ++j) {  // about n / 8: (c, -s) of j from (s, -c) of q - j
+    w[2 * j] = -w[2 * (q - j) + 1];
+    w[2 * j + 1] = -w[2 * (q - j)];
+  }
+  for (long long j = q + 1; j < n; ++j) {  // a quarter on: times -i
+    w[2 * j] = w[2 * (j - q) + 1];
+    w[2 * j + 1] = -w[2 * (j - q)];
+  }
+  return w;
+}
+
 // Per-pass twiddle tables in the two orders of FftDesc:
 // pass with radix R after Ns points stores exp(-2 pi i r k / (Ns R)) at
-// k (R-1) + r - 1 for k < Ns, r = 1 .. R-1; n - 1 entries in all.  Picked from
-// the n roots of unity, evaluated in long double and rounded once.
+// k (R-1) + r - 1 for k < Ns, r = 1 .. R-1; n - 1 entries in all.
 template <typename T>
 std::vector<T> twiddles(const FftDesc& d) {
-  const long double two_pi = 6.283185307179586476925286766559005768L;
-  std::vector<T> root(2 * static_cast<size_t>(d.n)), w;
-  for (long long j = 0; j < d.n; ++j) {
-    const long double ang = -two_pi * static_cast<long double>(j) / static_cast<long double>(d.n);
-    root[2 * j] = static_cast<T>(cosl(ang));
-    root[2 * j + 1] = static_cast<T>(sinl(ang));
-  }
+  const std::vector<T> root = roots<T>(d.n);
+  std::vector<T> w;
   w.reserve(4 * static_cast<size_t>(fft_table(d.n)));
   const std::pair<int, int> plans[2][8] = {
       {{7, d.c7}, {5, d.c5}, {3, d.c3}, {10, d.c10}, {6, d.c6}, {8, d.c8}, {4, d.c4}, {2, d.c2}},
@@ -216,23 +242,22 @@ uint64_t short_columns(int logn, int precision, uint64_t nl, uint64_t L) {
 template <typename T>
 std::vector<T> p2_twiddles(int logn) {
   const P2Plan P = p2_plan(logn), Q = p2_half_plan(logn);
+  const long long n = 1ll << logn;
+  const std::vector<T> root = roots<T>(n);
   std::vector<T> w;
-  const long double two_pi = 6.283185307179586476925286766559005768L;
   auto pass = [&](long long R, long long NS) {
     for (long long k = 0; k < NS; ++k)
       for (long long r = 0; r < R; ++r) {
-        const long double ang = -two_pi * static_cast<long double>(r * k) / static_cast<long double>(NS * R);
-        w.push_back(static_cast<T>(cosl(ang)));
-        w.push_back(static_cast<T>(sinl(ang)));
+        const T* const z = &root[2 * (r * k * (n / (NS * R)))];
+        w.push_back(z[0]);
+        w.push_back(z[1]);
       }
   };
   for (int i = 1; i < P.np; ++i) pass(p2_radix(P, i), p2_ns(P, i));
   for (int i = 1; i < Q.np; ++i) pass(p2_radix(Q, i), p2_ns(Q, i));
-  const long long n = 1ll << logn;
   for (long long k = 0; k < n / 2; ++k) {
-    const long double ang = two_pi * static_cast<long double>(k) / static_cast<long double>(n);
-    w.push_back(static_cast<T>(cosl(ang)));
-    w.push_back(static_cast<T>(sinl(ang)));
+    w.push_back(root[2 * k]);
+    w.push_back(-root[2 * k + 1]);
   }
   return w;
 }
